@@ -30,6 +30,7 @@
 
 #include "msx_device.h"
 #include "msx_internal.h"
+#include "msx_rows.h"
 #include "msx_sparse.h"
 
 namespace msx {
@@ -442,8 +443,7 @@ __global__ void __launch_bounds__(kThreads)
 }
 
 // ---------------------------------------------------------------------------
-// Value gradients.  G lanes per row.
-
+// Value gradients.  g[p] = cot[row(p)] * x[col(p)], G lanes per row.
 template <class V, class I>
 __global__ void __launch_bounds__(kThreads)
     spmv_data_vjp(const I *__restrict__ indices, const I *__restrict__ indptr,
@@ -465,13 +465,101 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-// One wave per block.  The wave takes 64 / G rows at a time, G lanes per row
-// (lane = one stored value; long rows take several rounds).  X and cot are
-// read in column tiles of kVjpTile: the wave loads each active value's X row
-// segment and each row's cot segment with coalesced loads (two rows per
-// instruction) into LDS, then every lane adds its tile's products in q order
-// from LDS, so each value's sum runs from zero over q = 0 .. k-1 in order.
-constexpr int kVjpTile = 32;
+// The kernels below split the values evenly, not the rows: a wave takes a run
+// of consecutive positions and finds their rows (msx_rows.h), so a row of
+// 37,500 values is as fast as the same values in short rows.
+
+constexpr int kVjpUnroll = 4;  // 64-position steps whose loads a wave issues together
+
+// The same gradient, 256 positions per wave: four index loads, then four
+// gathers of x, in flight at once, the rows found meanwhile.  Positions no
+// row holds (before indptr[0], from indptr[n_rows] on) are left as they are.
+// For matrices whose plan lists long rows; on rows of 16 the row search is a
+// chain that G lanes per row do not have (1.3 M rows: 145 us there, 177 us
+// here), on rows of up to 37,500 the longest row is the other's chain
+// (300,007 power-law rows: VJP1_BEFORE us there, VJP1_AFTER us here).
+template <class V, class I>
+__global__ void __launch_bounds__(kThreads)
+    spmv_data_vjp_split(const I *__restrict__ indices, const I *__restrict__ indptr,
+                  const typename V::Storage *__restrict__ x,
+                  const typename V::Storage *__restrict__ cot, typename V::Storage *__restrict__ out,
+                  int64_t n_rows, int64_t nnz, int64_t n_cols) {
+  using S = typename V::Storage;
+  using A = typename V::Acc;
+  constexpr int kSpan = kVjpUnroll * kWave;
+  const int lane = threadIdx.x % kWave;
+  const int64_t p_end = clamp64(static_cast<int64_t>(indptr[n_rows]), 0, nnz);
+  const int64_t p_begin = clamp64(static_cast<int64_t>(indptr[0]), 0, p_end);
+  const int64_t waves = static_cast<int64_t>(gridDim.x) * (kThreads / kWave);
+  for (int64_t b0 = (static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave) * kSpan;
+       b0 < p_end; b0 += waves * kSpan) {
+    int64_t c[kVjpUnroll];
+    S xv[kVjpUnroll];
+#pragma unroll
+    for (int u = 0; u < kVjpUnroll; ++u) {
+      const int64_t p = b0 + u * kWave + lane;
+      c[u] = static_cast<int64_t>(indices[p < p_end ? p : p_end - 1]);
+    }
+    if (n_cols > 0) {
+#pragma unroll
+      for (int u = 0; u < kVjpUnroll; ++u)
+        xv[u] = x[c[u] >= 0 && c[u] < n_cols ? c[u] : 0];
+    }
+    int64_t row = wave_row_of(indptr, n_rows, b0, lane);
+#pragma unroll
+    for (int u = 0; u < kVjpUnroll; ++u) {
+      const int64_t b = b0 + u * kWave;
+      if (b >= p_end) break;
+      const int64_t p = b + lane;
+      const A g = V::widen(cot[lane_rows(indptr, n_rows, b, lane, row)]);
+      if (p >= p_begin && p < p_end)
+        out[p] = V::narrow((c[u] >= 0 && c[u] < n_cols) ? amul(g, V::widen(xv[u])) : vzero<A>());
+    }
+  }
+}
+
+// Sixteen bytes of a row, at any element alignment (global memory takes
+// unaligned accesses).
+template <class S>
+struct Chunk16 {
+  S v[16 / sizeof(S)];
+};
+template <class S>
+__device__ inline Chunk16<S> load_chunk16(const S *__restrict__ p) {
+  Chunk16<S> r;
+  __builtin_memcpy(&r, p, 16);
+  return r;
+}
+// The first n elements at p and zeros, for rows shorter than sixteen bytes.
+template <class S>
+__device__ inline Chunk16<S> load_short(const S *__restrict__ p, int64_t n) {
+  Chunk16<S> r{};
+#pragma unroll
+  for (int c = 0; c < static_cast<int>(16 / sizeof(S)); ++c)
+    if (c < n) r.v[c] = p[c];
+  return r;
+}
+
+// g[p] = sum_q cot[row(p), q] * X[col(p), q] from zero in q order.  One wave
+// per workgroup and run of positions, one value per lane.  X and cot are read
+// in column tiles of 128 accumulator bytes: each of the 64 values' X row
+// segments and each distinct row's cot segment, in 16-byte loads (eight rows
+// of 128 bytes an instruction) that are all issued before the first LDS
+// store, then every lane adds its tile's products in q order from LDS, four
+// elements a read (a row's 144 LDS bytes keep 16 lanes' reads on different
+// banks).  Bound by the gather of the X rows.
+// Power-law matrix, 300,007 rows, 3.9 M values, rows up to 37,500, float32,
+// k = 32: 18,229 us with G lanes per row (the longest row's rounds in
+// sequence, 4-byte loads) -> VJP_AFTER us.
+template <class V>
+struct VjpTile {
+  static constexpr int kCols = 128 / static_cast<int>(sizeof(typename V::Acc));
+  static constexpr int kPitch = kCols + 16 / static_cast<int>(sizeof(typename V::Acc));
+  static constexpr int kVec = 16 / static_cast<int>(sizeof(typename V::Storage));
+  static constexpr int kLanes = kCols / kVec;       // lanes per row segment
+  static constexpr int kRows = kWave / kLanes;      // row segments per load instruction
+  static constexpr int kLoads = kWave / kRows;      // instructions for 64 rows
+};
 
 template <class V, class I>
 __global__ void __launch_bounds__(kWave)
@@ -479,65 +567,101 @@ __global__ void __launch_bounds__(kWave)
                   const typename V::Storage *__restrict__ X, int64_t ldx,
                   const typename V::Storage *__restrict__ cot, int64_t ldc,
                   typename V::Storage *__restrict__ out, int64_t n_rows, int64_t nnz,
-                  int64_t n_cols, int64_t k, int G) {
+                  int64_t n_cols, int64_t k, int steps) {
+  using S = typename V::Storage;
   using A = typename V::Acc;
-  __shared__ A xs[kWave][kVjpTile + 1];
-  __shared__ A cs[kWave][kVjpTile + 1];
-  __shared__ int cl[kWave];  // column of each lane's value, -1 when none
+  using T = VjpTile<V>;
+  constexpr int E = 16 / static_cast<int>(sizeof(A));  // elements of one LDS read
+  struct alignas(16) Read {
+    A v[E];
+  };
+  __shared__ alignas(16) A xs[kWave][T::kPitch];
+  __shared__ alignas(16) A cs[kWave][T::kPitch];
+  __shared__ int32_t cl[kWave];  // X row of each lane's value
+  __shared__ int32_t rl[kWave];  // the distinct rows of the 64 values
   const int lane = threadIdx.x;
-  const int R = kWave / G;
-  const int g = lane / G, j = lane - g * G;
-  const int half = lane >> 5, qq = lane & 31;
-  for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * R; r0 < n_rows;
-       r0 += static_cast<int64_t>(gridDim.x) * R) {
-    const int64_t row = r0 + g;
-    int64_t s = 0, e = 0;
-    if (row < n_rows) {
-      s = clamp64(static_cast<int64_t>(indptr[row]), 0, nnz);
-      e = clamp64(static_cast<int64_t>(indptr[row + 1]), s, nnz);
-    }
-    const int rows_here = static_cast<int>(r0 + R <= n_rows ? R : n_rows - r0);
-    for (int64_t base = 0;; base += G) {
-      const int64_t p = s + base + j;
-      const bool act = p < e;
-      const uint64_t mask = __ballot(act);
-      if (mask == 0) break;  // wave-uniform
-      int c = -1;
-      if (act) {
-        const int64_t cv = static_cast<int64_t>(indices[p]);
-        c = (cv >= 0 && cv < n_cols) ? static_cast<int>(cv) : -1;
-      }
-      cl[lane] = c;
+  const int seg = lane % T::kLanes, sub = lane / T::kLanes;
+  const int64_t p_end = clamp64(static_cast<int64_t>(indptr[n_rows]), 0, nnz);
+  const int64_t p_begin = clamp64(static_cast<int64_t>(indptr[0]), 0, p_end);
+  const int64_t span = static_cast<int64_t>(steps) * kWave;
+  for (int64_t b0 = static_cast<int64_t>(blockIdx.x) * span; b0 < p_end;
+       b0 += static_cast<int64_t>(gridDim.x) * span) {
+    int64_t row = wave_row_of(indptr, n_rows, b0, lane);
+    for (int64_t b = b0; b < b0 + span && b < p_end; b += kWave) {
+      const int64_t p = b + lane;
+      const int64_t cv = static_cast<int64_t>(indices[p < p_end ? p : p_end - 1]);
+      const bool ok = cv >= 0 && cv < n_cols;
+      const int64_t r = lane_rows(indptr, n_rows, b, lane, row);
+      // slot of the lane's row among the distinct rows
+      const int before = __shfl_up(static_cast<int>(r), 1, kWave);
+      const bool fresh = lane == 0 || before != static_cast<int>(r);
+      const uint64_t starts = __ballot(fresh);
+      const int slot = __popcll(starts & (~uint64_t{0} >> (kWave - 1 - lane))) - 1;
+      const int n_slots = __popcll(starts);
+      cl[lane] = ok ? static_cast<int32_t>(cv) : 0;
+      if (fresh) rl[slot] = static_cast<int32_t>(r);
       __syncthreads();
       A acc = vzero<A>();
-      for (int64_t q0 = 0; q0 < k; q0 += kVjpTile) {
-        const int qn = static_cast<int>(k - q0 < kVjpTile ? k - q0 : kVjpTile);
-        // X row segments of the active values (two per instruction) and the
-        // cot segments of the group's rows: every load is issued before the
-        // first LDS store, so a wave keeps them all in flight.
-        // Slots a lane does not read (no value, dropped column, q >= qn)
-        // hold zeros.
-        using S = typename V::Storage;
-        S xv[kWave / 2], cv[kWave / 2];
+      for (int64_t q0 = 0; q0 < k; q0 += T::kCols) {
+        const int qn = static_cast<int>(k - q0 < T::kCols ? k - q0 : T::kCols);
+        // Loads `load(row pointer)` of the 64 X rows and of the slots' cot
+        // rows, put into LDS by `put`.
+        auto stage = [&](auto load, auto put) {
+          Chunk16<S> xv[T::kLoads];
+          if (n_cols > 0) {
 #pragma unroll
-        for (int t = 0; t < kWave / 2; ++t) {
-          const int cc = cl[2 * t + half];
-          xv[t] = (cc >= 0 && qq < qn) ? X[static_cast<int64_t>(cc) * ldx + q0 + qq] : S{};
-          const int gi = 2 * t + half;
-          cv[t] = (gi < rows_here && qq < qn) ? cot[(r0 + gi) * ldc + q0 + qq] : S{};
-        }
+            for (int t = 0; t < T::kLoads; ++t)
+              xv[t] = load(X + static_cast<int64_t>(cl[t * T::kRows + sub]) * ldx);
+          }
+          const Chunk16<S> cv0 = load(cot + static_cast<int64_t>(rl[sub < n_slots ? sub : 0]) * ldc);
+          if (n_cols > 0) {
 #pragma unroll
-        for (int t = 0; t < kWave / 2; ++t) {
-          xs[2 * t + half][qq] = V::widen(xv[t]);
-          cs[2 * t + half][qq] = V::widen(cv[t]);
+            for (int t = 0; t < T::kLoads; ++t) put(xs[t * T::kRows + sub], xv[t]);
+          }
+          put(cs[sub], cv0);
+          for (int t = T::kRows; t < n_slots; t += T::kRows) {
+            const int at = t + sub;
+            put(cs[at], load(cot + static_cast<int64_t>(rl[at < n_slots ? at : 0]) * ldc));
+          }
+        };
+        if (qn == T::kCols) {
+          const int64_t q = q0 + seg * T::kVec;
+          stage([&](const S *r) { return load_chunk16(r + q); },
+                [&](A *to, const Chunk16<S> &v) {
+#pragma unroll
+                  for (int c = 0; c < T::kVec; ++c) to[seg * T::kVec + c] = V::widen(v.v[c]);
+                });
+        } else if (k >= T::kVec) {
+          // the last tile: no lane reads past k, the lanes that would read
+          // the row's last sixteen bytes again and store the same columns
+          const int64_t q = q0 + seg * T::kVec < k - T::kVec ? q0 + seg * T::kVec : k - T::kVec;
+          const int to0 = static_cast<int>(q - q0);
+          stage([&](const S *r) { return load_chunk16(r + q); },
+                [&](A *to, const Chunk16<S> &v) {
+#pragma unroll
+                  for (int c = 0; c < T::kVec; ++c)
+                    if (to0 + c >= 0) to[to0 + c] = V::widen(v.v[c]);
+                });
+        } else if (seg == 0) {
+          stage([&](const S *r) { return load_short(r, k); },
+                [&](A *to, const Chunk16<S> &v) {
+#pragma unroll
+                  for (int c = 0; c < T::kVec; ++c) to[c] = V::widen(v.v[c]);
+                });
         }
         __syncthreads();
-        if (c >= 0)
-          for (int q = 0; q < qn; ++q) acc = vadd(acc, amul(cs[g][q], xs[lane][q]));
+        int e = 0;
+        for (; e + E <= qn; e += E) {
+          const Read a = *reinterpret_cast<const Read *>(&cs[slot][e]);
+          const Read x4 = *reinterpret_cast<const Read *>(&xs[lane][e]);
+#pragma unroll
+          for (int c = 0; c < E; ++c) acc = vadd(acc, amul(a.v[c], x4.v[c]));
+        }
+        for (; e < qn; ++e) acc = vadd(acc, amul(cs[slot][e], xs[lane][e]));
         __syncthreads();
       }
-      if (act) out[p] = V::narrow(acc);
-      __syncthreads();  // cl is rewritten by the next round
+      if (p >= p_begin && p < p_end) out[p] = V::narrow(ok ? acc : vzero<A>());
+      __syncthreads();  // cl and rl are rewritten by the next step
     }
   }
 }
@@ -652,13 +776,21 @@ template <class V, class I>
 struct SpmvDataVjpOp {
   static msx_status run(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *indices,
                         const void *indptr, const void *x, const void *cot, void *out,
-                        hipStream_t stream) {
+                        bool long_rows, hipStream_t stream) {
     using S = typename V::Storage;
-    const int G = lanes_for(n_rows, nnz);
-    hipLaunchKernelGGL((spmv_data_vjp<V, I>), dim3(grid_for(n_rows * G)), dim3(kThreads), 0, stream,
-                       static_cast<const I *>(indices), static_cast<const I *>(indptr),
-                       static_cast<const S *>(x), static_cast<const S *>(cot), static_cast<S *>(out),
-                       n_rows, nnz, n_cols, G);
+    const auto *ix = static_cast<const I *>(indices);
+    const auto *ip = static_cast<const I *>(indptr);
+    if (long_rows) {
+      const int64_t threads = (nnz + kVjpUnroll - 1) / kVjpUnroll;
+      hipLaunchKernelGGL((spmv_data_vjp_split<V, I>), dim3(grid_for(threads)), dim3(kThreads), 0,
+                         stream, ix, ip, static_cast<const S *>(x), static_cast<const S *>(cot),
+                         static_cast<S *>(out), n_rows, nnz, n_cols);
+    } else {
+      const int G = lanes_for(n_rows, nnz);
+      hipLaunchKernelGGL((spmv_data_vjp<V, I>), dim3(grid_for(n_rows * G)), dim3(kThreads), 0,
+                         stream, ix, ip, static_cast<const S *>(x), static_cast<const S *>(cot),
+                         static_cast<S *>(out), n_rows, nnz, n_cols, G);
+    }
     MSX_HIP_TRY(hipGetLastError());
     return MSX_OK;
   }
@@ -670,13 +802,16 @@ struct SpmmDataVjpOp {
                         const void *indptr, int64_t k, const void *X, int64_t ldx, const void *cot,
                         int64_t ldc, void *out, hipStream_t stream) {
     using S = typename V::Storage;
-    const int G = lanes_for(n_rows, nnz);
-    const int64_t groups = (n_rows + kWave / G - 1) / (kWave / G);
-    const uint32_t grid = static_cast<uint32_t>(std::min<int64_t>(std::max<int64_t>(groups, 1), kMaxGrid));
+    // a row search per run of `steps` x 64 positions: longer runs once there
+    // are runs for several waves on each of the 1,024 SIMDs
+    const int64_t waves = (nnz + kWave - 1) / kWave;
+    const int steps = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(8, waves / 8192)));
+    const int64_t runs = (waves + steps - 1) / steps;
+    const uint32_t grid = static_cast<uint32_t>(std::min<int64_t>(std::max<int64_t>(runs, 1), kMaxGrid));
     hipLaunchKernelGGL((spmm_data_vjp<V, I>), dim3(grid), dim3(kWave), 0, stream,
                        static_cast<const I *>(indices), static_cast<const I *>(indptr),
                        static_cast<const S *>(X), ldx, static_cast<const S *>(cot), ldc,
-                       static_cast<S *>(out), n_rows, nnz, n_cols, k, G);
+                       static_cast<S *>(out), n_rows, nnz, n_cols, k, steps);
     MSX_HIP_TRY(hipGetLastError());
     return MSX_OK;
   }
@@ -1313,6 +1448,7 @@ extern "C" msx_status msx_csr_spmv_data_vjp(msx_vtype vt, msx_itype it, int64_t 
   if (plan != nullptr && plan->bound && plan->vtype == vt && panel_data_vjp_fits(plan))
     return launch_panel_data_vjp(plan, indptr, x, cot, out, static_cast<hipStream_t>(stream));
   return dispatch<SpmvDataVjpOp>(vt, it, n_rows, n_cols, nnz, indices, indptr, x, cot, out,
+                                 plan != nullptr && plan->n_long > 0,
                                  static_cast<hipStream_t>(stream));
 }
 
