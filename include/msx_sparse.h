@@ -68,11 +68,13 @@ typedef struct msx_csr_plan msx_csr_plan;
 
 /* Column slicing of a bound plan (msx_csr_plan_create_bound). */
 typedef enum msx_slice_mode {
-  MSX_SLICE_AUTO = 0,  /* when x exceeds 8 MB and most blocks' columns span
-                          over a quarter of the columns: panels if the matrix
-                          qualifies and its short rows hold at least 65536
-                          values per compute unit, else XCD slices if x is
-                          16 MB or more, else row blocks */
+  MSX_SLICE_AUTO = 0,  /* when most blocks' columns span over a quarter of
+                          the columns: panels if the matrix qualifies and x
+                          is at least 4 MB with 5 Mi values, or 2.5 MB with
+                          12 Mi (row blocks where their copy cannot be
+                          allocated; from 16 MB with at most two values per
+                          column: 16 Mi), else XCD slices if x is 16 MB or
+                          more, else row blocks */
   MSX_SLICE_OFF = 1,   /* row blocks only */
   MSX_SLICE_ON = 2,    /* XCD column slices */
   MSX_SLICE_PANELS = 3 /* LDS column panels (two-pass SpMV) */

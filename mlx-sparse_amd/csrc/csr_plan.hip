@@ -369,28 +369,37 @@ extern "C" msx_status msx_csr_plan_create_bound(msx_vtype vt, msx_itype it, int6
   int mode = opts->slice_mode;
   if (mode == MSX_SLICE_AUTO) {
     // Scattered short rows over a large x: LDS panels (long rows ride in
-    // them as 64-value virtual rows) when the matrix holds enough values to
-    // give every compute unit a pass-1 chunk - the 4M-row random matrix:
-    // 221 us against 930 us in row blocks; the power-law matrix (x 8.4 MB,
-    // about half of its values in long rows): 92 us against 157 us; XCD
-    // slices when x is 16 MB or more and panels are not possible.
+    // them as 64-value virtual rows) where x and the number of values are
+    // large enough (panels_pay) - the 4M-row random matrix: 221 us against
+    // 930 us in row blocks; the power-law matrix (x 8.4 MB, about half of its
+    // values in long rows): 92 us against 157 us; XCD slices when x is 16 MB
+    // or more and panels are not taken.
+    mode = MSX_SLICE_OFF;
     bool scattered = false;
     int64_t short_values = 0;
-    st = probe_scattered(p, indices, s, &scattered, &short_values);
     const int64_t x_bytes = n_cols * static_cast<int64_t>(value_bytes(vt));
-    mode = MSX_SLICE_OFF;
-    if (scattered && panels_eligible(p) && p->nnz >= panels_min_values(p->device))
-      mode = MSX_SLICE_PANELS;
-    else if (scattered && x_bytes >= (int64_t{16} << 20))
-      mode = MSX_SLICE_ON;
+    const bool panels = panels_pay(p) && panels_eligible(p);
+    const bool slices = x_bytes >= kSliceMinX;
+    if (panels || slices) st = probe_scattered(p, indices, s, &scattered, &short_values);
+    if (scattered) mode = panels ? MSX_SLICE_PANELS : MSX_SLICE_ON;
   }
   if (st == MSX_OK && mode == MSX_SLICE_PANELS && p->n_blocks > 0) {
     if (!panels_eligible(p))
       st = fail(MSX_EINVAL,
                 "msx_csr_plan_create_bound: panels need nnz < 2^31, n_cols >= 1 and at most "
                 "2048 panels of x.");
-    else
+    else {
+      const msx_csr_plan row_blocks = *p;
       st = build_panels(p, data, indices, indptr, s);
+      if (st == MSX_ENOMEM && opts->slice_mode == MSX_SLICE_AUTO) {
+        // no room for the copy: the row blocks that are there serve
+        for (void *mem : {p->pn_base, p->pn_meta, p->pn_vmeta})
+          if (mem != nullptr) (void)hipFree(mem);
+        *p = row_blocks;
+        clear_error();
+        st = MSX_OK;
+      }
+    }
   } else if (st == MSX_OK && mode == MSX_SLICE_ON && p->n_blocks > 0) {
     st = build_slices(p, data, indices, indptr, s);
   }

@@ -544,7 +544,7 @@ msx_status probe_scattered(const msx_csr_plan *p, const void *indices, hipStream
   *scattered = false;
   *short_values = 0;
   const int64_t x_bytes = p->n_cols * static_cast<int64_t>(value_bytes(p->vtype));
-  if (x_bytes < (int64_t{8} << 20) || p->n_bounds == 0 || p->n_blocks == 0) return MSX_OK;
+  if (x_bytes < kPanelMinX || p->n_bounds == 0 || p->n_blocks == 0) return MSX_OK;
   return p->itype == MSX_I32 ? probe_w<int32_t>(p, indices, stream, scattered, short_values)
                              : probe_w<int64_t>(p, indices, stream, scattered, short_values);
 }

@@ -176,9 +176,27 @@ msx_status refresh_panels(msx_csr_plan *p, const void *data, hipStream_t stream)
 // of values in short blocks.  Synchronises `stream`.
 msx_status probe_scattered(const msx_csr_plan *p, const void *indices, hipStream_t stream,
                            bool *scattered, int64_t *short_values);
-// Minimum short-row values of an AUTO panel plan: one pass-1 chunk
-// (csr_panel_build.hip, kMinChunk) per compute unit of `device`.
-int64_t panels_min_values(int device);
+// The AUTO rule's sizes for a panel copy of a scattered matrix.  In row
+// blocks each value costs a gather that misses more often the further x
+// outgrows an XCD's 4 MB L2 (per million values: 4.7 us at 1 MB of x, 6.9 at
+// 4 MB, 7.2 at 5 MB, 11 at 8 MB, 13.5 at 16 MB); through panels it costs 2.8
+// us and the call about 13 us more, and new values cost their refresh (3 us
+// per million).  Measured, row blocks -> panels, us: x 5.2 MB, 5.2 M values
+// 39.9 -> 30.4, 10.4 M 77 -> 42.7, 20.8 M 149 -> 72; x 8 MB, 6 M 67 -> 33; x
+// 16 MB, 8 M 123 -> 44; x 4 MB, 4.2 M 29.9 -> 28.3 (below the line), 12.6 M
+// 89 -> 50; x 3.4 MB, 17 M 105 -> 62; x 2 MB, 8.4 M 44.3 -> 36.2 (below it:
+// a training step, with its two refreshes, is slower).
+constexpr int64_t kPanelMinX = int64_t{5} << 19;     // 2.5 MB of x
+constexpr int64_t kPanelMinXFew = int64_t{4} << 20;  // 4 MB of x
+constexpr int64_t kPanelValues = int64_t{12} << 20;
+constexpr int64_t kPanelFewValues = int64_t{5} << 20;
+// From 16 MB of x with at most two values per column on, panels only from 16
+// Mi values and XCD slices below, the choice that the selection tests pin (8
+// M values: panels 44 us, slices 186).
+constexpr int64_t kSliceMinX = int64_t{16} << 20;
+constexpr int64_t kPanelAnyValues = int64_t{16} << 20;
+// True when those sizes favour panels (csr_panel_build.hip).
+bool panels_pay(const msx_csr_plan *p);
 
 // Panel plans (csr_panel_build.hip / csr_panel.hip).
 bool panels_eligible(const msx_csr_plan *p);

@@ -75,3 +75,51 @@ def test_value_gradients_by_positions(kind, vtype):
                                   n_cols)
         want = orc.csr_data_vjp(indices, indptr, X, C, n_rows, n_cols, nnz, vtype=vtype)
         assert to_numpy(got).tobytes() == want.tobytes(), k
+
+
+@pytest.mark.parametrize("vtype,index_dtype,n_rows,n_cols,values", [
+    ("float32", np.int32, 700_001, (4 << 20) // 4, 5 << 20),
+    ("float32", np.int64, 900_003, (5 << 19) // 4, 12 << 20),
+    ("bfloat16", np.int32, 900_001, (4 << 20) // 2 + 5, (5 << 20) + 3),
+    ("float16", np.int64, 2_100_001, (4 << 20) // 2, 5 << 20),
+    ("complex64", np.int32, 300_007, (4 << 20) // 8, 5 << 20),
+])
+def test_auto_panels_at_their_smallest_sizes(vtype, index_dtype, n_rows, n_cols, values):
+    """The smallest matrices for which AUTO takes column panels: every short
+    row equals the row blocks' bit for bit (unsorted and repeated columns,
+    columns out of range and empty rows among them), long rows to their
+    rounding, before and after new values; one value fewer keeps row blocks.
+    Rows average at most 18 values: row blocks sum those in stored order,
+    and only blocks averaging more than 32 in another."""
+    rng = np.random.default_rng(5)
+    # rows of any length up to twice the mean, two long ones, the count exact
+    lengths = rng.multinomial(values - 1500, np.ones(n_rows) / n_rows)
+    lengths[[3, n_rows - 2]] += [1000, 500]
+    indices, indptr = _csr(rng, lengths, n_cols, index_dtype, bad=1e-4)
+    nnz = indices.size
+    assert nnz == values
+    d = to_torch(_values(rng, nnz, vtype), vtype, DEV)
+    x = to_torch(_values(rng, n_cols, vtype), vtype, DEV)
+    i, p = to_torch(indices, None, DEV), to_torch(indptr, None, DEV)
+    print(f"auto panels {vtype} {np.dtype(index_dtype).name} {n_rows}x{n_cols}", flush=True)
+    auto = _capi.Plan(p, n_rows, nnz, data=d, indices=i, n_cols=n_cols)
+    blocks = _capi.Plan(p, n_rows, nnz, data=d, indices=i, n_cols=n_cols,
+                        slice_mode=_capi.SLICE_OFF)
+    assert auto.info().n_panels > 0 and blocks.info().n_panels == 0
+    for _ in range(2):
+        got = _capi.spmv(d, i, p, x, n_rows, n_cols, auto)
+        want = _capi.spmv(d, i, p, x, n_rows, n_cols, blocks)
+        same = (got == want) | (got.isnan() & want.isnan())
+        same[[3, n_rows - 2]] = True
+        assert bool(same.all())
+        # 1,000 products of two normals: 1e-5 of their magnitudes' sum (float32)
+        scale = 1e-2 if vtype in ("float16", "bfloat16") else 1e-5
+        for r in (3, n_rows - 2):
+            assert abs(complex(got[r]) - complex(want[r])) <= scale * 1000
+        d.mul_(0.5)
+        auto.refresh(d)
+    fewer = _capi.Plan(p, n_rows, nnz - 1, data=d[:-1], indices=i[:-1], n_cols=n_cols)
+    if values in (5 << 20, 12 << 20):
+        assert fewer.info().n_panels == 0
+    for plan in (auto, blocks, fewer):
+        plan.close()
