@@ -34,6 +34,9 @@ namespace {
 constexpr int kThreads = 256;
 constexpr uint32_t kMaxGrid = 1u << 20;
 constexpr int64_t kMaxBatchGrid = 65535;  // batches per launch (grid y extent)
+// A row is spmm_long's when it is long for the plan and longer than this many
+// mean rows: where most rows are alike, lane groups keep more of them going.
+constexpr int64_t kLongMeans = 16;
 
 template <class S, int CW>
 struct Vec {
@@ -74,6 +77,16 @@ __device__ inline void store_vec(S *p, const Vec<S, CW> &v) {
 
 __device__ inline int64_t clamp64(int64_t v, int64_t lo, int64_t hi) {
   return v < lo ? lo : (v > hi ? hi : v);
+}
+
+// True when `row` is in the plan's ascending list of long rows.
+__device__ inline bool listed(const int32_t *__restrict__ long_rows, int64_t n_long, int64_t row) {
+  int64_t lo = 0, hi = n_long;
+  while (lo < hi) {
+    const int64_t mid = lo + (hi - lo) / 2;
+    if (long_rows[mid] < row) lo = mid + 1; else hi = mid;
+  }
+  return lo < n_long && long_rows[lo] == row;
 }
 
 constexpr int kChunk = 8;         // values per chunk of a row (shuffle path)
@@ -173,14 +186,18 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
 // Float32 rows of 16-byte chunks are held to 72 registers, 7 waves per SIMD
 // (k = 256 on the 3D Poisson matrix: 1,641 -> 1,607 us; at 64 registers the
 // spills cost 30 %).
-template <class V, class I, int CW, bool SHUF, int LRT = 0, bool NTY = true>
+// SKIP: rows of more than max_len values that the plan lists are left to
+// spmm_long.  Its own instance: the test's registers cost the LR = 8 one two
+// spills (k = 32 on the 3D Poisson matrix: 176 -> 214 us).
+template <class V, class I, int CW, bool SHUF, int LRT = 0, bool NTY = true, bool SKIP = false>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(std::is_same_v<V, F32> && CW == 4 ? 7 : 1, 8)))
     spmm_rows(const typename V::Storage *__restrict__ data, const I *__restrict__ indices,
               const I *__restrict__ indptr, const typename V::Storage *__restrict__ X,
               int64_t ldx, typename V::Storage *__restrict__ Y, int64_t ldy, int64_t n_rows,
               int64_t nnz, int64_t n_cols, int64_t k, int LR_rt, int64_t n_col_tiles, int64_t x_batch,
-              int64_t y_batch) {
+              int64_t y_batch, int64_t max_len, const int32_t *__restrict__ long_rows,
+              int64_t n_long) {
   using S = typename V::Storage;
   using A = typename V::Acc;
   const int LR = LRT > 0 ? LRT : LR_rt;
@@ -202,6 +219,9 @@ __attribute__((amdgpu_waves_per_eu(std::is_same_v<V, F32> && CW == 4 ? 7 : 1, 8)
     if (row >= n_rows) continue;
     const int64_t s = clamp64(static_cast<int64_t>(indptr[row]), 0, nnz);
     const int64_t e = clamp64(static_cast<int64_t>(indptr[row + 1]), s, nnz);
+    if constexpr (SKIP) {
+      if (e - s > max_len && listed(long_rows, n_long, row)) continue;
+    }
     A acc[CW];
     // Lanes past k still take part in the shuffles; they read column 0.
     const S *Xc = X + (col < k ? col : 0);
@@ -263,12 +283,13 @@ __global__ void __launch_bounds__(kThreads)
 // every X row in its L2, halving (G = 2) the X window that a stencil's far
 // neighbours need, at the cost of reading each row's indices/data G times.
 // Sums per column are in stored order, as in spmm_rows.
-template <class V, class I, int CW, bool NTY = true>
+template <class V, class I, int CW, bool NTY = true, bool SKIP = false>
 __global__ void __launch_bounds__(kThreads)
     spmm_linetile(const typename V::Storage *__restrict__ data, const I *__restrict__ indices,
                   const I *__restrict__ indptr, const typename V::Storage *__restrict__ X,
                   int64_t ldx, typename V::Storage *__restrict__ Y, int64_t ldy, int64_t n_rows,
-                  int64_t nnz, int64_t n_cols, int G, int64_t x_batch, int64_t y_batch) {
+                  int64_t nnz, int64_t n_cols, int G, int64_t x_batch, int64_t y_batch,
+                  int64_t max_len, const int32_t *__restrict__ long_rows, int64_t n_long) {
   using S = typename V::Storage;
   using A = typename V::Acc;
   X += blockIdx.y * x_batch;
@@ -292,6 +313,9 @@ __global__ void __launch_bounds__(kThreads)
     if (row >= n_rows) continue;
     const int64_t s = clamp64(static_cast<int64_t>(indptr[row]), 0, nnz);
     const int64_t e = clamp64(static_cast<int64_t>(indptr[row + 1]), s, nnz);
+    if constexpr (SKIP) {
+      if (e - s > max_len && listed(long_rows, n_long, row)) continue;
+    }
     A acc[CW];
     const S *Xc = X + col;
     row_segment<V, I, CW, true>(
@@ -302,6 +326,197 @@ __global__ void __launch_bounds__(kThreads)
     for (int c = 0; c < CW; ++c) out.v[c] = V::narrow(acc[c]);
     store_vec<S, CW, NTY>(Y + row * ldy + col, out);
   }
+}
+
+// ---------------------------------------------------------------------------
+// Long rows.  Each output is one sum in stored order, so a lane group that
+// walks a long row alone waits for its X rows chunk by chunk (69 ns a value at
+// k = 32).  Here one workgroup takes a long row and a tile of TC columns:
+// eight waves gather X rows (16-byte loads at any alignment), form the
+// products and put them into LDS, one tile of B values ahead of the ninth
+// wave, whose lanes add one column each, in order, from LDS.  Their loads run
+// two tiles ahead (the next tile's X rows and the indices after it are in
+// registers while a tile is summed), so the chain of additions, not the
+// memory's latency, sets the pace.  The products and the order are
+// spmm_rows', so are the bits.
+// 32 KB of products a tile, two of them: two workgroups per compute unit.
+// Power-law matrix, 300,007 rows, 3.9 M values, the longest rows 37,500,
+// float32: k = 32 2,604 -> 204 us and 80 us for the other rows, k = 128
+// 5,300 -> 288 and 149.  A tile takes 0.6 us and 3.1 ns a value; the chain
+// alone (a wave adding from LDS) 2.8 ns a value, 107 us for such a row.
+constexpr int kLongProducers = 512;
+constexpr int kLongThreads = kLongProducers + kWave;
+constexpr int kLongTileBytes = 32768;
+
+template <class V, int TC>
+struct LongTile {
+  static constexpr int kVec = 16 / static_cast<int>(sizeof(typename V::Storage));
+  static constexpr int kLanes = TC / kVec;  // lanes per X row segment
+  static constexpr int kValues = kLongTileBytes / (TC * static_cast<int>(sizeof(typename V::Acc)));
+  static constexpr int kRowsPerStep = kLongProducers / kLanes;
+  static constexpr int kSteps = kValues / kRowsPerStep;
+  static_assert(kLanes >= 1 && kSteps >= 1 && kValues % kRowsPerStep == 0, "tile shape");
+};
+
+// Barrier that orders LDS only: the loads of the next tiles stay in flight.
+__device__ inline void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The very long rows go first (z = 0): started last, the longest would run
+// alone at the end.  kForm: 2: k is a multiple of TC, no lane passes k and the
+// LDS stores are whole; 1: the lanes that would pass k read the row's last
+// sixteen bytes; 0: X rows hold less than sixteen bytes.  Every load is unconditional (past
+// the row: its last value, not summed): under a branch each would be waited
+// for at once.
+constexpr int64_t kVeryLong = 4096;
+
+template <class V, class I, int TC, int kForm>
+__global__ void __launch_bounds__(kLongThreads)
+    spmm_long(const typename V::Storage *__restrict__ data, const I *__restrict__ indices,
+              const I *__restrict__ indptr, const typename V::Storage *__restrict__ X, int64_t ldx,
+              typename V::Storage *__restrict__ Y, int64_t ldy, int64_t n_rows, int64_t nnz,
+              int64_t n_cols, int64_t k, const int32_t *__restrict__ long_rows, int64_t max_len) {
+  using S = typename V::Storage;
+  using A = typename V::Acc;
+  using T = LongTile<V, TC>;
+  __shared__ alignas(16) A prod[2][T::kValues][TC];
+  const int64_t row = long_rows[blockIdx.x];
+  if (row < 0 || row >= n_rows) return;
+  const int64_t s = clamp64(static_cast<int64_t>(indptr[row]), 0, nnz);
+  const int64_t e = clamp64(static_cast<int64_t>(indptr[row + 1]), s, nnz);
+  if (e - s <= max_len) return;  // spmm_rows' (every branch here is the workgroup's)
+  if ((e - s > kVeryLong) != (blockIdx.z == 0)) return;
+  const int64_t c0 = static_cast<int64_t>(blockIdx.y) * TC;
+  const int tiles = static_cast<int>((e - s + T::kValues - 1) / T::kValues);
+  if (threadIdx.x < kLongProducers) {
+    const int seg = threadIdx.x % T::kLanes, sub = threadIdx.x / T::kLanes;
+    // the lane's kVec columns: [col, col + kVec) of X, all below k (a lane
+    // that would pass k takes the row's last ones, as its neighbour does)
+    const int64_t want = c0 + seg * T::kVec;
+    const int64_t col = kForm == 2 ? want : kForm == 1 ? (want < k - T::kVec ? want : k - T::kVec) : 0;
+    const int to = static_cast<int>(col - c0);  // LDS column, negative in part past k
+    const S *__restrict__ Xc = X + col;
+    // Loads complete in issue order, so a tile's indices are loaded before
+    // the X rows of the tile ahead of it: waiting for them then leaves those
+    // in flight.  Tile t uses stage t % 2 of everything.
+    I col_of[2][T::kSteps];  // as loaded: looked at one tile later, not waited for here
+    S val_of[2][T::kSteps], a_of[2][T::kSteps];
+    bool ok[2][T::kSteps];
+    Vec<S, T::kVec> xv[2][T::kSteps];
+    auto index = [&](int tile, auto stage) {
+      constexpr int G = decltype(stage)::value;
+#pragma unroll
+      for (int u = 0; u < T::kSteps; ++u) {
+        int64_t p = s + static_cast<int64_t>(tile) * T::kValues + u * T::kRowsPerStep + sub;
+        p = p < e ? p : e - 1;
+        col_of[G][u] = indices[p];
+        val_of[G][u] = data[p];
+      }
+    };
+    auto gather = [&](auto stage) {
+      constexpr int G = decltype(stage)::value;
+#pragma unroll
+      for (int u = 0; u < T::kSteps; ++u) {
+        a_of[G][u] = val_of[G][u];
+        ok[G][u] = static_cast<uint64_t>(static_cast<int64_t>(col_of[G][u])) < static_cast<uint64_t>(n_cols);
+      }
+      if constexpr (kForm > 0) {
+#pragma unroll
+        for (int u = 0; u < T::kSteps; ++u)
+          __builtin_memcpy(&xv[G][u], Xc + (ok[G][u] ? static_cast<int64_t>(col_of[G][u]) : 0) * ldx, 16);
+      } else {
+#pragma unroll
+        for (int u = 0; u < T::kSteps; ++u)
+#pragma unroll
+          for (int c = 0; c < T::kVec; ++c)
+            if (c < k) xv[G][u].v[c] = Xc[(ok[G][u] ? static_cast<int64_t>(col_of[G][u]) : 0) * ldx + c];
+      }
+    };
+    auto put = [&](auto stage) {
+      constexpr int G = decltype(stage)::value;
+#pragma unroll
+      for (int u = 0; u < T::kSteps; ++u) {
+        A *at = &prod[G][u * T::kRowsPerStep + sub][0];
+        const A a = V::widen(a_of[G][u]);
+        A out[T::kVec];
+#pragma unroll
+        for (int c = 0; c < T::kVec; ++c)
+          out[c] = ok[G][u] ? vmul_acc<V>(a, xv[G][u].v[c]) : vzero<A>();  // adds nothing
+        if constexpr (kForm == 2) {
+#pragma unroll
+          for (int c = 0; c < T::kVec; ++c) at[seg * T::kVec + c] = out[c];
+        } else {
+#pragma unroll
+          for (int c = 0; c < T::kVec; ++c)
+            if (to + c >= 0) at[to + c] = out[c];
+        }
+      }
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    index(0, even);
+    index(1, odd);
+    gather(even);
+    index(2, even);
+    gather(odd);
+    for (int t = 0; t < tiles; t += 2) {
+      put(even);
+      index(t + 3, odd);
+      gather(even);
+      lds_barrier();
+      if (t + 1 == tiles) break;
+      put(odd);
+      index(t + 4, even);
+      gather(odd);
+      lds_barrier();
+    }
+    lds_barrier();
+    return;
+  }
+  const int lane = threadIdx.x - kLongProducers;
+  A acc = vzero<A>();
+  __builtin_amdgcn_s_setprio(3);  // the chain goes before the producers on its SIMD
+  lds_barrier();
+  for (int t = 0; t < tiles; ++t) {
+    const int64_t left = e - s - static_cast<int64_t>(t) * T::kValues;
+    const int n = left < T::kValues ? static_cast<int>(left) : T::kValues;
+    const A *__restrict__ from = &prod[t & 1][0][lane < TC ? lane : 0];
+    // 16 values are read while the 16 before them are added (2.8 ns a value,
+    // the latency of the addition; 2.6 from registers)
+    constexpr int G = 16;
+    int v = 0;
+    if (n >= G) {
+      A b[2][G];
+      auto read = [&](A(&to)[G], int at) {
+#pragma unroll
+        for (int u = 0; u < G; ++u) to[u] = from[(at + u) * TC];
+      };
+      auto add = [&](const A(&b0)[G]) {
+#pragma unroll
+        for (int u = 0; u < G; ++u) acc = vadd(acc, b0[u]);
+      };
+      read(b[0], 0);
+      // past the last whole group the next is read all the same, inside the tile
+      for (; v + G <= n; v += 2 * G) {
+        read(b[1], v + 2 * G <= T::kValues ? v + G : 0);
+        __builtin_amdgcn_sched_barrier(0);
+        add(b[0]);
+        if (v + 2 * G > n) {
+          v += G;
+          break;
+        }
+        read(b[0], v + 3 * G <= T::kValues ? v + 2 * G : 0);
+        __builtin_amdgcn_sched_barrier(0);
+        add(b[1]);
+      }
+    }
+    for (; v < n; ++v) acc = vadd(acc, from[v * TC]);
+    lds_barrier();
+  }
+  if (lane < TC && c0 + lane < k) Y[row * ldy + c0 + lane] = V::narrow(acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -943,6 +1158,24 @@ msx_status spmm_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *d
       return MSX_OK;
     }
   }
+  // Long rows of the plan, one workgroup each, when they are the exception.
+  int64_t max_len = INT64_MAX, n_long = 0;
+  const int32_t *long_rows = nullptr;
+  if (batch == 1 && plan != nullptr && plan->n_long > 0 && plan->n_rows == n_rows && n_cols > 0) {
+    max_len = std::max<int64_t>(plan->block_nnz, kLongMeans * (nnz / n_rows));
+    long_rows = plan->long_rows;
+    n_long = plan->n_long;
+    auto go = [&](auto kern, int tc) {
+      hipLaunchKernelGGL(kern, dim3(static_cast<uint32_t>(plan->n_long), static_cast<uint32_t>((k + tc - 1) / tc), 2),
+                         dim3(kLongThreads), 0, stream, data, indices, indptr, X, ldx, Y, ldy,
+                         n_rows, nnz, n_cols, k, plan->long_rows, max_len);
+    };
+    if (k > 32) go(k % 64 == 0 ? spmm_long<V, I, 64, 2> : spmm_long<V, I, 64, 1>, 64);
+    else if (k > 16) go(k == 32 ? spmm_long<V, I, 32, 2> : spmm_long<V, I, 32, 1>, 32);
+    else if (k >= CWV) go(k == 16 ? spmm_long<V, I, 16, 2> : spmm_long<V, I, 16, 1>, 16);
+    else go(spmm_long<V, I, 16, 0>, 16);
+    MSX_HIP_TRY(hipGetLastError());
+  }
   const int G = static_cast<int>(row_bytes / 128);
   if (vec && row_bytes == 256) {
     constexpr int LRT = 128 / 16;
@@ -953,10 +1186,13 @@ msx_status spmm_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *d
     // on XCD x % 8 when batches are stacked along y.
     for (int64_t b0 = 0; b0 < batch; b0 += kMaxBatchGrid) {
       const uint32_t nb = static_cast<uint32_t>(std::min<int64_t>(batch - b0, kMaxBatchGrid));
-      auto kern = y_nt ? spmm_linetile<V, I, CWV, true> : spmm_linetile<V, I, CWV, false>;
+      auto kern = n_long > 0 ? spmm_linetile<V, I, CWV, true, true>
+                  : y_nt     ? spmm_linetile<V, I, CWV, true>
+                             : spmm_linetile<V, I, CWV, false>;
       hipLaunchKernelGGL(kern, dim3(static_cast<uint32_t>(slots * kNumXcd), nb),
                          dim3(kThreads), 0, stream, data, indices, indptr, X + b0 * x_batch, ldx,
-                         Y + b0 * y_batch, ldy, n_rows, nnz, n_cols, G, x_batch, y_batch);
+                         Y + b0 * y_batch, ldy, n_rows, nnz, n_cols, G, x_batch, y_batch, max_len,
+                         long_rows, n_long);
       MSX_HIP_TRY(hipGetLastError());
     }
     return MSX_OK;
@@ -975,23 +1211,28 @@ msx_status spmm_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *d
     S *Yb = Y + b0 * y_batch;
     auto launch = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(grid, nb), dim3(kThreads), 0, stream, data, indices, indptr, Xb,
-                         ldx, Yb, ldy, n_rows, nnz, n_cols, k, LR, n_col_tiles, x_batch, y_batch);
+                         ldx, Yb, ldy, n_rows, nnz, n_cols, k, LR, n_col_tiles, x_batch, y_batch, max_len, long_rows,
+                         n_long);
     };
     if (vec) {
-      auto go = [&](auto nt) {
-        constexpr bool NT = decltype(nt)::value;
+      auto go = [&](auto nt, auto skip) {
+        constexpr bool NT = decltype(nt)::value, SK = decltype(skip)::value;
         switch (LR) {
-        case 1: launch(spmm_rows<V, I, CWV, false, 1, NT>); break;
-        case 2: launch(spmm_rows<V, I, CWV, false, 2, NT>); break;
-        case 4: launch(spmm_rows<V, I, CWV, false, 4, NT>); break;
-        case 8: launch(spmm_rows<V, I, CWV, true, 8, NT>); break;
-        case 16: launch(spmm_rows<V, I, CWV, true, 16, NT>); break;
-        case 32: launch(spmm_rows<V, I, CWV, true, 32, NT>); break;
-        default: launch(spmm_rows<V, I, CWV, true, 64, NT>); break;
+        case 1: launch(spmm_rows<V, I, CWV, false, 1, NT, SK>); break;
+        case 2: launch(spmm_rows<V, I, CWV, false, 2, NT, SK>); break;
+        case 4: launch(spmm_rows<V, I, CWV, false, 4, NT, SK>); break;
+        case 8: launch(spmm_rows<V, I, CWV, true, 8, NT, SK>); break;
+        case 16: launch(spmm_rows<V, I, CWV, true, 16, NT, SK>); break;
+        case 32: launch(spmm_rows<V, I, CWV, true, 32, NT, SK>); break;
+        default: launch(spmm_rows<V, I, CWV, true, 64, NT, SK>); break;
         }
       };
-      if (y_nt) go(std::true_type{});
-      else go(std::false_type{});
+      if (n_long > 0) go(std::true_type{}, std::true_type{});  // a plan: batch 1, Y non-temporal
+      else if (y_nt) go(std::true_type{}, std::false_type{});
+      else go(std::false_type{}, std::false_type{});
+    } else if (n_long > 0) {
+      if (LR >= kChunk) launch(spmm_rows<V, I, 1, true, 0, true, true>);
+      else launch(spmm_rows<V, I, 1, false, 0, true, true>);
     } else {
       if (LR >= kChunk) launch(spmm_rows<V, I, 1, true>);
       else launch(spmm_rows<V, I, 1, false>);

@@ -477,7 +477,7 @@ constexpr int kVjpUnroll = 4;  // 64-position steps whose loads a wave issues to
 // For matrices whose plan lists long rows; on rows of 16 the row search is a
 // chain that G lanes per row do not have (1.3 M rows: 145 us there, 177 us
 // here), on rows of up to 37,500 the longest row is the other's chain
-// (300,007 power-law rows: VJP1_BEFORE us there, VJP1_AFTER us here).
+// (300,007 power-law rows: 1,370 us there, 28 us here).
 template <class V, class I>
 __global__ void __launch_bounds__(kThreads)
     spmv_data_vjp_split(const I *__restrict__ indices, const I *__restrict__ indptr,
@@ -550,7 +550,7 @@ __device__ inline Chunk16<S> load_short(const S *__restrict__ p, int64_t n) {
 // banks).  Bound by the gather of the X rows.
 // Power-law matrix, 300,007 rows, 3.9 M values, rows up to 37,500, float32,
 // k = 32: 18,229 us with G lanes per row (the longest row's rounds in
-// sequence, 4-byte loads) -> VJP_AFTER us.
+// sequence, 4-byte loads) -> 82 us.
 template <class V>
 struct VjpTile {
   static constexpr int kCols = 128 / static_cast<int>(sizeof(typename V::Acc));

@@ -123,3 +123,38 @@ def test_auto_panels_at_their_smallest_sizes(vtype, index_dtype, n_rows, n_cols,
         assert fewer.info().n_panels == 0
     for plan in (auto, blocks, fewer):
         plan.close()
+
+
+@pytest.mark.parametrize("vtype", VTYPES)
+@pytest.mark.parametrize("index_dtype", [np.int32, np.int64])
+def test_spmm_long_rows_in_stored_order(vtype, index_dtype):
+    """Long rows of a plan, a workgroup each, equal the oracle bit for bit at
+    column counts around every tile width (16, 32, 64 columns) and below a
+    16-byte load, rows a tile of products long, one value more and less
+    among them; also where indptr changed after the plan was built (a row
+    longer than it was then, and a listed row now short)."""
+    rng = np.random.default_rng(43)
+    lengths = rng.integers(0, 6, 2500)
+    lengths[[0, 7, 900, 901, 1300, 2100, 2499]] = [5000, 257, 256, 255, 129, 1024, 2000]
+    n_rows, n_cols = len(lengths), 3001
+    indices, indptr = _csr(rng, lengths, n_cols, index_dtype, bad=0.01)
+    nnz = indices.size
+    data = _values(rng, nnz, vtype)
+    d, i = to_torch(data, vtype, DEV), to_torch(indices, None, DEV)
+    p = to_torch(indptr, None, DEV)
+    plan = _capi.Plan(p, n_rows, nnz, 64, data=d, indices=i, n_cols=n_cols)
+    assert plan.info().n_long_rows == 7
+    # a column out of range adds nothing, as a zero does
+    good = (indices >= 0) & (indices < n_cols)
+    held, cols = np.where(good, data, np.zeros_like(data)), np.where(good, indices, 0)
+    moved = indptr.copy()
+    moved[8:901] = moved[901]  # row 7 takes the rows after it, rows 8 to 900 are empty
+    for ptr in (indptr, moved):
+        p.copy_(to_torch(ptr, None, DEV))
+        for k in (1, 2, 3, 7, 16, 17, 32, 33, 63, 64, 65, 100, 130):
+            X = _values(rng, (n_cols, k), vtype)
+            print(f"spmm long rows {vtype} {np.dtype(index_dtype).name} k={k}", flush=True)
+            got = _capi.spmm(d, i, p, to_torch(X, vtype, DEV), n_rows, n_cols, plan=plan)
+            want = orc.csr_matmul(held, cols.astype(index_dtype), ptr, X, n_rows, vtype=vtype)
+            assert to_numpy(got).tobytes() == want.tobytes(), k
+    plan.close()
