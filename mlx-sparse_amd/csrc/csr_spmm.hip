@@ -56,6 +56,40 @@ __device__ inline Vec<S, CW> load_vec(const S *p) {
   }
 }
 
+// CW elements as the dwords they were loaded in, taken apart where they are
+// used: 16-bit elements taken apart at the load (a Vec filled under a branch)
+// had every load of a chunk waited for before the next (k = 64 on the 3D
+// Poisson matrix, bfloat16: 372 -> 204 us).
+template <class S, int CW>
+struct Packed {
+  static constexpr int kBytes = CW * static_cast<int>(sizeof(S));
+  static constexpr int kWords = (kBytes + 3) / 4;
+  uint32_t w[kWords];
+  __device__ inline S at(int c) const {
+    if constexpr (sizeof(S) == 2) {
+      return static_cast<S>(w[c / 2] >> (16 * (c & 1)));
+    } else if constexpr (sizeof(S) == 4) {
+      return __builtin_bit_cast(S, w[c]);
+    } else {
+      return __builtin_bit_cast(S, static_cast<uint64_t>(w[2 * c]) | (static_cast<uint64_t>(w[2 * c + 1]) << 32));
+    }
+  }
+};
+
+// ANY: at any element alignment (global memory takes unaligned accesses).
+template <class S, int CW, bool ANY = false>
+__device__ inline Packed<S, CW> load_packed(const S *p) {
+  Packed<S, CW> r;
+  if constexpr (CW * sizeof(S) < 4) {
+    r.w[0] = *reinterpret_cast<const uint16_t *>(p);
+  } else if constexpr (!ANY && CW * sizeof(S) == 16) {
+    r = __builtin_bit_cast(Packed<S, CW>, *reinterpret_cast<const uint4 *>(p));
+  } else {
+    __builtin_memcpy(&r, p, CW * sizeof(S));
+  }
+  return r;
+}
+
 // Y is written once and not read back by the kernel: 16-byte stores are
 // non-temporal (measured at k = 8 / 64 / 256 on the 3D Poisson matrix: 63 ->
 // 52, 362 -> 351, 1,694 -> 1,650 us), unless the caller reads Y again right
@@ -121,7 +155,7 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
     for (; p + kUnrollDirect <= e; p += kUnrollDirect) {
       int cu[kUnrollDirect];
       A au[kUnrollDirect];
-      Vec<S, CW> xv[kUnrollDirect];
+      Packed<S, CW> xv[kUnrollDirect];
 #pragma unroll
       for (int u = 0; u < kUnrollDirect; ++u) {
         const I c = indices[p + u];
@@ -135,16 +169,16 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
       for (int u = 0; u < kUnrollDirect; ++u)
         if (cu[u] >= 0) {
 #pragma unroll
-          for (int c = 0; c < CW; ++c) acc[c] = vmadd<V>(acc[c], au[u], xv[u].v[c]);
+          for (int c = 0; c < CW; ++c) acc[c] = vmadd<V>(acc[c], au[u], xv[u].at(c));
         }
     }
     for (; p < e; ++p) {
       const I c = indices[p];
       if (static_cast<uint64_t>(static_cast<int64_t>(c)) < static_cast<uint64_t>(n_cols)) {
         const A a = V::widen(data[p]);
-        const Vec<S, CW> xv = fetch(static_cast<int>(c));
+        const Packed<S, CW> xv = fetch(static_cast<int>(c));
 #pragma unroll
-        for (int q = 0; q < CW; ++q) acc[q] = vmadd<V>(acc[q], a, xv.v[q]);
+        for (int q = 0; q < CW; ++q) acc[q] = vmadd<V>(acc[q], a, xv.at(q));
       }
     }
     return;
@@ -164,7 +198,7 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
       cu[u] = __shfl(ci, u, LR);
       au[u] = shfl_idx(av, u, LR);
     }
-    Vec<S, CW> xv[kChunk];
+    Packed<S, CW> xv[kChunk];
 #pragma unroll
     for (int u = 0; u < kChunk; ++u)
       if (cu[u] >= 0) xv[u] = fetch(cu[u]);
@@ -172,7 +206,7 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
     for (int u = 0; u < kChunk; ++u)
       if (cu[u] >= 0) {
 #pragma unroll
-        for (int c = 0; c < CW; ++c) acc[c] = vmadd<V>(acc[c], au[u], xv[u].v[c]);
+        for (int c = 0; c < CW; ++c) acc[c] = vmadd<V>(acc[c], au[u], xv[u].at(c));
       }
   };
   // The first chunk outside the loop: rows of up to 8 values (stencils)
@@ -182,16 +216,22 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
 }
 
 // LRT: the group width LR as a compile-time constant (a runtime width in
-// every shuffle and index measured 6 % slower at k = 256); 0 takes LR_rt.
+// every shuffle and index measured 6 % slower at k = 256); 0 takes LR_rt (one
+// column a lane: 268 us at k = 3 on 1 M rows of 16, constant widths 281).
 // Float32 rows of 16-byte chunks are held to 72 registers, 7 waves per SIMD
 // (k = 256 on the 3D Poisson matrix: 1,641 -> 1,607 us; at 64 registers the
 // spills cost 30 %).
 // SKIP: rows of more than max_len values that the plan lists are left to
 // spmm_long.  Its own instance: the test's registers cost the LR = 8 one two
 // spills (k = 32 on the 3D Poisson matrix: 176 -> 214 us).
-template <class V, class I, int CW, bool SHUF, int LRT = 0, bool NTY = true, bool SKIP = false>
+// ANY: rows of any length k >= CW at any element alignment: the lane whose
+// columns would pass k takes the row's last CW instead (its neighbour's in
+// part, the same sums), so every load and store is whole.  16-bit, k = 100,
+// 300,007 rows of 20: one 2-byte column per lane 683 us, this 266.
+template <class V, class I, int CW, bool SHUF, int LRT, bool NTY = true, bool SKIP = false,
+          bool ANY = false>
 __global__ void __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(std::is_same_v<V, F32> && CW == 4 ? 7 : 1, 8)))
+__attribute__((amdgpu_waves_per_eu(std::is_same_v<V, F32> && CW == 4 && !ANY ? 7 : 1, 8)))
     spmm_rows(const typename V::Storage *__restrict__ data, const I *__restrict__ indices,
               const I *__restrict__ indptr, const typename V::Storage *__restrict__ X,
               int64_t ldx, typename V::Storage *__restrict__ Y, int64_t ldy, int64_t n_rows,
@@ -215,7 +255,8 @@ __attribute__((amdgpu_waves_per_eu(std::is_same_v<V, F32> && CW == 4 ? 7 : 1, 8)
     const int64_t rt = n_col_tiles == 1 ? t : t / n_col_tiles;
     const int64_t ct = t - rt * n_col_tiles;
     const int64_t row = rt * rows_per_group + g;
-    const int64_t col = ct * tile_cols + static_cast<int64_t>(l) * CW;
+    const int64_t want = ct * tile_cols + static_cast<int64_t>(l) * CW;
+    const int64_t col = ANY && want > k - CW ? k - CW : want;
     if (row >= n_rows) continue;
     const int64_t s = clamp64(static_cast<int64_t>(indptr[row]), 0, nnz);
     const int64_t e = clamp64(static_cast<int64_t>(indptr[row + 1]), s, nnz);
@@ -226,13 +267,15 @@ __attribute__((amdgpu_waves_per_eu(std::is_same_v<V, F32> && CW == 4 ? 7 : 1, 8)
     // Lanes past k still take part in the shuffles; they read column 0.
     const S *Xc = X + (col < k ? col : 0);
     row_segment<V, I, CW, SHUF>(
-        data, indices, [&](int c) { return load_vec<S, CW>(Xc + static_cast<int64_t>(c) * ldx); },
+        data, indices,
+        [&](int c) { return load_packed<S, CW, ANY>(Xc + static_cast<int64_t>(c) * ldx); },
         n_cols, s, e, l, LR, acc);
-    if (col >= k) continue;
+    if (want >= k) continue;
     Vec<S, CW> out;
 #pragma unroll
     for (int c = 0; c < CW; ++c) out.v[c] = V::narrow(acc[c]);
-    store_vec<S, CW, NTY>(Y + row * ldy + col, out);
+    if constexpr (ANY) __builtin_memcpy(Y + row * ldy + col, &out, sizeof(out));
+    else store_vec<S, CW, NTY>(Y + row * ldy + col, out);
   }
 }
 
@@ -262,7 +305,7 @@ __global__ void __launch_bounds__(kThreads)
     A acc[CW];
     const S *Xc = Xt + static_cast<int64_t>(l) * CW;
     row_segment<V, I, CW, (LR >= kChunk)>(
-        data, indices, [&](int c) { return load_vec<S, CW>(Xc + static_cast<int64_t>(c) * kpad); },
+        data, indices, [&](int c) { return load_packed<S, CW>(Xc + static_cast<int64_t>(c) * kpad); },
         n_cols, s, e, l, LR, acc);
 #pragma unroll
     for (int c = 0; c < CW; ++c) {
@@ -319,7 +362,7 @@ __global__ void __launch_bounds__(kThreads)
     A acc[CW];
     const S *Xc = X + col;
     row_segment<V, I, CW, true>(
-        data, indices, [&](int c) { return load_vec<S, CW>(Xc + static_cast<int64_t>(c) * ldx); },
+        data, indices, [&](int c) { return load_packed<S, CW>(Xc + static_cast<int64_t>(c) * ldx); },
         n_cols, s, e, l, LR, acc);
     Vec<S, CW> out;
 #pragma unroll
@@ -1197,7 +1240,9 @@ msx_status spmm_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *d
     }
     return MSX_OK;
   }
-  const int CW = vec ? CWV : 1;
+  // Sixteen bytes a lane; shorter rows (k < CWV, at most eight lanes) one
+  // column a lane (float32, k = 3, 1 M rows of 16: 268 us, two columns 285).
+  const int CW = k >= CWV ? CWV : 1;
   const int64_t lanes = (k + CW - 1) / CW;
   int LR = 1;
   while (LR < lanes && LR < 64) LR <<= 1;
@@ -1230,12 +1275,29 @@ msx_status spmm_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *d
       if (n_long > 0) go(std::true_type{}, std::true_type{});  // a plan: batch 1, Y non-temporal
       else if (y_nt) go(std::true_type{}, std::false_type{});
       else go(std::false_type{}, std::false_type{});
-    } else if (n_long > 0) {
-      if (LR >= kChunk) launch(spmm_rows<V, I, 1, true, 0, true, true>);
-      else launch(spmm_rows<V, I, 1, false, 0, true, true>);
+    } else if (CW == CWV) {
+      auto go = [&](auto skip) {
+        constexpr bool SK = decltype(skip)::value;
+        switch (LR) {
+        case 1: launch(spmm_rows<V, I, CWV, false, 1, false, SK, true>); break;
+        case 2: launch(spmm_rows<V, I, CWV, false, 2, false, SK, true>); break;
+        case 4: launch(spmm_rows<V, I, CWV, false, 4, false, SK, true>); break;
+        case 8: launch(spmm_rows<V, I, CWV, true, 8, false, SK, true>); break;
+        case 16: launch(spmm_rows<V, I, CWV, true, 16, false, SK, true>); break;
+        case 32: launch(spmm_rows<V, I, CWV, true, 32, false, SK, true>); break;
+        default: launch(spmm_rows<V, I, CWV, true, 64, false, SK, true>); break;
+        }
+      };
+      if (n_long > 0) go(std::true_type{});
+      else go(std::false_type{});
     } else {
-      if (LR >= kChunk) launch(spmm_rows<V, I, 1, true>);
-      else launch(spmm_rows<V, I, 1, false>);
+      auto go = [&](auto skip) {
+        constexpr bool SK = decltype(skip)::value;
+        if (LR >= kChunk) launch(spmm_rows<V, I, 1, true, 0, true, SK>);
+        else launch(spmm_rows<V, I, 1, false, 0, true, SK>);
+      };
+      if (n_long > 0) go(std::true_type{});
+      else go(std::false_type{});
     }
     MSX_HIP_TRY(hipGetLastError());
   }

@@ -158,3 +158,30 @@ def test_spmm_long_rows_in_stored_order(vtype, index_dtype):
             want = orc.csr_matmul(held, cols.astype(index_dtype), ptr, X, n_rows, vtype=vtype)
             assert to_numpy(got).tobytes() == want.tobytes(), k
     plan.close()
+
+
+@pytest.mark.parametrize("vtype", VTYPES)
+def test_spmm_rows_of_any_length_and_alignment(vtype):
+    """Rows of X and Y that are no multiple of sixteen bytes, or start off
+    one: every column equals the oracle's bit for bit and nothing is written
+    past a row's end (rows of a wider buffer, first element skipped)."""
+    rng = np.random.default_rng(47)
+    lengths = rng.integers(0, 21, 700)
+    lengths[[0, 1, 2, 3]] = [8, 9, 16, 17]
+    n_rows, n_cols = len(lengths), 513
+    indices, indptr = _csr(rng, lengths, n_cols)
+    data = _values(rng, indices.size, vtype)
+    d = to_torch(data, vtype, DEV)
+    i, p = to_torch(indices, None, DEV), to_torch(indptr, None, DEV)
+    for k in (1, 2, 3, 4, 5, 6, 7, 9, 12, 15, 20, 31, 33, 64, 100, 127, 257, 515):
+        X = _values(rng, (n_cols, k), vtype)
+        want = orc.csr_matmul(data, indices, indptr, X, n_rows, vtype=vtype)
+        for pad, skip in ((0, 0), (3, 1)):
+            wide = torch.zeros(n_cols, k + pad + skip, dtype=d.dtype, device=DEV)
+            wide[:, skip:skip + k] = to_torch(X, vtype, DEV)
+            out = torch.full((n_rows, k + pad + skip), 7, dtype=d.dtype, device=DEV)
+            print(f"spmm ragged {vtype} k={k} pad={pad} skip={skip}", flush=True)
+            _capi.spmm(d, i, p, wide[:, skip:skip + k], n_rows, n_cols, Y=out[:, skip:skip + k])
+            got = out[:, skip:skip + k].contiguous()
+            assert to_numpy(got).tobytes() == want.tobytes(), (k, pad)
+            assert bool((out[:, :skip] == 7).all()) and bool((out[:, skip + k:] == 7).all())
