@@ -303,6 +303,21 @@ msx_status msx_csr_batched_spmv(msx_vtype vt, msx_itype it, int64_t n_rows,
                                 void *Y, int64_t ldy, void *stream);
 
 /*
+ * The same with the caller's device scratch: at least
+ * msx_csr_batched_spmv_scratch bytes (0 for one vector), 16-byte aligned,
+ * free for reuse once the call's work on `stream` is done.
+ */
+size_t msx_csr_batched_spmv_scratch(msx_vtype vt, int64_t n_rows,
+                                    int64_t n_cols, int64_t batch);
+msx_status msx_csr_batched_spmv_ws(msx_vtype vt, msx_itype it, int64_t n_rows,
+                                   int64_t n_cols, int64_t nnz,
+                                   const void *data, const void *indices,
+                                   const void *indptr, int64_t batch,
+                                   const void *X, int64_t ldx, void *Y,
+                                   int64_t ldy, void *scratch,
+                                   size_t scratch_bytes, void *stream);
+
+/*
  * Batched SpMM on the device: Y[b] = A X[b] for b < batch.  X[b] starts at
  * X + b * x_batch (row-major n_cols x k, row stride ldx), Y[b] at
  * Y + b * y_batch (n_rows x k, row stride ldy); strides in elements.  Summed

@@ -78,6 +78,12 @@ def build(verbose: bool = True) -> Path:
 
     import pybind11  # noqa: PLC0415 - build-time dependency only
 
+    import torch  # noqa: PLC0415 - its headers and libraries, for the binding
+
+    torch_dir = Path(torch.__file__).resolve().parent
+    torch_flags = [f"-I{torch_dir / 'include'}",
+                   f"-I{torch_dir / 'include/torch/csrc/api/include'}",
+                   f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}"]
     py_inc = sysconfig.get_paths()["include"]
     bind_srcs = [SRC / "bindings.cpp", SRC / "common" / "validate.cpp",
                  SRC / "sparse" / "csr_matvec" / "csr_matvec.cpp",
@@ -90,8 +96,10 @@ def build(verbose: bool = True) -> Path:
     for s in bind_srcs:
         o = BUILD / ("bind_" + s.stem + ".o")
         bind_objs.append(o)
+        # torch's headers are not warning-free under -Wextra
+        extra = [*torch_flags, "-Wno-extra"] if s.name == "bindings.cpp" else []
         jobs.append(["g++", *CXX_FLAGS, "-fvisibility=hidden", f"-I{pybind11.get_include()}",
-                     f"-I{py_inc}", "-c", str(s), "-o", str(o)])
+                     f"-I{py_inc}", *extra, "-c", str(s), "-o", str(o)])
 
     workers = min(len(jobs), max(1, min(8, os.cpu_count() or 1)))
     with ThreadPoolExecutor(max_workers=workers) as pool:
@@ -106,7 +114,8 @@ def build(verbose: bool = True) -> Path:
     ext = OUT_DIR / ("_ext" + _ext_suffix())
     tmp = ext.with_suffix(".tmp")
     _run(["g++", "-shared", "-fPIC", "-o", str(tmp), *map(str, bind_objs),
-          f"-L{OUT_DIR}", "-lmsx_sparse", "-Wl,-rpath,$ORIGIN"])
+          f"-L{OUT_DIR}", "-lmsx_sparse", "-Wl,-rpath,$ORIGIN", f"-L{torch_dir / 'lib'}",
+          "-ltorch_python", "-ltorch_cpu", "-lc10"])
     os.replace(tmp, ext)
     if verbose:
         print(f"built {lib.relative_to(REPO)} and {ext.relative_to(REPO)}")

@@ -249,38 +249,51 @@ msx_status check_batched(const char *op, msx_vtype vt, msx_itype it, int64_t n_r
 
 using namespace msx;
 
-extern "C" msx_status msx_csr_batched_spmv(msx_vtype vt, msx_itype it, int64_t n_rows,
-                                           int64_t n_cols, int64_t nnz, const void *data,
-                                           const void *indices, const void *indptr, int64_t batch,
-                                           const void *X, int64_t ldx, void *Y, int64_t ldy,
-                                           void *stream_v) {
-  clear_error();
-  const char *op = "csr_batched_matvec";
-  msx_status st = check_batched(op, vt, it, n_rows, n_cols, nnz, data, indices, indptr, batch);
+namespace {
+
+// The transposed operand Xt (n_cols x kpad) and the result Yt of the widths
+// that do not store straight to Y.  Columns are padded so that a row is a
+// whole number of 16-byte vectors (the SpMM's vector path); padding columns
+// read zero.
+struct BatchScratch {
+  int64_t kpad;
+  size_t bx, by;
+};
+
+BatchScratch batch_scratch(msx_vtype vt, int64_t n_rows, int64_t n_cols, int64_t batch) {
+  const int64_t sv = static_cast<int64_t>(value_bytes(vt));
+  const int64_t per16 = 16 / sv;
+  BatchScratch b;
+  b.kpad = (batch + per16 - 1) / per16 * per16;
+  b.bx = static_cast<size_t>(std::max<int64_t>(n_cols, 1) * b.kpad * sv);
+  b.by = static_cast<size_t>(n_rows * b.kpad * sv);
+  return b;
+}
+
+msx_status check_batched_spmv(msx_vtype vt, msx_itype it, int64_t n_rows, int64_t n_cols,
+                              int64_t nnz, const void *data, const void *indices,
+                              const void *indptr, int64_t batch, const void *X, int64_t ldx,
+                              void *Y, int64_t ldy) {
+  msx_status st = check_batched("csr_batched_matvec", vt, it, n_rows, n_cols, nnz, data, indices, indptr, batch);
   if (st != MSX_OK) return st;
   if (ldx < n_cols || ldy < n_rows)
     return fail(MSX_EINVAL, "csr_batched_matvec row strides must be at least the vector lengths.");
   if (batch > 0 && n_rows > 0 && Y == nullptr) return fail(MSX_EINVAL, "csr_batched_matvec Y is NULL.");
   if (batch > 0 && n_cols > 0 && nnz > 0 && X == nullptr)
     return fail(MSX_EINVAL, "csr_batched_matvec X is NULL.");
-  if (batch == 0 || n_rows == 0) return MSX_OK;
-  auto stream = static_cast<hipStream_t>(stream_v);
-  if (batch == 1)  // one vector is a one-column SpMM, no transposes
-    return launch_spmm_batched(vt, it, n_rows, n_cols, nnz, data, indices, indptr, 1, 1, X, 0, 1,
-                               Y, 0, 1, true, stream);
-  // Columns padded so that a row of the transposed operands is a whole number
-  // of 16-byte vectors (the SpMM's vector path); padding columns read zero.
-  const int64_t sv = static_cast<int64_t>(value_bytes(vt));
-  const int64_t per16 = 16 / sv;
-  const int64_t kpad = (batch + per16 - 1) / per16 * per16;
-  const size_t bx = static_cast<size_t>(std::max<int64_t>(n_cols, 1) * kpad * sv);
-  const size_t by = static_cast<size_t>(n_rows * kpad * sv);
-  char *scratch = nullptr;
-  MSX_HIP_TRY(hipMallocAsync(reinterpret_cast<void **>(&scratch), bx + by, stream));
-  void *Xt = scratch, *Yt = scratch + bx;
+  return MSX_OK;
+}
+
+msx_status run_batched_spmv(msx_vtype vt, msx_itype it, int64_t n_rows, int64_t n_cols,
+                            int64_t nnz, const void *data, const void *indices,
+                            const void *indptr, int64_t batch, const void *X, int64_t ldx, void *Y,
+                            int64_t ldy, void *scratch, hipStream_t stream) {
+  const BatchScratch b = batch_scratch(vt, n_rows, n_cols, batch);
+  const int64_t kpad = b.kpad;
+  void *Xt = scratch, *Yt = static_cast<char *>(scratch) + b.bx;
   const bool thin = kpad <= kNarrow;
-  st = thin ? narrow(vt, true, X, batch, kpad, n_cols, ldx, Xt, stream)
-            : transpose(vt, X, batch, kpad, n_cols, ldx, Xt, kpad, stream);
+  msx_status st = thin ? narrow(vt, true, X, batch, kpad, n_cols, ldx, Xt, stream)
+                       : transpose(vt, X, batch, kpad, n_cols, ldx, Xt, kpad, stream);
   // Up to 8 16-byte vectors per row of Xt the sums go straight to Y;
   // otherwise through an n_rows x kpad SpMM result and its transpose.
   bool direct = false;
@@ -294,6 +307,57 @@ extern "C" msx_status msx_csr_batched_spmv(msx_vtype vt, msx_itype it, int64_t n
       st = thin ? narrow(vt, false, Yt, batch, kpad, n_rows, ldy, Y, stream)
                 : transpose(vt, Yt, n_rows, n_rows, batch, kpad, Y, ldy, stream);
   }
+  return st;
+}
+
+}  // namespace
+
+extern "C" size_t msx_csr_batched_spmv_scratch(msx_vtype vt, int64_t n_rows, int64_t n_cols,
+                                               int64_t batch) {
+  if (!valid_vtype(vt) || n_rows <= 0 || n_cols < 0 || batch <= 1) return 0;
+  const BatchScratch b = batch_scratch(vt, n_rows, n_cols, batch);
+  return b.bx + b.by;
+}
+
+extern "C" msx_status msx_csr_batched_spmv_ws(msx_vtype vt, msx_itype it, int64_t n_rows,
+                                              int64_t n_cols, int64_t nnz, const void *data,
+                                              const void *indices, const void *indptr,
+                                              int64_t batch, const void *X, int64_t ldx, void *Y,
+                                              int64_t ldy, void *scratch, size_t scratch_bytes,
+                                              void *stream) {
+  clear_error();
+  msx_status st = check_batched_spmv(vt, it, n_rows, n_cols, nnz, data, indices, indptr, batch, X,
+                                     ldx, Y, ldy);
+  if (st != MSX_OK) return st;
+  if (batch == 0 || n_rows == 0) return MSX_OK;
+  auto s = static_cast<hipStream_t>(stream);
+  if (batch == 1)  // one vector is a one-column SpMM, no transposes
+    return launch_spmm_batched(vt, it, n_rows, n_cols, nnz, data, indices, indptr, 1, 1, X, 0, 1,
+                               Y, 0, 1, true, s);
+  if (scratch == nullptr || scratch_bytes < msx_csr_batched_spmv_scratch(vt, n_rows, n_cols, batch) ||
+      (reinterpret_cast<uintptr_t>(scratch) & 15u) != 0)
+    return fail(MSX_EINVAL, "csr_batched_matvec scratch must be 16-byte aligned and hold "
+                            "msx_csr_batched_spmv_scratch bytes.");
+  return run_batched_spmv(vt, it, n_rows, n_cols, nnz, data, indices, indptr, batch, X, ldx, Y,
+                          ldy, scratch, s);
+}
+
+extern "C" msx_status msx_csr_batched_spmv(msx_vtype vt, msx_itype it, int64_t n_rows,
+                                           int64_t n_cols, int64_t nnz, const void *data,
+                                           const void *indices, const void *indptr, int64_t batch,
+                                           const void *X, int64_t ldx, void *Y, int64_t ldy,
+                                           void *stream_v) {
+  clear_error();
+  msx_status st = check_batched_spmv(vt, it, n_rows, n_cols, nnz, data, indices, indptr, batch, X,
+                                     ldx, Y, ldy);
+  if (st != MSX_OK) return st;
+  const size_t bytes = msx_csr_batched_spmv_scratch(vt, n_rows, n_cols, batch);
+  auto stream = static_cast<hipStream_t>(stream_v);
+  void *scratch = nullptr;
+  if (bytes > 0) MSX_HIP_TRY(hipMallocAsync(&scratch, bytes, stream));
+  st = msx_csr_batched_spmv_ws(vt, it, n_rows, n_cols, nnz, data, indices, indptr, batch, X, ldx,
+                               Y, ldy, scratch, bytes, stream_v);
+  if (scratch == nullptr) return st;
   const hipError_t e = hipFreeAsync(scratch, stream);
   if (st == MSX_OK && e != hipSuccess) return hip_fail(e, "csr_batched_matvec scratch release");
   return st;

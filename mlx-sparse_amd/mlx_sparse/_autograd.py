@@ -25,7 +25,10 @@ runs (per-range partial outputs added in range order).
 
 from __future__ import annotations
 
+import inspect
+
 import torch
+from torch.autograd import forward_ad
 
 import mlx_sparse._native as _native
 
@@ -70,8 +73,8 @@ def rmatvec(a, data: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     _, indices, indptr = a.buffers(data.device)
     ah = _adjoint_csr(a, data)
     if ah is not None:
-        d, i, p = ah.buffers(data.device)
-        return _native.csr_matvec(d, i, p, g, ah.shape, plan=ah.plan(data.device))
+        (d, i, p), plan = ah.prepared(data.device)
+        return _native.csr_matvec(d, i, p, g, ah.shape, plan=plan)
     return _native.csr_matvec_transpose(_conj(data), indices, indptr, g, a.shape)
 
 
@@ -80,9 +83,19 @@ def rmatmat(a, data: torch.Tensor, G: torch.Tensor) -> torch.Tensor:
     _, indices, indptr = a.buffers(data.device)
     ah = _adjoint_csr(a, data)
     if ah is not None:
-        d, i, p = ah.buffers(data.device)
-        return _native.csr_matmul(d, i, p, G, ah.shape, plan=ah.plan(data.device))
+        (d, i, p), plan = ah.prepared(data.device)
+        return _native.csr_matmul(d, i, p, G, ah.shape, plan=plan)
     return _native.csr_matmul_transpose(_conj(data), indices, indptr, G, a.shape)
+
+
+def _call(function, *args):
+    """``function.apply(*args)``; its forward alone where no derivative of it
+    can be asked for (a plain backward pass: gradients off, no transform and
+    no forward-mode level active)."""
+    if (torch.is_grad_enabled() or torch._C._are_functorch_transforms_active()
+            or forward_ad._current_level >= 0):
+        return function.apply(*args)
+    return function.forward(*args)
 
 
 _SECOND_ORDER = ("second-order derivatives of CSR products with respect to the stored values "
@@ -102,8 +115,8 @@ class CSRMatVec(torch.autograd.Function):
 
     @staticmethod
     def forward(data, x, a, planned=True):
-        _, indices, indptr = a.buffers(data.device)
         plan = _own_plan(a, data) if planned else None
+        _, indices, indptr = a.buffers(data.device)
         return _native.csr_matvec(data, indices, indptr, x, a.shape, plan=plan)
 
     @staticmethod
@@ -119,9 +132,9 @@ class CSRMatVec(torch.autograd.Function):
         data, x = ctx.saved_tensors
         g_data = g_x = None
         if ctx.needs_input_grad[0]:
-            g_data = MatVecDataVjp.apply(x, g, ctx.a)
+            g_data = _call(MatVecDataVjp, x, g, ctx.a)
         if ctx.needs_input_grad[1]:
-            g_x = AdjointMatVec.apply(data, g, ctx.a, ctx.planned)
+            g_x = _call(AdjointMatVec, data, g, ctx.a, ctx.planned)
         return g_data, g_x, None, None
 
     @staticmethod
@@ -169,9 +182,9 @@ class CSRMatMul(torch.autograd.Function):
         data, X = ctx.saved_tensors
         g_data = g_X = None
         if ctx.needs_input_grad[0]:
-            g_data = MatMulDataVjp.apply(X, G, ctx.a)
+            g_data = _call(MatMulDataVjp, X, G, ctx.a)
         if ctx.needs_input_grad[1]:
-            g_X = AdjointMatMul.apply(data, G, ctx.a, ctx.planned)
+            g_X = _call(AdjointMatMul, data, G, ctx.a, ctx.planned)
         return g_data, g_X, None, None
 
     @staticmethod
@@ -252,11 +265,11 @@ class MatVecDataVjp(torch.autograd.Function):
 
     @staticmethod
     def forward(x, g, a):
-        _, indices, indptr = a.buffers(x.device)
         # the gradient does not read the values: the plan serves whatever
         # values it is bound to
+        (_, indices, indptr), plan = a.prepared(x.device)
         return _native.csr_matvec_data_vjp(indices, indptr, _conj(x), g.contiguous(), a.shape,
-                                           plan=a.plan(x.device))
+                                           plan=plan)
 
     @staticmethod
     def setup_context(ctx, inputs, output):
@@ -284,3 +297,11 @@ class MatMulDataVjp(torch.autograd.Function):
     @staticmethod
     def backward(ctx, go):
         raise NotImplementedError(_SECOND_ORDER)
+
+
+# torch binds the default arguments of a forward that has its own
+# setup_context by its signature, on every call; kept on the function it is
+# not worked out anew (15 us a call).
+for _function in (CSRMatVec, CSRMatMul, AdjointMatVec, AdjointMatMul, MatVecDataVjp,
+                  MatMulDataVjp):
+    _function.forward.__signature__ = inspect.signature(_function.forward)

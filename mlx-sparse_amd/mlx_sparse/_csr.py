@@ -26,6 +26,8 @@ from dataclasses import dataclass, field
 
 import torch
 
+from mlx_sparse import runtime
+from mlx_sparse._ext_loader import extension
 from mlx_sparse._typing import Shape2D, ValidationMode
 from mlx_sparse._validation import (
     ensure_array,
@@ -36,14 +38,23 @@ from mlx_sparse._validation import (
 )
 
 
-def _stamp(t: torch.Tensor) -> tuple[int, int]:
-    """Storage address and version counter of a tensor: what a cache entry
-    built from it must still match.  Inference tensors keep no version
-    counter; they count as unchanged while their storage is."""
-    try:
-        return (t.data_ptr(), t._version)
-    except RuntimeError:
-        return (t.data_ptr(), -1)
+# Cache keys of a device: building its name anew cost 1 us a call.
+_DEVICE_NAMES: dict[torch.device, str] = {}
+
+
+def _device_name(device: torch.device) -> str:
+    name = _DEVICE_NAMES.get(device)
+    if name is None:
+        name = _DEVICE_NAMES.setdefault(device, str(device))
+    return name
+
+
+def _indexed(device) -> torch.device:
+    if not isinstance(device, torch.device):
+        device = torch.device(device)
+    if device.type == "cuda" and device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
+    return device
 
 
 @dataclass(frozen=True, slots=True)
@@ -103,17 +114,19 @@ class CSRArray:
 
     # -- device copies and plans -----------------------------------------
     def _stamps(self) -> tuple:
-        return (_stamp(self.data), _stamp(self.indices), _stamp(self.indptr))
+        """Storage address and version counter of each buffer: what a cache
+        entry built from them must still match.  Inference tensors keep no
+        version counter; they count as unchanged while their storage is."""
+        return extension().stamps(self.data, self.indices, self.indptr)
 
     def buffers(self, device) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
         """``(data, indices, indptr)`` contiguous on ``device`` (cached; a
         tensor already contiguous on ``device`` is used as it is, a copy is
         made again when its source changed)."""
-        device = torch.device(device)
-        if device.type == "cuda" and device.index is None:
-            device = torch.device("cuda", torch.cuda.current_device())
-        key = ("buffers", str(device))
-        now = self._stamps()
+        return self._buffers(_indexed(device), self._stamps())
+
+    def _buffers(self, device: torch.device, now: tuple):
+        key = ("buffers", _device_name(device))
         hit = self._cache.get(key)
         if hit is not None and hit[0] == now:
             return hit[1]
@@ -128,30 +141,35 @@ class CSRArray:
         """The GPU plan for ``device``, bound to :meth:`buffers` (None on the
         CPU, or when the ``gpu_plan`` runtime option is off).  Built once;
         refreshed when the values changed, rebuilt when the structure did."""
-        from mlx_sparse import runtime
+        device = _indexed(device if device is not None else self.device)
+        return self.prepared(device)[1] if device.type == "cuda" and runtime.gpu_plan() else None
 
-        device = torch.device(device) if device is not None else self.device
-        if device.type != "cuda" or not runtime.get(runtime.RuntimeOption.GPU_PLAN):
-            return None
-        data, indices, indptr = self.buffers(device)
-        key = ("plan", str(indptr.device))
+    def prepared(self, device) -> tuple:
+        """``(buffers(device), plan(device))``, the cached state looked up
+        and checked once for both."""
+        device = _indexed(device)
         now = self._stamps()
+        bufs = self._buffers(device, now)
+        if device.type != "cuda" or not runtime.gpu_plan():
+            return bufs, None
+        key = ("plan", _device_name(device))
         hit = self._cache.get(key)
         if hit is not None:
             built, plan = hit
             if built[1:] == now[1:]:
                 if built[0] != now[0]:
-                    plan.refresh(data)
+                    plan.refresh(bufs[0])
                     self._cache[key] = (now, plan)
-                return plan
+                return bufs, plan
         from mlx_sparse import _native
 
         # bound to these buffers: may hold a reordered copy of the values
+        data, indices, indptr = bufs
         plan = _native.csr_plan(indptr, self.shape[0], self.nnz, data=data, indices=indices,
                                 n_cols=self.shape[1],
                                 slice_mode=int(runtime.get(runtime.RuntimeOption.GPU_SLICE)))
         self._cache[key] = (now, plan)
-        return plan
+        return bufs, plan
 
     def _with_values(self, data: torch.Tensor) -> "CSRArray":
         """The same structure with other values, taking over this array's

@@ -14,6 +14,7 @@ from __future__ import annotations
 import math
 
 import torch
+from torch.autograd import forward_ad
 
 import mlx_sparse._native as _native
 from mlx_sparse._csr import CSRArray
@@ -35,10 +36,10 @@ def _tracked(*tensors: torch.Tensor) -> bool:
     open) or a torch.func transform (vmap, grad, jvp) is active."""
     if torch._C._are_functorch_transforms_active():
         return True
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
-        return True
-    from torch.autograd import forward_ad
-
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if t.requires_grad:
+                return True
     return forward_ad._current_level >= 0
 
 
@@ -66,8 +67,8 @@ def csr_matvec(a: CSRArray, x) -> torch.Tensor:
         from mlx_sparse._autograd import CSRMatVec
 
         return CSRMatVec.apply(a.data.to(x.device), x, a, True)
-    data, indices, indptr = a.buffers(device)
-    return _native.csr_matvec(data, indices, indptr, x, a.shape, plan=a.plan(device))
+    (data, indices, indptr), plan = a.prepared(device)
+    return _native.csr_matvec(data, indices, indptr, x, a.shape, plan=plan)
 
 
 def _csr_matmul_rank2(a: CSRArray, rhs: torch.Tensor) -> torch.Tensor:
@@ -76,9 +77,9 @@ def _csr_matmul_rank2(a: CSRArray, rhs: torch.Tensor) -> torch.Tensor:
         from mlx_sparse._autograd import CSRMatMul
 
         return CSRMatMul.apply(a.data.to(rhs.device), rhs, a, True)
-    data, indices, indptr = a.buffers(rhs.device)
     # the cached bound plan carries the column windows of the row tiles
-    return _native.csr_matmul(data, indices, indptr, rhs, a.shape, plan=a.plan(rhs.device))
+    (data, indices, indptr), plan = a.prepared(rhs.device)
+    return _native.csr_matmul(data, indices, indptr, rhs, a.shape, plan=plan)
 
 
 def _csr_matmul_batched(a: CSRArray, rhs: torch.Tensor) -> torch.Tensor:

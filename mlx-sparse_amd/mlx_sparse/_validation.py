@@ -12,6 +12,8 @@ from collections.abc import Sequence
 import numpy as np
 import torch
 
+from mlx_sparse._device import default_torch_device
+from mlx_sparse._ext_loader import extension
 from mlx_sparse._typing import INDEX_DTYPES, VALUE_DTYPES, Shape2D, ValidationMode
 
 
@@ -39,9 +41,9 @@ def normalize_validation_mode(validate: ValidationMode) -> str:
 
 def ensure_array(value, *, dtype=None, device=None) -> torch.Tensor:
     """Convert to a tensor on ``device`` (the default device when None)."""
-    from mlx_sparse._device import default_torch_device
-
-    target = default_torch_device() if device is None else torch.device(device)
+    target = default_torch_device() if device is None else device
+    if not isinstance(target, torch.device):
+        target = torch.device(target)
     if isinstance(value, torch.Tensor):
         t = value
     elif isinstance(value, np.ndarray):
@@ -123,6 +125,9 @@ def validate_csr_values(indices, indptr, shape: Shape2D, nnz: int) -> None:
 
 
 def validate_csr_matvec_inputs(data, indices, indptr, x, shape: Shape2D) -> None:
+    # the checks below in one native call; they word the error when it fails
+    if extension().product_operands_ok(data, indices, indptr, x, 1, shape[0], shape[1]):
+        return
     validate_csr_metadata(data, indices, indptr, shape)
     if x.ndim != 1:
         raise ValueError(f"csr_matvec expects a rank-1 RHS, got shape={_shape(x)}.")
@@ -140,6 +145,8 @@ def validate_csr_matvec_inputs(data, indices, indptr, x, shape: Shape2D) -> None
 
 
 def validate_csr_matmul_inputs(data, indices, indptr, rhs, shape: Shape2D) -> None:
+    if extension().product_operands_ok(data, indices, indptr, rhs, 2, shape[0], shape[1]):
+        return
     validate_csr_metadata(data, indices, indptr, shape)
     if rhs.ndim != 2:
         raise ValueError(f"csr_matmul expects a rank-2 RHS, got shape={_shape(rhs)}.")

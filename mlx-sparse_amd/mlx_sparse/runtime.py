@@ -78,6 +78,12 @@ def get(option: RuntimeOption | str) -> Any:
     return True if raw is None else _parse_bool(raw)
 
 
+def gpu_plan() -> bool:
+    """``get(RuntimeOption.GPU_PLAN)``, asked on every product."""
+    raw = os.environ.get("MLX_SPARSE_GPU_PLAN")
+    return True if raw is None else _parse_bool(raw)
+
+
 def _normalize_option(option) -> str:
     if isinstance(option, RuntimeOption):
         return option.value

@@ -9,12 +9,18 @@
 // `csr_matvec_data_vjp` / `csr_matmul_data_vjp`; the solvers, :1470-1482
 // `csr_gmres` among them): same names and argument
 // order (data, indices, indptr, x | rhs, n_rows, n_cols).  Arrays are torch
-// tensors; the module reads their pointer, dtype, shape, strides and device
-// through the tensor's Python attributes, so no torch headers are compiled
-// here.  Inputs are made contiguous (the reference's mx::contiguous), the
+// tensors; the module takes the at::Tensor out of the Python object and reads
+// its pointer, dtype, shape, strides and device from it (through the tensor's
+// Python attributes a call of five operands spent 10 us here, more than the
+// launch).  Inputs are made contiguous (the reference's mx::contiguous), the
 // output is allocated with torch.empty on the inputs' device, device work is
 // ordered on torch's current stream for that device, and errors surface as
 // ValueError (std::invalid_argument), RuntimeError or MemoryError.
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/autograd/python_variable.h>
+
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 
@@ -39,70 +45,106 @@ using msx::DType;
 
 namespace {
 
+// Looked up once and never released: at exit the interpreter is gone before
+// static objects are.
 py::module_ &torch() {
-  static py::module_ mod = py::module_::import("torch");
-  return mod;
+  static auto *mod = new py::module_(py::module_::import("torch"));
+  return *mod;
 }
 
-DType dtype_of(const std::string &name) {
-  if (name == "float32") return DType::Float32;
-  if (name == "float16") return DType::Float16;
-  if (name == "bfloat16") return DType::BFloat16;
-  if (name == "complex64") return DType::Complex64;
-  if (name == "int32") return DType::Int32;
-  if (name == "int64") return DType::Int64;
-  return DType::Other;
+DType dtype_of(at::ScalarType t) {
+  switch (t) {
+  case at::kFloat: return DType::Float32;
+  case at::kHalf: return DType::Float16;
+  case at::kBFloat16: return DType::BFloat16;
+  case at::kComplexFloat: return DType::Complex64;
+  case at::kInt: return DType::Int32;
+  case at::kLong: return DType::Int64;
+  default: return DType::Other;
+  }
 }
 
-std::string dtype_name(py::handle dtype) {
-  std::string s = py::str(dtype);
-  const std::string prefix = "torch.";
-  if (s.rfind(prefix, 0) == 0) s = s.substr(prefix.size());
-  return s;
+// torch's spelling of a dtype, for error texts.
+std::string dtype_name(at::ScalarType t) {
+  switch (t) {
+  case at::kFloat: return "float32";
+  case at::kHalf: return "float16";
+  case at::kBFloat16: return "bfloat16";
+  case at::kComplexFloat: return "complex64";
+  case at::kInt: return "int32";
+  case at::kLong: return "int64";
+  case at::kShort: return "int16";
+  case at::kDouble: return "float64";
+  case at::kComplexDouble: return "complex128";
+  case at::kBool: return "bool";
+  case at::kByte: return "uint8";
+  case at::kChar: return "int8";
+  default: return c10::toString(t);
+  }
 }
 
-int device_index(py::handle tensor) {
-  py::object dev = tensor.attr("device");
-  const std::string type = py::str(dev.attr("type"));
-  if (type == "cpu") return -1;
-  if (type != "cuda") throw std::invalid_argument("mlx_sparse supports cpu and HIP (cuda) tensors only, got " + type + ".");
-  py::object idx = dev.attr("index");
-  return idx.is_none() ? torch().attr("cuda").attr("current_device")().cast<int>() : idx.cast<int>();
+DType dtype_of(py::handle dtype) {
+  if (!THPDtype_Check(dtype.ptr())) return DType::Other;
+  return dtype_of(reinterpret_cast<THPDtype *>(dtype.ptr())->scalar_type);
 }
 
-ArrayView view_of(py::handle t) {
+const at::Tensor &tensor_of(py::handle t) {
+  if (!THPVariable_Check(t.ptr())) throw py::type_error("mlx_sparse expects a torch tensor.");
+  return THPVariable_Unpack(t.ptr());
+}
+
+int current_device() {
+  static auto *f = new py::object(torch().attr("_C").attr("_cuda_getDevice"));
+  return (*f)().cast<int>();
+}
+
+int device_index(const at::Tensor &t) {
+  const at::Device d = t.device();
+  if (d.is_cpu()) return -1;
+  if (!d.is_cuda())
+    throw std::invalid_argument("mlx_sparse supports cpu and HIP (cuda) tensors only, got " +
+                                c10::DeviceTypeName(d.type(), true) + ".");
+  return d.has_index() ? d.index() : current_device();
+}
+
+ArrayView view_of(const at::Tensor &t) {
   ArrayView v;
-  v.dtype_name = dtype_name(t.attr("dtype"));
-  v.dtype = dtype_of(v.dtype_name);
-  v.ndim = t.attr("dim")().cast<int>();
+  v.dtype_name = dtype_name(t.scalar_type());
+  v.dtype = dtype_of(t.scalar_type());
+  v.ndim = static_cast<int>(t.dim());
   if (v.ndim <= 3) {
-    auto shape = t.attr("shape").cast<std::vector<int64_t>>();
-    auto strides = t.attr("stride")().cast<std::vector<int64_t>>();
     for (int i = 0; i < v.ndim; ++i) {
-      v.shape[i] = shape[i];
-      v.strides[i] = strides[i];
+      v.shape[i] = t.size(i);
+      v.strides[i] = t.stride(i);
     }
   }
-  v.ptr = reinterpret_cast<void *>(t.attr("data_ptr")().cast<uintptr_t>());
   v.device = device_index(t);
+  v.ptr = t.data_ptr();
   return v;
 }
 
+ArrayView view_of(py::handle t) { return view_of(tensor_of(t)); }
+
 py::object as_tensor(py::handle obj) {
-  if (py::isinstance(obj, torch().attr("Tensor"))) return py::reinterpret_borrow<py::object>(obj);
+  if (THPVariable_Check(obj.ptr())) return py::reinterpret_borrow<py::object>(obj);
   return torch().attr("as_tensor")(obj);
 }
 
-py::object contiguous(py::handle obj) { return as_tensor(obj).attr("contiguous")(); }
+py::object contiguous(py::handle obj) {
+  py::object t = as_tensor(obj);
+  if (tensor_of(t).is_contiguous()) return t;
+  return t.attr("contiguous")();
+}
 
+// The stream torch's current stream of `device` wraps.
 void *stream_for(int device) {
   if (device < 0) return nullptr;
-  const int current = torch().attr("cuda").attr("current_device")().cast<int>();
+  const int current = current_device();
   if (current != device)
     throw std::invalid_argument("mlx_sparse: GPU operands must be on the current device (cuda:" +
                                 std::to_string(current) + "), got cuda:" + std::to_string(device) + ".");
-  py::object s = torch().attr("cuda").attr("current_stream")(device);
-  return reinterpret_cast<void *>(s.attr("cuda_stream").cast<uintptr_t>());
+  static auto *f = new py::object(torch().attr("_C").attr("_cuda_getCurrentRawStream"));
+  return reinterpret_cast<void *>((*f)(device).cast<uintptr_t>());
 }
 
 // Owner of a device plan; destroyed with the Python object.
@@ -187,11 +229,52 @@ const msx_csr_plan *plan_ptr(const py::object &plan) {
   return plan.cast<std::shared_ptr<Plan>>()->p;
 }
 
-py::object empty_like_out(const ArrayView &data, py::handle data_obj, py::tuple shape) {
-  py::dict kw;
-  kw["dtype"] = data_obj.attr("dtype");
-  kw["device"] = data_obj.attr("device");
-  return torch().attr("empty")(shape, **kw);
+py::object empty_like_out(const ArrayView &, py::handle like, py::tuple shape) {
+  std::vector<int64_t> dims;
+  for (py::handle d : shape) dims.push_back(d.cast<int64_t>());
+  return py::reinterpret_steal<py::object>(
+      THPVariable_Wrap(at::empty(dims, tensor_of(like).options().requires_grad(false))));
+}
+
+// Device scratch of one call from torch's caching allocator (the stream-ordered
+// one of the C ABI gives its memory back at every synchronisation and maps it
+// anew: 40 us a call), kept until the call's kernels are enqueued; torch
+// orders its reuse on the current stream.
+at::Tensor scratch_for(msx::ExecContext &ctx, py::handle like, size_t bytes) {
+  if (ctx.stream == nullptr && tensor_of(like).is_cpu()) return {};
+  if (bytes == 0) return {};
+  at::Tensor t = at::empty({static_cast<int64_t>(bytes)}, at::TensorOptions().dtype(at::kByte).device(tensor_of(like).device()));
+  ctx.scratch = t.data_ptr();
+  ctx.scratch_bytes = bytes;
+  return t;
+}
+
+// What CSRArray's caches are checked against: storage address and version
+// counter of the three buffers (inference tensors keep no counter: -1).
+py::tuple stamps(py::handle data, py::handle indices, py::handle indptr) {
+  const auto one = [](py::handle o) {
+    const at::Tensor &t = tensor_of(o);
+    return py::make_tuple(reinterpret_cast<uintptr_t>(t.data_ptr()),
+                          t.is_inference() ? int64_t{-1} : static_cast<int64_t>(t._version()));
+  };
+  return py::make_tuple(one(data), one(indices), one(indptr));
+}
+
+// True when a product's operands pass every metadata check (ranks, dtypes,
+// lengths): the Python validators, which word the errors, run only otherwise.
+bool product_operands_ok(py::handle data_o, py::handle indices_o, py::handle indptr_o,
+                         py::handle rhs_o, int rhs_ndim, int64_t n_rows, int64_t n_cols) {
+  for (py::handle h : {data_o, indices_o, indptr_o, rhs_o})
+    if (!THPVariable_Check(h.ptr())) return false;
+  const at::Tensor &data = tensor_of(data_o), &indices = tensor_of(indices_o),
+                   &indptr = tensor_of(indptr_o), &rhs = tensor_of(rhs_o);
+  if (data.dim() != 1 || indices.dim() != 1 || indptr.dim() != 1 || rhs.dim() != rhs_ndim)
+    return false;
+  const DType vt = dtype_of(data.scalar_type()), it = dtype_of(indices.scalar_type());
+  return msx::is_value_dtype(vt) && rhs.scalar_type() == data.scalar_type() &&
+         (it == DType::Int32 || it == DType::Int64) &&
+         indptr.scalar_type() == indices.scalar_type() && data.size(0) == indices.size(0) &&
+         indptr.size(0) == n_rows + 1 && rhs.size(0) == n_cols;
 }
 
 py::object csr_matvec(py::handle data_o, py::handle indices_o, py::handle indptr_o, py::handle x_o,
@@ -250,6 +333,10 @@ py::object csr_batched_matvec(py::handle data_o, py::handle indices_o, py::handl
   ctx.n_threads = n_threads;
   ctx.stream = vd.device >= 0 ? stream_for(vd.device) : nullptr;
   if (vd.device >= 0) {
+    const at::Tensor scratch = scratch_for(
+        ctx, data, msx::is_value_dtype(vd.dtype)
+                       ? msx_csr_batched_spmv_scratch(msx::to_vtype(vd.dtype), n_rows, n_cols, vr.shape[0])
+                       : 0);
     msx::csr_batched_matvec(vd, vi, vp, vr, vo, n_rows, n_cols, ctx);
   } else {
     py::gil_scoped_release nogil;
@@ -596,8 +683,7 @@ py::tuple mm_read_csr(const std::string &path, py::object dtype, py::object inde
                       int n_threads) {
   msx_mm_info info{};
   msx::check_status(msx_mm_info_read(path.c_str(), &info), "mmread");
-  const std::string vname = dtype_name(dtype), iname = dtype_name(index_dtype);
-  const DType vd = dtype_of(vname), id = dtype_of(iname);
+  const DType vd = dtype_of(dtype), id = dtype_of(index_dtype);
   if (!msx::is_value_dtype(vd))
     throw std::invalid_argument("mmread dtype must be float32, float16, bfloat16 or complex64.");
   if (id != DType::Int32 && id != DType::Int64)
@@ -622,7 +708,7 @@ py::tuple mm_read_csr(const std::string &path, py::object dtype, py::object inde
 py::object mm_read_dense(const std::string &path, py::object dtype, int n_threads) {
   msx_mm_info info{};
   msx::check_status(msx_mm_info_read(path.c_str(), &info), "mmread");
-  const DType vd = dtype_of(dtype_name(dtype));
+  const DType vd = dtype_of(dtype);
   if (!msx::is_value_dtype(vd))
     throw std::invalid_argument("mmread dtype must be float32, float16, bfloat16 or complex64.");
   py::object out = host_empty(info.n_rows * info.n_cols, dtype);
@@ -714,6 +800,11 @@ PYBIND11_MODULE(_ext, m) {
 
   m.def("_compiled_capabilities", &compiled_capabilities,
         "Return compile-time native backend facts for capability reporting.");
+  m.def("stamps", &stamps, py::arg("data"), py::arg("indices"), py::arg("indptr"),
+        "(storage address, version counter) of each of the three buffers.");
+  m.def("product_operands_ok", &product_operands_ok, py::arg("data"), py::arg("indices"),
+        py::arg("indptr"), py::arg("rhs"), py::arg("rhs_ndim"), py::arg("n_rows"),
+        py::arg("n_cols"), "True when a product's operands pass every metadata check.");
   m.def("csr_plan", &make_plan, py::arg("indptr"), py::arg("n_rows"), py::arg("nnz"),
         py::arg("block_nnz") = 0, py::arg("data") = py::none(), py::arg("indices") = py::none(),
         py::arg("n_cols") = -1, py::arg("slice_mode") = 0,

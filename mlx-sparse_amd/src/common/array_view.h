@@ -3,6 +3,7 @@
 // layer itself never sees a framework type.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include <string>
@@ -39,6 +40,8 @@ struct ArrayView {
 struct ExecContext {
   void *stream = nullptr;  // hipStream_t for device arrays
   int n_threads = 0;       // host worker count (0: resolve from the environment)
+  void *scratch = nullptr;  // device scratch, as many bytes as the call asks for
+  size_t scratch_bytes = 0;
 };
 
 }  // namespace msx

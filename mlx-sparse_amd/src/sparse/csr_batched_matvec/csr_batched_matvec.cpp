@@ -40,9 +40,9 @@ void csr_batched_matvec(const ArrayView &data, const ArrayView &indices, const A
   const msx_itype it = to_itype(indices.dtype);
   const int64_t nnz = data.size();
   if (data.device >= 0) {
-    check_status(msx_csr_batched_spmv(vt, it, n_rows, n_cols, nnz, data.ptr, indices.ptr,
-                                      indptr.ptr, batch, rhs.ptr, n_cols, out.ptr, n_rows,
-                                      ctx.stream),
+    check_status(msx_csr_batched_spmv_ws(vt, it, n_rows, n_cols, nnz, data.ptr, indices.ptr,
+                                         indptr.ptr, batch, rhs.ptr, n_cols, out.ptr, n_rows,
+                                         ctx.scratch, ctx.scratch_bytes, ctx.stream),
                  "csr_batched_matvec");
   } else {
     check_status(msx_csr_batched_spmv_cpu(vt, it, n_rows, n_cols, nnz, data.ptr, indices.ptr,
