@@ -84,6 +84,11 @@ __device__ inline int64_t clamp64(int64_t v, int64_t lo, int64_t hi) {
 __device__ inline float amul(float a, float b) { return a * b; }
 __device__ inline c64 amul(c64 a, c64 b) { return vmul<C64>(a, b); }
 
+__device__ inline float shfl_lane(float v, int src) { return __shfl(v, src, kWave); }
+__device__ inline c64 shfl_lane(c64 v, int src) {
+  return c64{__shfl(v.re, src, kWave), __shfl(v.im, src, kWave)};
+}
+
 __device__ inline void atomic_acc(float *p, float v) { unsafeAtomicAdd(p, v); }
 __device__ inline void atomic_acc(c64 *p, c64 v) {
   float *f = reinterpret_cast<float *>(p);
@@ -385,7 +390,16 @@ msx_status transpose_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const vo
 }
 
 // ---------------------------------------------------------------------------
-// Transposed products by atomic scatter.  G lanes per row of A.
+// Transposed products by atomic scatter.  Bound by the atomics: about 20 G
+// requests a second over the chip, whatever their scope, a request being the
+// up to 64 consecutive bytes that one instruction adds to.
+
+// A^T x, G lanes per row of A: the lanes of neighbouring rows then add to
+// neighbouring columns on stencils and bands (64 consecutive positions a wave
+// instead: 3D Poisson 100^3 48 -> 82 us).  A row of more than kWholeRow values
+// is left to the whole workgroup after its other rows (300,007 power-law rows,
+// the longest 37,500: 2,165 -> 237 us at 1,024).
+constexpr int64_t kWholeRow = 256;
 
 template <class V, class I>
 __global__ void __launch_bounds__(kThreads)
@@ -394,39 +408,79 @@ __global__ void __launch_bounds__(kThreads)
                  typename V::Acc *__restrict__ acc, int64_t n_rows, int64_t nnz, int64_t n_cols,
                  int G) {
   using A = typename V::Acc;
-  const int64_t rows_per_block = kThreads / G;
+  __shared__ int32_t whole[kThreads];
+  __shared__ int n_whole;
+  const int rows_per_block = kThreads / G;
   const int j = threadIdx.x % G;
-  for (int64_t row = static_cast<int64_t>(blockIdx.x) * rows_per_block + threadIdx.x / G;
-       row < n_rows; row += static_cast<int64_t>(gridDim.x) * rows_per_block) {
-    const int64_t s = clamp64(static_cast<int64_t>(indptr[row]), 0, nnz);
-    const int64_t e = clamp64(static_cast<int64_t>(indptr[row + 1]), s, nnz);
+  const auto scatter = [&](int64_t row, int64_t s, int64_t e, int first, int step) {
     const A xr = V::widen(x[row]);
-    for (int64_t p = s + j; p < e; p += G) {
+    for (int64_t p = s + first; p < e; p += step) {
       const int64_t c = static_cast<int64_t>(indices[p]);
       if (c >= 0 && c < n_cols) atomic_acc(acc + c, amul(V::widen(data[p]), xr));
     }
+  };
+  if (threadIdx.x == 0) n_whole = 0;
+  __syncthreads();
+  for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows_per_block; r0 < n_rows;
+       r0 += static_cast<int64_t>(gridDim.x) * rows_per_block) {
+    const int64_t row = r0 + threadIdx.x / G;
+    if (row < n_rows) {
+      const int64_t s = clamp64(static_cast<int64_t>(indptr[row]), 0, nnz);
+      const int64_t e = clamp64(static_cast<int64_t>(indptr[row + 1]), s, nnz);
+      if (e - s <= kWholeRow) scatter(row, s, e, j, G);
+      else if (j == 0) whole[atomicAdd(&n_whole, 1)] = static_cast<int32_t>(row);
+    }
+    __syncthreads();
+    const int n = n_whole;  // at most a row per group
+    for (int i = 0; i < n; ++i) {
+      const int64_t w = whole[i];
+      const int64_t s = clamp64(static_cast<int64_t>(indptr[w]), 0, nnz);
+      const int64_t e = clamp64(static_cast<int64_t>(indptr[w + 1]), s, nnz);
+      scatter(w, s, e, static_cast<int>(threadIdx.x), kThreads);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) n_whole = 0;
+    __syncthreads();
   }
 }
 
-// One wave per row of A; lanes over the k columns of X.
+// A^T X: a wave takes 64 consecutive positions and finds their rows
+// (msx_rows.h), so a row of any length is shared by as many waves as its
+// values need; then its values in turn, L lanes (a power of two, at least k up
+// to 64) over the k columns of one value's output row, 64 / L values at a time.  One wave per row and one value at a time: 1 M values in
+// rows of 16, k = 4 116 -> 57 us; power-law rows, 100,007 of them, 1.2 M
+// values, k = 32 5,230 -> 112 us (the longest row's 12,500 values in
+// sequence).  Sorting the values into a transpose for the call was slower
+// (150 us and 60 us a million values, then the gathers).
 template <class V, class I>
 __global__ void __launch_bounds__(kThreads)
     scatter_spmm(const typename V::Storage *__restrict__ data, const I *__restrict__ indices,
                  const I *__restrict__ indptr, const typename V::Storage *__restrict__ X,
                  int64_t ldx, typename V::Acc *__restrict__ acc, int64_t lda, int64_t n_rows,
-                 int64_t nnz, int64_t n_cols, int64_t k) {
+                 int64_t nnz, int64_t n_cols, int64_t k, int L) {
+  using A = typename V::Acc;
   const int lane = threadIdx.x % kWave;
+  const int sub = lane / L, q0 = lane % L, per = kWave / L;
+  const int64_t p_end = clamp64(static_cast<int64_t>(indptr[n_rows]), 0, nnz);
+  const int64_t p_begin = clamp64(static_cast<int64_t>(indptr[0]), 0, p_end);
   const int64_t waves = static_cast<int64_t>(gridDim.x) * (kThreads / kWave);
-  for (int64_t row = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave;
-       row < n_rows; row += waves) {
-    const int64_t s = clamp64(static_cast<int64_t>(indptr[row]), 0, nnz);
-    const int64_t e = clamp64(static_cast<int64_t>(indptr[row + 1]), s, nnz);
-    for (int64_t p = s; p < e; ++p) {
-      const int64_t c = static_cast<int64_t>(indices[p]);
-      if (c < 0 || c >= n_cols) continue;
-      const typename V::Acc a = V::widen(data[p]);
-      for (int64_t q = lane; q < k; q += kWave)
-        atomic_acc(acc + c * lda + q, amul(a, V::widen(X[row * ldx + q])));
+  for (int64_t b = (static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave) * kWave;
+       b < p_end; b += waves * kWave) {
+    const int64_t p = b + lane;
+    const bool held = p >= p_begin && p < p_end;
+    int64_t c = held ? static_cast<int64_t>(indices[p]) : -1;
+    if (c >= n_cols) c = -1;
+    const A a = held ? V::widen(data[p]) : A{};
+    int64_t row = wave_row_of(indptr, n_rows, b, lane);
+    row = lane_rows(indptr, n_rows, b, lane, row);
+    for (int t = 0; t < kWave; t += per) {
+      const int cv = __shfl(static_cast<int>(c), t + sub, kWave);
+      const int rv = __shfl(static_cast<int>(row), t + sub, kWave);
+      const A av = shfl_lane(a, t + sub);
+      if (cv < 0) continue;
+      for (int64_t q = q0; q < k; q += L)
+        atomic_acc(acc + static_cast<int64_t>(cv) * lda + q,
+                   amul(av, V::widen(X[static_cast<int64_t>(rv) * ldx + q])));
     }
   }
 }
@@ -755,10 +809,13 @@ struct SpmmTransposeOp {
     }
     hipLaunchKernelGGL((fill_rows<A>), dim3(grid_for(n_cols * k)), dim3(kThreads), 0, stream, acc,
                        n_cols, k, lda);
-    hipLaunchKernelGGL((scatter_spmm<V, I>), dim3(grid_for(n_rows * kWave)), dim3(kThreads), 0,
-                       stream, static_cast<const S *>(data), static_cast<const I *>(indices),
-                       static_cast<const I *>(indptr), static_cast<const S *>(X), ldx, acc, lda,
-                       n_rows, nnz, n_cols, k);
+    int L = 1;
+    while (L < k && L < kWave) L <<= 1;
+    if (n_rows > 0)
+      hipLaunchKernelGGL((scatter_spmm<V, I>), dim3(grid_for(nnz)), dim3(kThreads), 0, stream,
+                         static_cast<const S *>(data), static_cast<const I *>(indices),
+                         static_cast<const I *>(indptr), static_cast<const S *>(X), ldx, acc, lda,
+                         n_rows, nnz, n_cols, k, L);
     if (!direct)
       hipLaunchKernelGGL((narrow_rows<V>), dim3(grid_for(n_cols * k)), dim3(kThreads), 0, stream,
                          acc, n_cols, k, lda, static_cast<S *>(Y), ldy);

@@ -185,3 +185,28 @@ def test_spmm_rows_of_any_length_and_alignment(vtype):
             got = out[:, skip:skip + k].contiguous()
             assert to_numpy(got).tobytes() == want.tobytes(), (k, pad)
             assert bool((out[:, :skip] == 7).all()) and bool((out[:, skip + k:] == 7).all())
+
+
+@pytest.mark.parametrize("kind", ["one_row", "edges", "empty_runs", "skewed"])
+@pytest.mark.parametrize("vtype", ["float32", "bfloat16", "complex64"])
+def test_transposed_products_by_positions(kind, vtype):
+    """The atomic transposed products on every row structure, k from 1 past a
+    wave's lanes: small integers, so every order of additions is exact."""
+    rng = np.random.default_rng(59)
+    lengths = _row_lengths(kind, rng)
+    n_rows, n_cols = len(lengths), 777
+    index_dtype = np.int64 if kind == "edges" else np.int32
+    indices, indptr = _csr(rng, lengths, n_cols, index_dtype, bad=0.02)
+    small = lambda *shape: storage(rng.integers(-1, 2, shape).astype(np.float64), vtype)  # noqa: E731
+    data = small(indices.size)
+    good = (indices >= 0) & (indices < n_cols)
+    held, cols = np.where(good, data, np.zeros_like(data)), np.where(good, indices, 0)
+    d, i, p = to_torch(data, vtype, DEV), to_torch(indices, None, DEV), to_torch(indptr, None, DEV)
+    for k in (0, 1, 2, 3, 5, 8, 33, 64, 70):
+        X = small(n_rows, k) if k else small(n_rows)
+        want = orc.csr_transpose_product(held, cols.astype(index_dtype), indptr, X, n_rows, n_cols,
+                                         vtype=vtype)
+        print(f"transposed products {kind} {vtype} k={k}", flush=True)
+        f = _capi.spmm_transpose if k else _capi.spmv_transpose
+        got = f(d, i, p, to_torch(X, vtype, DEV), n_rows, n_cols)
+        np.testing.assert_array_equal(to_numpy(got), want)
