@@ -106,8 +106,8 @@ __global__ void __launch_bounds__(kSolverThreads)
 // p.ap, p.p, ap.ap, non-finite p/ap.  From the second iteration on, first
 // checks the previous direction pass (any non-finite p stops with -3) and
 // commits the residual norm it left.
-__global__ void __launch_bounds__(kSolverThreads)
-    cg_alpha(const float *__restrict__ p, const float *__restrict__ ap, int64_t n, int32_t it,
+__device__ inline void
+    cg_alpha_pass(const float *__restrict__ p, const float *__restrict__ ap, int64_t n, int32_t it,
              const double *dir_part, double *part, int nparts, CgState *st) {
   if (!st->running) return;
   double pin[kSlots] = {0.0, 0.0, 0.0, 0.0};
@@ -134,11 +134,16 @@ __global__ void __launch_bounds__(kSolverThreads)
   });
   write_partials(v, part);
 }
+__global__ void __launch_bounds__(kSolverThreads)
+    cg_alpha(const float *__restrict__ p, const float *__restrict__ ap, int64_t n, int32_t it,
+             const double *dir_part, double *part, int nparts, CgState *st) {
+  cg_alpha_pass(p, ap, n, it, dir_part, part, nparts, st);
+}
 
 // alpha from the alpha pass (cg.cpp:158-199), then x += alpha p and
 // r -= alpha ap in double, rounded once; r.r and non-finite counts.
-__global__ void __launch_bounds__(kSolverThreads)
-    cg_update(float *__restrict__ x, float *__restrict__ r, const float *__restrict__ p,
+__device__ inline void
+    cg_update_pass(float *__restrict__ x, float *__restrict__ r, const float *__restrict__ p,
               const float *__restrict__ ap, int64_t n, int32_t it, const double *alpha_part,
               double *part, int nparts, CgState *st) {
   if (!st->running) return;
@@ -184,11 +189,17 @@ __global__ void __launch_bounds__(kSolverThreads)
   });
   write_partials(v, part);
 }
+__global__ void __launch_bounds__(kSolverThreads)
+    cg_update(float *__restrict__ x, float *__restrict__ r, const float *__restrict__ p,
+              const float *__restrict__ ap, int64_t n, int32_t it, const double *alpha_part,
+              double *part, int nparts, CgState *st) {
+  cg_update_pass(x, r, p, ap, n, it, alpha_part, part, nparts, st);
+}
 
 // Convergence and beta from the update pass (cg.cpp:200-238), then
 // p = r + beta p; non-finite p values are counted for the next alpha pass.
-__global__ void __launch_bounds__(kSolverThreads)
-    cg_direction(const float *__restrict__ r, float *__restrict__ p, int64_t n, int32_t it,
+__device__ inline void
+    cg_direction_pass(const float *__restrict__ r, float *__restrict__ p, int64_t n, int32_t it,
                  const double *upd_part, double *part, int nparts, CgState *st) {
   if (!st->running) return;
   double pin[kSlots];
@@ -229,6 +240,11 @@ __global__ void __launch_bounds__(kSolverThreads)
     st->completed = it;
     st->rr_next = rr_new;
   }
+}
+__global__ void __launch_bounds__(kSolverThreads)
+    cg_direction(const float *__restrict__ r, float *__restrict__ p, int64_t n, int32_t it,
+                 const double *upd_part, double *part, int nparts, CgState *st) {
+  cg_direction_pass(r, p, n, it, upd_part, part, nparts, st);
 }
 
 // One workgroup, after the last launched iteration: settles the check the
@@ -299,8 +315,8 @@ __global__ void __launch_bounds__(kSolverThreads)
   }
 }
 
-__global__ void __launch_bounds__(kSolverThreads)
-    pcg_alpha(const float *__restrict__ p, const float *__restrict__ ap, int64_t n, int32_t it,
+__device__ inline void
+    pcg_alpha_pass(const float *__restrict__ p, const float *__restrict__ ap, int64_t n, int32_t it,
               double *part, CgState *st) {
   if (!st->running) return;
   if (it > 1 && blockIdx.x == 0 && threadIdx.x == 0) st->rr = st->rr_next;
@@ -313,11 +329,16 @@ __global__ void __launch_bounds__(kSolverThreads)
   })
   write_partials(v, part);
 }
+__global__ void __launch_bounds__(kSolverThreads)
+    pcg_alpha(const float *__restrict__ p, const float *__restrict__ ap, int64_t n, int32_t it,
+              double *part, CgState *st) {
+  pcg_alpha_pass(p, ap, n, it, part, st);
+}
 
 // alpha (pcg.cpp:165-184), then x += alpha p; r -= alpha ap; z = inv_diag r;
 // r.r and r.z.
-__global__ void __launch_bounds__(kSolverThreads)
-    pcg_update(float *__restrict__ x, float *__restrict__ r, float *__restrict__ z,
+__device__ inline void
+    pcg_update_pass(float *__restrict__ x, float *__restrict__ r, float *__restrict__ z,
                const float *__restrict__ p, const float *__restrict__ ap,
                const float *__restrict__ inv_diag, int64_t n, int32_t it,
                const double *alpha_part, double *part, int nparts, CgState *st) {
@@ -357,10 +378,17 @@ __global__ void __launch_bounds__(kSolverThreads)
   });
   write_partials(v, part);
 }
+__global__ void __launch_bounds__(kSolverThreads)
+    pcg_update(float *__restrict__ x, float *__restrict__ r, float *__restrict__ z,
+               const float *__restrict__ p, const float *__restrict__ ap,
+               const float *__restrict__ inv_diag, int64_t n, int32_t it,
+               const double *alpha_part, double *part, int nparts, CgState *st) {
+  pcg_update_pass(x, r, z, p, ap, inv_diag, n, it, alpha_part, part, nparts, st);
+}
 
 // Convergence, rho and beta (pcg.cpp:186-232), then p = z + beta p.
-__global__ void __launch_bounds__(kSolverThreads)
-    pcg_direction(const float *__restrict__ z, float *__restrict__ p, int64_t n, int32_t it,
+__device__ inline void
+    pcg_direction_pass(const float *__restrict__ z, float *__restrict__ p, int64_t n, int32_t it,
                   const double *upd_part, int nparts, CgState *st) {
   if (!st->running) return;
   double pin[kSlots];
@@ -391,11 +419,45 @@ __global__ void __launch_bounds__(kSolverThreads)
   for_rounds<2>(vec, n, first, [&](int64_t i, const float(&e)[2]) { p[i] = e[0] + beta * e[1]; });
   if (lead) st->rr_next = rho_new;
 }
+__global__ void __launch_bounds__(kSolverThreads)
+    pcg_direction(const float *__restrict__ z, float *__restrict__ p, int64_t n, int32_t it,
+                  const double *upd_part, int nparts, CgState *st) {
+  pcg_direction_pass(z, p, n, it, upd_part, nparts, st);
+}
 
 __global__ void pcg_finish(CgState *st) {
   if (threadIdx.x == 0 && st->running) st->running = 0;
 }
 
+
+// Iterations k0 .. k1 of a small system in one workgroup (msx_solver.h): the
+// passes above in turn, until the solve stops.
+template <class I, bool J, int kValues>
+__global__ void __launch_bounds__(kSolverThreads)
+    cg_group(GroupMatrix<I> a, float *x, float *r, float *z, float *p, float *ap,
+             const float *inv_diag, int64_t n, int32_t k0, int32_t k1, double *alpha_part,
+             double *upd_part, double *dir_part, CgState *st) {
+  extern __shared__ __align__(16) float lds[];
+  GroupValues<kValues> m;
+  group_load(a, m, lds);
+  for (int32_t k = k0; k <= k1; ++k) {
+    if (!group_running(st)) return;
+    group_spmv(a, m, p, ap, lds);
+    if constexpr (J) {
+      pcg_alpha_pass(p, ap, n, k, alpha_part, st);
+      __syncthreads();
+      pcg_update_pass(x, r, z, p, ap, inv_diag, n, k, alpha_part, upd_part, 1, st);
+      __syncthreads();
+      pcg_direction_pass(z, p, n, k, upd_part, 1, st);
+    } else {
+      cg_alpha_pass(p, ap, n, k, dir_part, alpha_part, 1, st);
+      __syncthreads();
+      cg_update_pass(x, r, p, ap, n, k, alpha_part, upd_part, 1, st);
+      __syncthreads();
+      cg_direction_pass(r, p, n, k, upd_part, dir_part, 1, st);
+    }
+  }
+}
 
 __global__ void copy_vec(const float *__restrict__ src, float *__restrict__ dst, int64_t n) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kSolverThreads + threadIdx.x; i < n;
@@ -411,6 +473,7 @@ struct Solve {
   const msx_csr_plan *plan;
   hipStream_t stream;
   uint32_t blocks;
+  bool group;  // the iterations run in one workgroup
 };
 
 msx_status spmv(const Solve &s, const float *x, float *y) {
@@ -423,7 +486,7 @@ msx_status spmv(const Solve &s, const float *x, float *y) {
 // The residual of the schedule: sqrt(r.r) (CG) or of the true r.r (PCG).
 template <class Step>
 msx_status drive(const Solve &s, int64_t maxiter, CgState *st_dev, CgState *st_host, bool pcg,
-                 Step step) {
+                 Step steps) {
   auto residual = [&]() {
     const double rr = pcg ? st_host->true_rr : st_host->rr;
     return std::sqrt(std::max(rr, 0.0));
@@ -432,11 +495,9 @@ msx_status drive(const Solve &s, int64_t maxiter, CgState *st_dev, CgState *st_h
   BatchSchedule schedule;
   int64_t batch = schedule.next(0, residual(), st_host->tol);  // the start's state
   while (done < maxiter) {
-    const int64_t todo = std::min(batch, maxiter - done);
-    for (int64_t k = 0; k < todo; ++k) {
-      msx_status e = step(static_cast<int32_t>(done + k + 1));
-      if (e != MSX_OK) return e;
-    }
+    const int64_t todo = std::min(s.group ? kGroupBatch : batch, maxiter - done);
+    const msx_status e = steps(static_cast<int32_t>(done + 1), static_cast<int32_t>(done + todo));
+    if (e != MSX_OK) return e;
     done += todo;
     MSX_HIP_TRY(hipMemcpyAsync(st_host, st_dev, sizeof(CgState), hipMemcpyDeviceToHost, s.stream));
     MSX_HIP_TRY(hipStreamSynchronize(s.stream));
@@ -529,7 +590,33 @@ msx_status solve(const Solve &s, const float *b, const float *x0, const float *i
       MSX_HIP_TRY(hipGetLastError());
       return MSX_OK;
     };
-    e = drive(s, maxiter, st, &host, pcg, step);
+    // iterations k0 .. k1, enqueued
+    auto steps = [&](int32_t k0, int32_t k1) -> msx_status {
+      if (s.group) {
+        auto go = [&](auto kern, auto matrix) -> msx_status {
+          MSX_HIP_TRY(group_lds_limit(reinterpret_cast<const void *>(kern)));
+          hipLaunchKernelGGL(kern, dim3(1), block, group_lds(n, s.nnz), s.stream, matrix, x, r, z,
+                             p, ap, inv_diag, n, k0, k1, alpha_part, upd_part, dir_part, st);
+          MSX_HIP_TRY(hipGetLastError());
+          return MSX_OK;
+        };
+        auto of = [&](auto index, auto values) -> msx_status {
+          using I = decltype(index);
+          constexpr int kValues = decltype(values)::value;
+          const GroupMatrix<I> a = group_matrix<I>(s);
+          return pcg ? go(cg_group<I, true, kValues>, a) : go(cg_group<I, false, kValues>, a);
+        };
+        const std::integral_constant<int, kGroupFew> few{};
+        const std::integral_constant<int, kGroupMany> many{};
+        const bool small = s.nnz <= int64_t{kGroupFew} * kSolverThreads;
+        if (s.it == MSX_I32) return small ? of(int32_t{}, few) : of(int32_t{}, many);
+        return small ? of(int64_t{}, few) : of(int64_t{}, many);
+      }
+      for (int32_t k = k0; k <= k1; ++k)
+        if (const msx_status es = step(k); es != MSX_OK) return es;
+      return MSX_OK;
+    };
+    e = drive(s, maxiter, st, &host, pcg, steps);
     if (e != MSX_OK) return e;
     if (pcg)
       hipLaunchKernelGGL(pcg_finish, dim3(1), dim3(kWave), 0, s.stream, st);
@@ -573,7 +660,8 @@ extern "C" msx_status msx_csr_cg(msx_itype it, int64_t n, int64_t nnz, const flo
   st = check_plan("csr_cg", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
   const Solve s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
-                blocks_for(n)};
+                in_one_group(plan, n, nnz, kGroupMany) ? 1 : blocks_for(n),
+                in_one_group(plan, n, nnz, kGroupMany)};
   return solve(s, b, x0, nullptr, x, rtol, atol, maxiter, result);
 }
 
@@ -591,6 +679,7 @@ extern "C" msx_status msx_csr_pcg_jacobi(msx_itype it, int64_t n, int64_t nnz, c
   st = check_plan("csr_pcg_jacobi", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
   const Solve s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
-                blocks_for(n)};
+                in_one_group(plan, n, nnz, kGroupMany) ? 1 : blocks_for(n),
+                in_one_group(plan, n, nnz, kGroupMany)};
   return solve(s, b, x0, inv_diag, x, rtol, atol, maxiter, result);
 }

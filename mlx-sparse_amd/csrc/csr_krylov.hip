@@ -175,8 +175,8 @@ __device__ inline bool bi_close(const double (&t)[kSlots], int32_t k, BiState *s
 // k - 1 first.  J: also p_hat = inv_diag p (its non-finite entries counted
 // with p's).
 template <bool J>
-__global__ void __launch_bounds__(kSolverThreads)
-    bi_p(const float *__restrict__ r, float *__restrict__ p, const float *__restrict__ v,
+__device__ inline void
+    bi_p_pass(const float *__restrict__ r, float *__restrict__ p, const float *__restrict__ v,
          const float *__restrict__ inv_diag, float *__restrict__ p_hat, int64_t n, int32_t k,
          int close_prev, const double *dots, double *part, int nparts, BiState *st) {
   if (!st->running) return;
@@ -236,10 +236,17 @@ __global__ void __launch_bounds__(kSolverThreads)
   write_partials(acc, part);
   if (lead()) st->rho[k & 1] = rho;
 }
+template <bool J>
+__global__ void __launch_bounds__(kSolverThreads)
+    bi_p(const float *__restrict__ r, float *__restrict__ p, const float *__restrict__ v,
+         const float *__restrict__ inv_diag, float *__restrict__ p_hat, int64_t n, int32_t k,
+         int close_prev, const double *dots, double *part, int nparts, BiState *st) {
+  bi_p_pass<J>(r, p, v, inv_diag, p_hat, n, k, close_prev, dots, part, nparts, st);
+}
 
 // The p pass's non-finite count, then r_hat.v and v.v.
-__global__ void __launch_bounds__(kSolverThreads)
-    bi_v(const float *__restrict__ r_hat, const float *__restrict__ v, int64_t n, int32_t k,
+__device__ inline void
+    bi_v_pass(const float *__restrict__ r_hat, const float *__restrict__ v, int64_t n, int32_t k,
          const double *p_part, double *part, int nparts, BiState *st) {
   if (!st->running) return;
   double pin[kSlots];
@@ -261,13 +268,18 @@ __global__ void __launch_bounds__(kSolverThreads)
   });
   write_partials(acc, part);
 }
+__global__ void __launch_bounds__(kSolverThreads)
+    bi_v(const float *__restrict__ r_hat, const float *__restrict__ v, int64_t n, int32_t k,
+         const double *p_part, double *part, int nparts, BiState *st) {
+  bi_v_pass(r_hat, v, n, k, p_part, part, nparts, st);
+}
 
 // alpha (bicgstab.cpp:232-255); s = r - alpha v, x += alpha p; s.s of the
 // unrounded s, non-finite count.  J: `p` is p_hat, and s_hat = inv_diag s
 // is written too (slot 2: its non-finite count).
 template <bool J>
-__global__ void __launch_bounds__(kSolverThreads)
-    bi_s(const float *__restrict__ r, const float *__restrict__ v, const float *__restrict__ p,
+__device__ inline void
+    bi_s_pass(const float *__restrict__ r, const float *__restrict__ v, const float *__restrict__ p,
          const float *__restrict__ inv_diag, float *__restrict__ x, float *__restrict__ s,
          float *__restrict__ s_hat, int64_t n, int32_t k, const double *v_part, double *part,
          int nparts, BiState *st) {
@@ -316,14 +328,22 @@ __global__ void __launch_bounds__(kSolverThreads)
     st->completed = k;
   }
 }
+template <bool J>
+__global__ void __launch_bounds__(kSolverThreads)
+    bi_s(const float *__restrict__ r, const float *__restrict__ v, const float *__restrict__ p,
+         const float *__restrict__ inv_diag, float *__restrict__ x, float *__restrict__ s,
+         float *__restrict__ s_hat, int64_t n, int32_t k, const double *v_part, double *part,
+         int nparts, BiState *st) {
+  bi_s_pass<J>(r, v, p, inv_diag, x, s, s_hat, n, k, v_part, part, nparts, st);
+}
 
 // The s-check (bicgstab.cpp:270-287; skipped when the host has already
 // run it), then t.s and t.t.  J: the reported residual becomes ||s||
 // (preconditioners/bicgstab/bicgstab.cpp:314), and a non-finite s_hat ends
 // the solve after the check.
 template <bool J>
-__global__ void __launch_bounds__(kSolverThreads)
-    bi_t(const float *__restrict__ s, const float *__restrict__ t_vec, int64_t n, int32_t k,
+__device__ inline void
+    bi_t_pass(const float *__restrict__ s, const float *__restrict__ t_vec, int64_t n, int32_t k,
          int check, const double *s_part, double *part, int nparts, BiState *st) {
   if (!st->running) return;
   double pin[kSlots] = {0.0, 0.0, 0.0, 0.0};
@@ -361,13 +381,19 @@ __global__ void __launch_bounds__(kSolverThreads)
   });
   write_partials(acc, part);
 }
+template <bool J>
+__global__ void __launch_bounds__(kSolverThreads)
+    bi_t(const float *__restrict__ s, const float *__restrict__ t_vec, int64_t n, int32_t k,
+         int check, const double *s_part, double *part, int nparts, BiState *st) {
+  bi_t_pass<J>(s, t_vec, n, k, check, s_part, part, nparts, st);
+}
 
 // omega (bicgstab.cpp:290-305); x += omega s, r = s - omega t.  Slots: r.r
 // of the unrounded r, non-finite count, r_hat.r and r.r of the stored r
 // (the next iteration's rho and r.r).  J: x += omega s_hat.
 template <bool J>
-__global__ void __launch_bounds__(kSolverThreads)
-    bi_r(const float *__restrict__ s, const float *__restrict__ t_vec,
+__device__ inline void
+    bi_r_pass(const float *__restrict__ s, const float *__restrict__ t_vec,
          const float *__restrict__ s_hat, float *__restrict__ x, float *__restrict__ r,
          const float *__restrict__ r_hat, int64_t n, int32_t k, const double *t_part,
          double *part, int nparts, BiState *st) {
@@ -410,6 +436,14 @@ __global__ void __launch_bounds__(kSolverThreads)
   });
   write_partials(acc, part);
   if (lead()) st->omega = omega;
+}
+template <bool J>
+__global__ void __launch_bounds__(kSolverThreads)
+    bi_r(const float *__restrict__ s, const float *__restrict__ t_vec,
+         const float *__restrict__ s_hat, float *__restrict__ x, float *__restrict__ r,
+         const float *__restrict__ r_hat, int64_t n, int32_t k, const double *t_part,
+         double *part, int nparts, BiState *st) {
+  bi_r_pass<J>(s, t_vec, s_hat, x, r, r_hat, n, k, t_part, part, nparts, st);
 }
 
 // One workgroup after the last launched iteration k: closes it.
@@ -600,8 +634,8 @@ __device__ inline bool mr_close(const double (&t)[kSlots], int32_t k, MrState *s
 // Closes iteration k - 1, then v = r2 / beta (minres.cpp:212-222); J: `r2`
 // is y = M r2, and a failed beta test is -2.
 template <bool J>
-__global__ void __launch_bounds__(kSolverThreads)
-    mr_v(const float *__restrict__ r2, float *__restrict__ v, int64_t n, int32_t k,
+__device__ inline void
+    mr_v_pass(const float *__restrict__ r2, float *__restrict__ v, int64_t n, int32_t k,
          const double *res_part, int nparts, MrState *st) {
   if (!st->running) return;
   double pin[kSlots] = {0.0, 0.0, 0.0, 0.0};
@@ -624,11 +658,17 @@ __global__ void __launch_bounds__(kSolverThreads)
     v[i] = static_cast<float>(inv_beta * static_cast<double>(e[0]));
   });
 }
+template <bool J>
+__global__ void __launch_bounds__(kSolverThreads)
+    mr_v(const float *__restrict__ r2, float *__restrict__ v, int64_t n, int32_t k,
+         const double *res_part, int nparts, MrState *st) {
+  mr_v_pass<J>(r2, v, n, k, res_part, nparts, st);
+}
 
 // av -= shift v, av -= (beta / oldb) r1 from the second iteration on
 // (minres.cpp:224-236); v.av.
-__global__ void __launch_bounds__(kSolverThreads)
-    mr_a(const float *__restrict__ v, float *__restrict__ av, const float *__restrict__ r1,
+__device__ inline void
+    mr_a_pass(const float *__restrict__ v, float *__restrict__ av, const float *__restrict__ r1,
          float shift, int64_t n, int32_t k, double *part, MrState *st) {
   if (!st->running) return;
   const Givens g = st->g[(k - 1) & 1];
@@ -657,12 +697,17 @@ __global__ void __launch_bounds__(kSolverThreads)
   }
   write_partials(acc, part);
 }
+__global__ void __launch_bounds__(kSolverThreads)
+    mr_a(const float *__restrict__ v, float *__restrict__ av, const float *__restrict__ r1,
+         float shift, int64_t n, int32_t k, double *part, MrState *st) {
+  mr_a_pass(v, av, r1, shift, n, k, part, st);
+}
 
 // alfa; av -= (alfa / beta) r2 (minres.cpp:238-246); the new r2's norm.
 // J: also y = inv_diag av, and the sum is av.y.
 template <bool J>
-__global__ void __launch_bounds__(kSolverThreads)
-    mr_b(float *__restrict__ av, const float *__restrict__ r2, const float *__restrict__ inv_diag,
+__device__ inline void
+    mr_b_pass(float *__restrict__ av, const float *__restrict__ r2, const float *__restrict__ inv_diag,
          float *__restrict__ y, int64_t n, int32_t k, const double *a_part, double *part,
          int nparts, MrState *st) {
   if (!st->running) return;
@@ -696,13 +741,20 @@ __global__ void __launch_bounds__(kSolverThreads)
   });
   write_partials(acc, part);
 }
+template <bool J>
+__global__ void __launch_bounds__(kSolverThreads)
+    mr_b(float *__restrict__ av, const float *__restrict__ r2, const float *__restrict__ inv_diag,
+         float *__restrict__ y, int64_t n, int32_t k, const double *a_part, double *part,
+         int nparts, MrState *st) {
+  mr_b_pass<J>(av, r2, inv_diag, y, n, k, a_part, part, nparts, st);
+}
 
 // The next Givens rotation (minres.cpp:248-275), then w and x
 // (minres.cpp:277-290).  The new w is written over w2 (the host swaps the
 // two).  Slots: non-finite count.  J: a failed beta test is -2.
 template <bool J>
-__global__ void __launch_bounds__(kSolverThreads)
-    mr_x(const float *__restrict__ v, const float *__restrict__ w, float *__restrict__ w2,
+__device__ inline void
+    mr_x_pass(const float *__restrict__ v, const float *__restrict__ w, float *__restrict__ w2,
          float *__restrict__ x, int64_t n, int32_t k, const double *a_part,
          const double *b_part, double *part, int nparts, MrState *st) {
   if (!st->running) return;
@@ -760,11 +812,18 @@ __global__ void __launch_bounds__(kSolverThreads)
     st->completed = k;
   }
 }
+template <bool J>
+__global__ void __launch_bounds__(kSolverThreads)
+    mr_x(const float *__restrict__ v, const float *__restrict__ w, float *__restrict__ w2,
+         float *__restrict__ x, int64_t n, int32_t k, const double *a_part,
+         const double *b_part, double *part, int nparts, MrState *st) {
+  mr_x_pass<J>(v, w, w2, x, n, k, a_part, b_part, part, nparts, st);
+}
 
 // The x pass's non-finite count, then b - (A x - shift x) (A x in ax).
 // Slots: r.r, non-finite count.
-__global__ void __launch_bounds__(kSolverThreads)
-    mr_r(const float *__restrict__ b, const float *__restrict__ x, const float *__restrict__ ax,
+__device__ inline void
+    mr_r_pass(const float *__restrict__ b, const float *__restrict__ x, const float *__restrict__ ax,
          float shift, int64_t n, int32_t k, const double *x_part, double *part, int nparts,
          MrState *st) {
   if (!st->running) return;
@@ -788,6 +847,12 @@ __global__ void __launch_bounds__(kSolverThreads)
   });
   write_partials(acc, part);
 }
+__global__ void __launch_bounds__(kSolverThreads)
+    mr_r(const float *__restrict__ b, const float *__restrict__ x, const float *__restrict__ ax,
+         float shift, int64_t n, int32_t k, const double *x_part, double *part, int nparts,
+         MrState *st) {
+  mr_r_pass(b, x, ax, shift, n, k, x_part, part, nparts, st);
+}
 
 // One workgroup after the last launched iteration k: closes it.
 __global__ void __launch_bounds__(kSolverThreads)
@@ -797,6 +862,67 @@ __global__ void __launch_bounds__(kSolverThreads)
   read_totals(res_part, nparts, t);
   if (!mr_close(t, k, st)) return;
   if (threadIdx.x == 0) st->running = 0;
+}
+
+// Iterations k0 .. k1 of a small system in one workgroup (msx_solver.h): the
+// passes above in turn, until the solve stops or pauses.
+template <class I, bool J>
+__global__ void __launch_bounds__(kSolverThreads)
+    bi_group(GroupMatrix<I> a, float *x, float *r, float *r_hat, float *p, float *v, float *sv,
+             float *tv, float *p_hat, float *s_hat, const float *inv_diag, int64_t n, int32_t k0,
+             int32_t k1, int close_prev, const double *dots, double *p_part, double *v_part,
+             double *s_part, double *t_part, double *r_part, BiState *st) {
+  extern __shared__ __align__(16) float lds[];
+  GroupValues<kGroupFew> m;
+  group_load(a, m, lds);
+  for (int32_t k = k0; k <= k1; ++k) {
+    if (!group_running(st)) return;
+    bi_p_pass<J>(r, p, v, inv_diag, p_hat, n, k, close_prev, dots, p_part, 1, st);
+    if (!group_running(st)) return;
+    group_spmv(a, m, p_hat, v, lds);
+    bi_v_pass(r_hat, v, n, k, p_part, v_part, 1, st);
+    __syncthreads();
+    bi_s_pass<J>(r, v, p_hat, inv_diag, x, sv, s_hat, n, k, v_part, s_part, 1, st);
+    if (!group_running(st)) return;
+    group_spmv(a, m, s_hat, tv, lds);
+    bi_t_pass<J>(sv, tv, n, k, 1, s_part, t_part, 1, st);
+    __syncthreads();
+    bi_r_pass<J>(sv, tv, s_hat, x, r, r_hat, n, k, t_part, r_part, 1, st);
+    close_prev = 1;
+    dots = r_part;
+  }
+}
+
+template <class I, bool J>
+__global__ void __launch_bounds__(kSolverThreads)
+    mr_group(GroupMatrix<I> a, const float *b, float *x, float *r1, float *r2, float *av, float *v,
+             float *w, float *w2, float *q, float *y, const float *inv_diag, float shift, int64_t n,
+             int32_t k0, int32_t k1, double *a_part, double *b_part, double *x_part,
+             double *res_part, MrState *st) {
+  extern __shared__ __align__(16) float lds[];
+  GroupValues<kGroupFew> m;
+  group_load(a, m, lds);
+  for (int32_t k = k0; k <= k1; ++k) {
+    if (!group_running(st)) return;
+    mr_v_pass<J>(J ? y : r2, v, n, k, res_part, 1, st);
+    if (!group_running(st)) return;
+    group_spmv(a, m, v, av, lds);
+    mr_a_pass(v, av, r1, shift, n, k, a_part, st);
+    __syncthreads();
+    mr_b_pass<J>(av, r2, inv_diag, y, n, k, a_part, b_part, 1, st);
+    __syncthreads();
+    mr_x_pass<J>(v, w, w2, x, n, k, a_part, b_part, x_part, 1, st);
+    float *t = r1;  // as the host's swaps: r1 <- r2 <- av, w2 <- w <- new w
+    r1 = r2;
+    r2 = av;
+    av = t;
+    t = w;
+    w = w2;
+    w2 = t;
+    if (!group_running(st)) return;
+    group_spmv(a, m, x, q, lds);
+    mr_r_pass(b, x, q, shift, n, k, x_part, res_part, 1, st);
+  }
 }
 
 __global__ void copy_vec(const float *__restrict__ src, float *__restrict__ dst, int64_t n) {
@@ -823,7 +949,23 @@ struct System {
   hipStream_t stream;
   dim3 grid, block;
   int nparts;
+  bool group;  // the iterations run in one workgroup
 };
+
+// Launches KERNEL<I, J>(matrix, args...) in one workgroup.
+template <class Kernel32, class Kernel64, class... Args>
+msx_status launch_group(const System &s, Kernel32 k32, Kernel64 k64, Args... args) {
+  const size_t lds = group_lds(s.n, s.nnz);
+  if (s.it == MSX_I32) {
+    MSX_HIP_TRY(group_lds_limit(reinterpret_cast<const void *>(k32)));
+    hipLaunchKernelGGL(k32, dim3(1), s.block, lds, s.stream, group_matrix<int32_t>(s), args...);
+  } else {
+    MSX_HIP_TRY(group_lds_limit(reinterpret_cast<const void *>(k64)));
+    hipLaunchKernelGGL(k64, dim3(1), s.block, lds, s.stream, group_matrix<int64_t>(s), args...);
+  }
+  MSX_HIP_TRY(hipGetLastError());
+  return MSX_OK;
+}
 
 msx_status spmv(const System &s, const float *x, float *y) {
   return launch_spmv(MSX_F32, s.it, s.n, s.n, s.nnz, s.data, s.indices, s.indptr, x, y, s.plan,
@@ -861,6 +1003,13 @@ msx_status read_state(const System &s, const State *dev, State *host) {
   MSX_HIP_TRY(hipMemcpyAsync(host, dev, sizeof(State), hipMemcpyDeviceToHost, s.stream));
   MSX_HIP_TRY(hipStreamSynchronize(s.stream));
   return MSX_OK;
+}
+
+// BiCGSTAB amplifies the rounding of its sums into its iteration count, so it
+// takes the one-workgroup loop only where the sums are grouped as before (one
+// workgroup's passes, up to 2,048 rows): the bits are then the same.
+bool bi_in_one_group(const msx_csr_plan *plan, int64_t n, int64_t nnz) {
+  return in_one_group(plan, n, nnz, kGroupFew) && blocks_for(n) == 1;
 }
 
 // J: the Jacobi loop, inv_diag non-null (p_hat and s_hat in two more
@@ -923,8 +1072,17 @@ msx_status bicgstab(const System &s, const float *b, const float *x0, const floa
   int64_t batch = schedule.next(0, host.residual, host.tol);  // the start's state
   for (;;) {
     if (host.running) {
-      const int64_t last = std::min(maxiter, next + batch - 1);
-      for (int64_t k = next; k <= last; ++k) {
+      const int64_t last = std::min(maxiter, next + (s.group ? kGroupBatch : batch) - 1);
+      if (s.group) {
+        e = launch_group(s, bi_group<int32_t, J>, bi_group<int64_t, J>, x, r, r_hat, p, v, sv, tv,
+                         p_hat, s_hat, inv_diag, n, static_cast<int32_t>(next),
+                         static_cast<int32_t>(last), close_prev, dots, p_part, v_part, s_part,
+                         t_part, r_part, st);
+        if (e != MSX_OK) return e;
+        close_prev = 1;
+        dots = r_part;
+      }
+      for (int64_t k = s.group ? last + 1 : next; k <= last; ++k) {
         const auto kk = static_cast<int32_t>(k);
         hipLaunchKernelGGL(bi_p<J>, s.grid, s.block, 0, s.stream, r, p, v, inv_diag, p_hat, n, kk,
                            close_prev, dots, p_part, np, st);
@@ -1016,8 +1174,19 @@ msx_status minres(const System &s, const float *b, const float *x0, const float 
   BatchSchedule schedule;  // its residual: the last iteration tested on the device
   int64_t batch = schedule.next(0, host.residual, host.tol);  // the start's state
   while (host.running && next <= maxiter) {
-    const int64_t last = std::min(maxiter, next + batch - 1);
-    for (int64_t k = next; k <= last; ++k) {
+    const int64_t last = std::min(maxiter, next + (s.group ? kGroupBatch : batch) - 1);
+    if (s.group) {
+      e = launch_group(s, mr_group<int32_t, J>, mr_group<int64_t, J>, b, x, r1, r2, av, v, w, w2, q,
+                       y, inv_diag, shift, n, static_cast<int32_t>(next),
+                       static_cast<int32_t>(last), a_part, b_part, x_part, res_part, st);
+      if (e != MSX_OK) return e;
+      for (int64_t k = next; k <= last; ++k) {
+        std::swap(r1, r2);
+        std::swap(r2, av);
+        std::swap(w, w2);
+      }
+    }
+    for (int64_t k = s.group ? last + 1 : next; k <= last; ++k) {
       const auto kk = static_cast<int32_t>(k);
       hipLaunchKernelGGL(mr_v<J>, s.grid, s.block, 0, s.stream, J ? y : r2, v, n, kk, res_part,
                          np, st);
@@ -1083,7 +1252,8 @@ extern "C" msx_status msx_csr_bicgstab(msx_itype it, int64_t n, int64_t nnz, con
   if (st != MSX_OK) return st;
   const uint32_t blocks = blocks_for(n);
   const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
-                 dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks)};
+                 dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks),
+                 bi_in_one_group(plan, n, nnz)};
   return bicgstab<false>(s, b, x0, nullptr, x, rtol, atol, maxiter, result);
 }
 
@@ -1104,7 +1274,8 @@ extern "C" msx_status msx_csr_bicgstab_jacobi(msx_itype it, int64_t n, int64_t n
   if (st != MSX_OK) return st;
   const uint32_t blocks = blocks_for(n);
   const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
-                 dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks)};
+                 dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks),
+                 bi_in_one_group(plan, n, nnz)};
   return bicgstab<true>(s, b, x0, inv_diag, x, rtol, atol, maxiter, result);
 }
 
@@ -1118,9 +1289,11 @@ extern "C" msx_status msx_csr_minres(msx_itype it, int64_t n, int64_t nnz, const
   if (st != MSX_OK) return st;
   st = check_plan("csr_minres", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
-  const uint32_t blocks = blocks_for(n);
+  const bool group = in_one_group(plan, n, nnz, kGroupFew);
+  const uint32_t blocks = group ? 1 : blocks_for(n);
   const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
-                 dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks)};
+                 dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks),
+                 group};
   return minres<false>(s, b, x0, nullptr, x, rtol, atol, maxiter, shift, result);
 }
 
@@ -1138,8 +1311,10 @@ extern "C" msx_status msx_csr_minres_jacobi(msx_itype it, int64_t n, int64_t nnz
   if (inv_diag == nullptr) return fail(MSX_EINVAL, "csr_minres_jacobi buffers must be non-NULL.");
   st = check_plan("csr_minres_jacobi", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
-  const uint32_t blocks = blocks_for(n);
+  const bool group = in_one_group(plan, n, nnz, kGroupFew);
+  const uint32_t blocks = group ? 1 : blocks_for(n);
   const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
-                 dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks)};
+                 dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks),
+                 group};
   return minres<true>(s, b, x0, inv_diag, x, rtol, atol, maxiter, shift, result);
 }

@@ -15,6 +15,7 @@
 #include <cmath>
 
 #include "msx_device.h"
+#include "msx_internal.h"
 
 namespace msx {
 namespace solver {
@@ -67,6 +68,11 @@ __device__ inline void load_partials(const double *part, int nparts, double (&v)
 }
 
 __device__ inline void reduce_partials(const double (&v)[kSlots], int nparts, double (&t)[kSlots]) {
+  if (nparts == 1) {  // load_partials gave every thread the one partial
+    for (int k = 0; k < kSlots; ++k) t[k] = v[k];
+    __syncthreads();  // what follows may write the solver state that was read before
+    return;
+  }
   __shared__ double sh[kSlots][kSolverThreads / kWave];
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const bool mine = static_cast<int>(threadIdx.x) < nparts;
@@ -191,6 +197,124 @@ class BatchSchedule {
   int64_t k_ = -1;
   double res_ = 0.0;
 };
+
+// ---------------------------------------------------------------------------
+// Small systems in one workgroup.  Below some thousands of rows an iteration's
+// four to seven kernels take 4 to 5 us each however little they do, and a
+// launch's gap between them; one workgroup that runs the product and the
+// passes of many iterations in turn pays a barrier in their place, at one
+// compute unit's rate.  The passes are the kernels' own, over one block.  The
+// matrix stays in registers for the launch (kValues values a thread), its row
+// pointers in LDS, so a product is one round of gathers of x.
+// Only for row-block plans without long rows (a row is one thread's sum).
+// Whole solves to 1e-5, kernels -> one workgroup, us: CG, Laplacian 30^2 673
+// -> 297, 63^2 726 -> 486; MINRES 35^2 975 -> 411, 63^2 981 -> 951 (there 48
+// values a thread do not fit the registers beside its passes, so MINRES and
+// BiCGSTAB stop at 16); BiCGSTAB 43^2 857 -> 592.  A pass takes about 2.5 us, the
+// latency of its two reductions.
+constexpr int64_t kGroupRows = 4608;
+constexpr int64_t kGroupBatch = 128;  // iterations a launch: it ends with the solve
+constexpr int kGroupFew = 16, kGroupMany = 48;  // values a thread
+
+template <class I>
+struct GroupMatrix {
+  const float *data;
+  const I *indices;
+  const I *indptr;
+  int64_t n, nnz;
+};
+
+// `values`: the most values a thread that the solver's loop is built for.
+inline bool in_one_group(const msx_csr_plan *plan, int64_t n, int64_t nnz, int values) {
+  return plan != nullptr && plan->n_long == 0 && plan->n_panels == 0 && plan->n_slices == 0 &&
+         n <= kGroupRows && nnz <= int64_t{values} * kSolverThreads;
+}
+
+// LDS of a launch: the products of all values, then n + 1 row pointers.
+inline size_t group_lds(int64_t n, int64_t nnz) {
+  return static_cast<size_t>(nnz + n + 1) * sizeof(float);
+}
+inline hipError_t group_lds_limit(const void *kernel) {
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             static_cast<int>(group_lds(kGroupRows, int64_t{kGroupMany} * kSolverThreads)));
+}
+
+template <class I, class System>
+GroupMatrix<I> group_matrix(const System &s) {
+  return {s.data, static_cast<const I *>(s.indices), static_cast<const I *>(s.indptr), s.n, s.nnz};
+}
+
+template <int kValues>
+struct GroupValues {
+  int32_t col[kValues];  // -1: no value, or a column out of range
+  float val[kValues];
+};
+
+// The thread's values (positions threadIdx.x + u * kSolverThreads) into
+// registers and the row pointers, held to [0, nnz], into LDS.
+template <int kValues, class I>
+__device__ inline void group_load(const GroupMatrix<I> &a, GroupValues<kValues> &m, float *lds) {
+  const int tid = static_cast<int>(threadIdx.x);
+  const uint32_t lim = col_limit32(a.n);
+#pragma unroll
+  for (int u = 0; u < kValues; ++u) {
+    const int64_t p = tid + u * kSolverThreads;
+    m.col[u] = -1;
+    m.val[u] = 0.0f;
+    if (p < a.nnz) {
+      const I c = a.indices[p];
+      m.col[u] = col_ok(c, a.n, lim) ? static_cast<int32_t>(c) : -1;
+      m.val[u] = a.data[p];
+    }
+  }
+  int32_t *ip = reinterpret_cast<int32_t *>(lds + a.nnz);
+  for (int64_t r = tid; r <= a.n; r += kSolverThreads) {
+    const int64_t p = static_cast<int64_t>(a.indptr[r]);
+    ip[r] = static_cast<int32_t>(p < 0 ? 0 : (p > a.nnz ? a.nnz : p));
+  }
+  __syncthreads();
+}
+
+// y = A x in one workgroup: all products in LDS, then a row a thread, in
+// stored order, rows of one to four values from their first product.
+template <int kValues, class I>
+__device__ inline void group_spmv(const GroupMatrix<I> &a, const GroupValues<kValues> &m,
+                                  const float *x, float *y, float *lds) {
+  const int tid = static_cast<int>(threadIdx.x);
+  const int nnz = static_cast<int>(a.nnz), n = static_cast<int>(a.n);
+  const int32_t *ip = reinterpret_cast<const int32_t *>(lds + nnz);
+  float xv[kValues];
+#pragma unroll
+  for (int u = 0; u < kValues; ++u) xv[u] = x[m.col[u] < 0 ? 0 : m.col[u]];
+#pragma unroll
+  for (int u = 0; u < kValues; ++u)
+    if (tid + u * kSolverThreads < nnz)
+      lds[tid + u * kSolverThreads] = m.col[u] < 0 ? 0.0f : m.val[u] * xv[u];
+  __syncthreads();
+  constexpr int U = 8;
+  for (int r = tid; r < n; r += kSolverThreads) {
+    int i = ip[r];
+    const int end = ip[r + 1];
+    float sum = i < end && end - i <= 4 ? lds[i++] : 0.0f;
+    for (; i < end; i += U) {
+      float t[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) t[u] = lds[i + u < end ? i + u : i];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i + u < end) sum = sum + t[u];
+    }
+    y[r] = sum;
+  }
+  __syncthreads();
+}
+
+// Whether the solve still runs, read after the pass before.
+template <class State>
+__device__ inline bool group_running(const State *st) {
+  __syncthreads();
+  return *const_cast<const volatile int32_t *>(&st->running) != 0;
+}
 
 // Workgroups of a solver pass over n elements (kUnroll per thread and round).
 inline uint32_t blocks_for(int64_t n) {

@@ -210,3 +210,59 @@ def test_transposed_products_by_positions(kind, vtype):
         f = _capi.spmm_transpose if k else _capi.spmv_transpose
         got = f(d, i, p, to_torch(X, vtype, DEV), n_rows, n_cols)
         np.testing.assert_array_equal(to_numpy(got), want)
+
+
+@pytest.mark.parametrize("solver", ["cg", "pcg", "minres", "bicgstab"])
+@pytest.mark.parametrize("rows", [1, 2, 513, 1500, 2048, 2049, 4608])
+def test_small_systems_in_one_workgroup(solver, rows):
+    """Solves of systems around the one-workgroup loop's sizes, rows of one to
+    nine values (more values a thread than 16 from 2,049 rows on), both index
+    types and a budget that ends inside a launch: status and iterations as
+    the oracle's, x within the tolerance's bound of the float64 solution
+    (condition number at most 5)."""
+    rng = np.random.default_rng(rows)
+    dense = {}
+    for i in range(rows):
+        for j in rng.integers(0, rows, 4):
+            if i != j:
+                v = rng.uniform(-0.2, 0.2)
+                dense[i, int(j)] = dense.get((i, int(j)), 0.0) + v
+                if solver != "bicgstab":
+                    dense[int(j), i] = dense[i, int(j)]
+    near = np.zeros(rows)
+    for (i, _), v in dense.items():
+        near[i] += abs(v)
+    for i in range(rows):
+        dense[i, i] = 2.0 * max(near.max(), 0.5)
+    keys = np.array(sorted(dense))
+    data = np.array([dense[tuple(k)] for k in keys], np.float32)
+    index_dtype = np.int64 if rows % 2 else np.int32
+    indices = keys[:, 1].astype(index_dtype)
+    indptr = np.searchsorted(keys[:, 0], np.arange(rows + 1)).astype(index_dtype)
+    b = rng.standard_normal(rows).astype(np.float32)
+    from scipy import sparse
+    from scipy.sparse.linalg import spsolve
+    exact = spsolve(sparse.csc_matrix((data.astype(np.float64), (keys[:, 0], keys[:, 1])),
+                                      shape=(rows, rows)), b.astype(np.float64))
+    d, i, p = (to_torch(t, None, DEV) for t in (data, indices, indptr))
+    plan = _capi.Plan(p, rows, data.size, data=d, indices=i, n_cols=rows)
+    bt, inv = to_torch(b, None, DEV), 1.0 / data[keys[:, 0] == keys[:, 1]]
+    print(f"one workgroup {solver} {rows}", flush=True)
+    for budget in (200, 2):
+        if solver in ("cg", "pcg"):
+            jac = to_torch(inv.astype(np.float32), None, DEV) if solver == "pcg" else None
+            x, info, res, its = _capi.cg(d, i, p, bt, rtol=1e-5, maxiter=budget, plan=plan,
+                                         inv_diag=jac)
+            want = (orc.csr_pcg_jacobi(data, indices, indptr, b, inv.astype(np.float32), rtol=1e-5,
+                                       maxiter=budget) if jac is not None else
+                    orc.csr_cg(data, indices, indptr, b, rtol=1e-5, maxiter=budget))
+        else:
+            x, info, res, its = _capi.krylov(solver, d, i, p, bt, rtol=1e-5, maxiter=budget,
+                                             plan=plan)
+            f = orc.csr_minres if solver == "minres" else orc.csr_bicgstab
+            want = f(data, indices, indptr, b, rtol=1e-5, maxiter=budget)
+        assert info == want[1] and abs(its - want[3]) <= 1, (info, its, want[1:])
+        if info == 0:
+            # |x - exact| <= cond * rtol * |x|, cond <= (2 + 1) / (2 - 1) of the row sums' bound
+            assert np.linalg.norm(to_numpy(x) - exact) <= 5e-5 * np.linalg.norm(exact)
+    plan.close()
