@@ -72,6 +72,31 @@ def test_batched_spmv_parity_and_strides(vtype, index_dtype):
 
 
 @pytest.mark.parametrize("vtype", VTYPES)
+@pytest.mark.parametrize("n_rows", [301, 262_143, 262_144])  # three vectors widen from 2^18 rows
+def test_batches_of_padded_widths(vtype, n_rows):
+    rng = np.random.default_rng(n_rows)
+    n_cols = 977
+    lengths = rng.integers(0, 3, n_rows)
+    indptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(indptr[-1])
+    indices = rng.integers(0, n_cols, nnz).astype(np.int32)
+    data = _values(rng, nnz, vtype)
+    d, i, p = (to_torch(a, vtype if a is data else None, DEV) for a in (data, indices, indptr))
+    per16 = 16 // data.itemsize
+    # one over, and all of, 2, 3, 5, 6 and 7 sixteen-byte vectors
+    for batch in sorted({2 * per16 + 1, 3 * per16, 5 * per16 + 1, 6 * per16, 7 * per16}):
+        X = _values(rng, (batch, n_cols), vtype)
+        want = _want_vectors(data, indices, indptr, X, n_rows, vtype)
+        Y = torch.zeros((batch, n_rows + 3), dtype=to_torch(X, vtype, DEV).dtype, device=DEV)
+        Y[:, n_rows:] = 2
+        _capi.batched_spmv(d, i, p, to_torch(X, vtype, DEV), n_rows, n_cols, Y=Y, ldx=n_cols,
+                           ldy=n_rows + 3)
+        assert torch.all(Y[:, n_rows:] == 2)
+        np.testing.assert_array_equal(_bytes(to_numpy(Y)[:, :n_rows]), _bytes(want),
+                                      err_msg=f"{vtype} batch={batch}")
+
+
+@pytest.mark.parametrize("vtype", VTYPES)
 def test_batched_spmm_parity_and_batch_strides(vtype):
     rng = np.random.default_rng(6)
     n_rows, n_cols = 900, 700
