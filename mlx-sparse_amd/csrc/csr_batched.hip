@@ -265,16 +265,17 @@ BatchScratch batch_scratch(msx_vtype vt, int64_t n_rows, int64_t n_cols, int64_t
   const int64_t per16 = 16 / sv;
   BatchScratch b;
   int64_t vectors = (batch + per16 - 1) / per16;
-  // Widths that store straight to Y (launch_spmv_batch_rows), where at most a
-  // quarter of the row is padding: without Yt and its transpose.  f32, 100^3
-  // Poisson: 26 right-hand sides 318 -> 166 us, 21 258 -> 152, 11 101 -> 86;
-  // c64, 400,003 banded rows: 14 176 -> 104, 11 144 -> 101.  Three vectors only
-  // from kPadRows rows on: Yt of fewer stays in the caches and the wider Xt
-  // costs as much (216,000 rows 25.5 -> 26.4 us, 200,003 c64 28.7 -> 29.5;
-  // 300,003 c64 60 -> 57, 512,000 47.5 -> 40.6).
+  // Widths that store straight to Y (launch_spmv_batch_rows), without Yt and
+  // its transpose, are worth up to three vectors of padding.  f32, 100^3
+  // Poisson: 26 right-hand sides 318 -> 166 us, 21 258 -> 152, 17 203 -> 143,
+  // 11 101 -> 86; f32, 500,003 random rows, 19 291 -> 206; c64, 400,003 banded
+  // rows: 14 176 -> 104, 11 144 -> 101, 9 124 -> 105.  Three vectors only from
+  // kPadRows rows on: Yt of fewer stays in the caches and the wider Xt costs
+  // as much (216,000 rows 25.5 -> 26.4 us, 200,003 c64 28.7 -> 29.5; 300,003
+  // c64 60 -> 57, 512,000 47.5 -> 40.6).
   constexpr int64_t kPadRows = 1 << 18;
   if (vectors == 3 && n_rows >= kPadRows) vectors = 4;
-  else if (vectors == 6 || vectors == 7) vectors = 8;
+  else if (vectors >= 5 && vectors <= 7) vectors = 8;
   b.kpad = vectors * per16;
   b.bx = static_cast<size_t>(std::max<int64_t>(n_cols, 1) * b.kpad * sv);
   b.by = static_cast<size_t>(n_rows * b.kpad * sv);
