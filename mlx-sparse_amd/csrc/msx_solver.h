@@ -68,7 +68,9 @@ __device__ inline void load_partials(const double *part, int nparts, double (&v)
 }
 
 __device__ inline void reduce_partials(const double (&v)[kSlots], int nparts, double (&t)[kSlots]) {
-  if (nparts == 1) {  // load_partials gave every thread the one partial
+  // The loops of one workgroup pass a literal 1: load_partials gave every thread
+  // the one partial.  Not a test at run time, which cost bi_v and bi_r 0.4 us of 8.
+  if (__builtin_constant_p(nparts) && nparts == 1) {
     for (int k = 0; k < kSlots; ++k) t[k] = v[k];
     __syncthreads();  // what follows may write the solver state that was read before
     return;
