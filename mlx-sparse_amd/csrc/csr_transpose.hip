@@ -468,13 +468,15 @@ __global__ void __launch_bounds__(kThreads)
        b < p_end; b += waves * kWave) {
     const int64_t p = b + lane;
     const bool held = p >= p_begin && p < p_end;
-    int64_t c = held ? static_cast<int64_t>(indices[p]) : -1;
-    if (c >= n_cols) c = -1;
+    // held to [0, n_cols) in 64 bits: the low half of a column below -2^31
+    // can be a valid one
+    const int64_t c64 = held ? static_cast<int64_t>(indices[p]) : -1;
+    const int c = c64 >= 0 && c64 < n_cols ? static_cast<int>(c64) : -1;
     const A a = held ? V::widen(data[p]) : A{};
     int64_t row = wave_row_of(indptr, n_rows, b, lane);
     row = lane_rows(indptr, n_rows, b, lane, row);
     for (int t = 0; t < kWave; t += per) {
-      const int cv = __shfl(static_cast<int>(c), t + sub, kWave);
+      const int cv = __shfl(c, t + sub, kWave);
       const int rv = __shfl(static_cast<int>(row), t + sub, kWave);
       const A av = shfl_lane(a, t + sub);
       if (cv < 0) continue;

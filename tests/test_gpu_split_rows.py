@@ -212,6 +212,29 @@ def test_transposed_products_by_positions(kind, vtype):
         np.testing.assert_array_equal(to_numpy(got), want)
 
 
+@pytest.mark.parametrize("vtype", ["float32", "bfloat16", "complex64"])
+def test_transposed_products_drop_columns_beyond_32_bits(vtype):
+    """64-bit columns out of range whose low 32 bits are a valid column add
+    nothing (small integers: every order of additions is exact)."""
+    rng = np.random.default_rng(67)
+    lengths = rng.integers(0, 12, 400)
+    n_rows, n_cols = len(lengths), 777
+    indices, indptr = _csr(rng, lengths, n_cols, np.int64)
+    small = lambda *shape: storage(rng.integers(-1, 2, shape).astype(np.float64), vtype)  # noqa: E731
+    data = small(indices.size)
+    bad = rng.random(indices.size) < 0.2
+    wide = indices + np.where(bad, rng.choice([-(1 << 31), -1, 1, 5], indices.size) << 32, 0)
+    held = np.where(bad, np.zeros_like(data), data)
+    d, i, p = to_torch(data, vtype, DEV), to_torch(wide, None, DEV), to_torch(indptr, None, DEV)
+    for k in (0, 1, 4, 33, 64, 70):
+        X = small(n_rows, k) if k else small(n_rows)
+        want = orc.csr_transpose_product(held, indices, indptr, X, n_rows, n_cols, vtype=vtype)
+        print(f"columns beyond 32 bits {vtype} k={k}", flush=True)
+        f = _capi.spmm_transpose if k else _capi.spmv_transpose
+        got = f(d, i, p, to_torch(X, vtype, DEV), n_rows, n_cols)
+        np.testing.assert_array_equal(to_numpy(got), want)
+
+
 @pytest.mark.parametrize("solver", ["cg", "pcg", "minres", "bicgstab"])
 @pytest.mark.parametrize("rows", [1, 2, 513, 1500, 2048, 2049, 4608])
 def test_small_systems_in_one_workgroup(solver, rows):
