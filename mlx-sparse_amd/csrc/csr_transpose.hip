@@ -444,30 +444,49 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-// A^T X: a wave takes 64 consecutive positions and finds their rows
-// (msx_rows.h), so a row of any length is shared by as many waves as its
-// values need; then its values in turn, L lanes (a power of two, at least k up
-// to 64) over the k columns of one value's output row, 64 / L values at a time.  One wave per row and one value at a time: 1 M values in
-// rows of 16, k = 4 116 -> 57 us; power-law rows, 100,007 of them, 1.2 M
-// values, k = 32 5,230 -> 112 us (the longest row's 12,500 values in
+// A^T X: a wave takes `span` consecutive positions (a power of two up to 64)
+// and finds their rows (msx_rows.h), so a row of any length is shared by as
+// many waves as its values need; then its values in turn, L lanes (a power of
+// two, at least k up to 64) over the k columns of one value's output row, 64 /
+// L values an instruction.  One wave per row and one value at a time: 1 M
+// values in rows of 16, k = 4 116 -> 57 us; power-law rows, 100,007 of them,
+// 1.2 M values, k = 32 5,230 -> 112 us (the longest row's 12,500 values in
 // sequence).  Sorting the values into a transpose for the call was slower
 // (150 us and 60 us a million values, then the gathers).
-template <class V, class I>
+// The span: a wave's steps, span * L / 64 of them, are a chain that small
+// matrices wait for, and a short span searches the rows for few values.  Eight
+// values for each of the 64 / L of a step, 16 at least and 64 at most: 2D
+// Laplacian 100^2, k = 128 a wave per row 26 us, 16 positions 27, 64 37; 3D
+// Poisson 46^3, k = 64 143, 146, 151; Laplacian 316^2, k = 2 16 positions 24,
+// 64 14.4.  complex64 steps add twice, half the span: Laplacian 100^2, k = 64 a
+// wave per row 43 us, 8 positions 46, 16 49, 64 56.
+inline int scatter_span(int L, size_t acc_bytes) {
+  const int steps = acc_bytes > 4 ? 4 : 8;
+  return std::min(kWave, std::max(2 * steps, steps * (kWave / L)));
+}
+// U: the steps whose X values are loaded before their atomics, eight with a
+// value a step (64 positions of the Laplacian above, k = 128: 54 us with one
+// load in flight, 49 with four, 37 with eight), else up to four.
+inline int scatter_ahead(int L, int span) {
+  return std::min(L == kWave ? 8 : 4, span * L / kWave);
+}
+
+template <class V, class I, int U>
 __global__ void __launch_bounds__(kThreads)
     scatter_spmm(const typename V::Storage *__restrict__ data, const I *__restrict__ indices,
                  const I *__restrict__ indptr, const typename V::Storage *__restrict__ X,
                  int64_t ldx, typename V::Acc *__restrict__ acc, int64_t lda, int64_t n_rows,
-                 int64_t nnz, int64_t n_cols, int64_t k, int L) {
+                 int64_t nnz, int64_t n_cols, int64_t k, int L, int span) {
   using A = typename V::Acc;
   const int lane = threadIdx.x % kWave;
   const int sub = lane / L, q0 = lane % L, per = kWave / L;
   const int64_t p_end = clamp64(static_cast<int64_t>(indptr[n_rows]), 0, nnz);
   const int64_t p_begin = clamp64(static_cast<int64_t>(indptr[0]), 0, p_end);
   const int64_t waves = static_cast<int64_t>(gridDim.x) * (kThreads / kWave);
-  for (int64_t b = (static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave) * kWave;
-       b < p_end; b += waves * kWave) {
+  for (int64_t b = (static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave) * span;
+       b < p_end; b += waves * span) {
     const int64_t p = b + lane;
-    const bool held = p >= p_begin && p < p_end;
+    const bool held = lane < span && p >= p_begin && p < p_end;
     // held to [0, n_cols) in 64 bits: the low half of a column below -2^31
     // can be a valid one
     const int64_t c64 = held ? static_cast<int64_t>(indices[p]) : -1;
@@ -475,14 +494,27 @@ __global__ void __launch_bounds__(kThreads)
     const A a = held ? V::widen(data[p]) : A{};
     int64_t row = wave_row_of(indptr, n_rows, b, lane);
     row = lane_rows(indptr, n_rows, b, lane, row);
-    for (int t = 0; t < kWave; t += per) {
-      const int cv = __shfl(c, t + sub, kWave);
-      const int rv = __shfl(static_cast<int>(row), t + sub, kWave);
-      const A av = shfl_lane(a, t + sub);
-      if (cv < 0) continue;
-      for (int64_t q = q0; q < k; q += L)
-        atomic_acc(acc + static_cast<int64_t>(cv) * lda + q,
-                   amul(av, V::widen(X[static_cast<int64_t>(rv) * ldx + q])));
+    for (int t = 0; t < span; t += per * U) {
+      int cv[U], rv[U];
+      A av[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int src = t + u * per + sub;
+        cv[u] = __shfl(c, src % kWave, kWave);
+        rv[u] = __shfl(static_cast<int>(row), src % kWave, kWave);
+        av[u] = shfl_lane(a, src % kWave);
+        if (src >= span) cv[u] = -1;
+      }
+      for (int64_t q = q0; q - q0 < k; q += L) {
+        const int64_t qx = q < k ? q : 0;
+        typename V::Storage xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) xv[u] = X[static_cast<int64_t>(rv[u]) * ldx + qx];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (cv[u] >= 0 && q < k)
+            atomic_acc(acc + static_cast<int64_t>(cv[u]) * lda + q, amul(av[u], V::widen(xv[u])));
+      }
     }
   }
 }
@@ -813,11 +845,22 @@ struct SpmmTransposeOp {
                        n_cols, k, lda);
     int L = 1;
     while (L < k && L < kWave) L <<= 1;
-    if (n_rows > 0)
-      hipLaunchKernelGGL((scatter_spmm<V, I>), dim3(grid_for(nnz)), dim3(kThreads), 0, stream,
-                         static_cast<const S *>(data), static_cast<const I *>(indices),
-                         static_cast<const I *>(indptr), static_cast<const S *>(X), ldx, acc, lda,
-                         n_rows, nnz, n_cols, k, L);
+    if (n_rows > 0 && k > 0) {
+      const int span = scatter_span(L, sizeof(A));
+      const int64_t waves = (nnz + span - 1) / span;
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid_for(waves * kWave)), dim3(kThreads), 0, stream,
+                           static_cast<const S *>(data), static_cast<const I *>(indices),
+                           static_cast<const I *>(indptr), static_cast<const S *>(X), ldx, acc, lda,
+                           n_rows, nnz, n_cols, k, L, span);
+      };
+      switch (scatter_ahead(L, span)) {
+      case 1: go(scatter_spmm<V, I, 1>); break;
+      case 2: go(scatter_spmm<V, I, 2>); break;
+      case 4: go(scatter_spmm<V, I, 4>); break;
+      default: go(scatter_spmm<V, I, 8>); break;
+      }
+    }
     if (!direct)
       hipLaunchKernelGGL((narrow_rows<V>), dim3(grid_for(n_cols * k)), dim3(kThreads), 0, stream,
                          acc, n_cols, k, lda, static_cast<S *>(Y), ldy);

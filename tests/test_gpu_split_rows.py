@@ -226,7 +226,7 @@ def test_transposed_products_drop_columns_beyond_32_bits(vtype):
     wide = indices + np.where(bad, rng.choice([-(1 << 31), -1, 1, 5], indices.size) << 32, 0)
     held = np.where(bad, np.zeros_like(data), data)
     d, i, p = to_torch(data, vtype, DEV), to_torch(wide, None, DEV), to_torch(indptr, None, DEV)
-    for k in (0, 1, 4, 33, 64, 70):
+    for k in (0, 1, 4, 12, 20, 33, 64, 70, 130):  # every run of positions a wave takes
         X = small(n_rows, k) if k else small(n_rows)
         want = orc.csr_transpose_product(held, indices, indptr, X, n_rows, n_cols, vtype=vtype)
         print(f"columns beyond 32 bits {vtype} k={k}", flush=True)
