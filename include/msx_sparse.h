@@ -80,12 +80,21 @@ typedef enum msx_slice_mode {
   MSX_SLICE_PANELS = 3 /* LDS column panels (two-pass SpMV) */
 } msx_slice_mode;
 
+/*
+ * msx_plan_options.flags: the plan holds no scratch for products and partial
+ * sums.  Each call that needs it is given it (msx_csr_spmv_ws,
+ * msx_csr_spmv_data_vjp_ws: msx_csr_plan_scratch bytes) or takes it from the
+ * stream-ordered allocator of its stream (the other entry points, the
+ * solvers), so calls that share the plan may run on several streams at once.
+ */
+#define MSX_PLAN_CALL_SCRATCH 1
+
 typedef struct msx_plan_options {
   int64_t block_nnz;  /* W: 0 = default (512 when rows average 20 or more
                          values and the values are not complex64, else 256),
                          else a power of two in [64, 1024] */
   int32_t slice_mode; /* msx_slice_mode */
-  int32_t reserved;   /* must be 0 */
+  int32_t flags;      /* 0 or MSX_PLAN_CALL_SCRATCH */
 } msx_plan_options;
 
 /* Summary of a plan, for callers that report or test it. */
@@ -136,7 +145,8 @@ msx_status msx_device_count(int *count);
  * W (0 = library default: 512 when nnz >= 20 * n_rows, else 256; otherwise
  * a power of two in [64, 1024]).
  * The plan holds scratch for long-row chunk sums: calls sharing one plan
- * must be ordered (one stream) - concurrent calls on a shared plan race.
+ * must be ordered (one stream) - concurrent calls on a shared plan race -
+ * unless it was built with MSX_PLAN_CALL_SCRATCH.
  *
  * Replaces the reference's per-launch kernel choice `nnz >= 32 * n_rows`
  * (reference: src/sparse/csr_matvec/csr_matvec.cpp:291-296), which has no
@@ -265,6 +275,19 @@ msx_status msx_csr_spmv(msx_vtype vt, msx_itype it, int64_t n_rows,
                         const void *indices, const void *indptr,
                         const void *x, void *y, const msx_csr_plan *plan,
                         void *stream);
+
+/*
+ * The same with the call's device scratch: at least msx_csr_plan_scratch
+ * bytes (0 for a plan that holds its own), 256-byte aligned, free for reuse
+ * once the call's work on `stream` is done.  NULL: from the stream-ordered
+ * allocator.
+ */
+size_t msx_csr_plan_scratch(const msx_csr_plan *plan);
+msx_status msx_csr_spmv_ws(msx_vtype vt, msx_itype it, int64_t n_rows,
+                           int64_t n_cols, int64_t nnz, const void *data,
+                           const void *indices, const void *indptr,
+                           const void *x, void *y, const msx_csr_plan *plan,
+                           void *scratch, size_t scratch_bytes, void *stream);
 
 /*
  * Y[i, c] = sum_p data[p] * X[indices[p], c] for c in [0, k), with X an
@@ -494,7 +517,7 @@ msx_status msx_csr_spmm_transpose_cpu(msx_vtype vt, msx_itype it,
  * are not compared: the gradient does not read them).  A bound panel plan
  * whose copy holds every value gathers x from LDS panels and uses the plan's
  * product buffer as scratch, so calls that overlap on one plan race, as SpMV
- * calls do.
+ * calls do; with MSX_PLAN_CALL_SCRATCH it lies in the call's scratch (_ws).
  *
  * Replace csr_matvec_data_vjp and csr_matmul_data_vjp (reference:
  * src/sparse/csr_matvec_data_vjp/csr_matvec_data_vjp.cpp,
@@ -505,6 +528,12 @@ msx_status msx_csr_spmv_data_vjp(msx_vtype vt, msx_itype it, int64_t n_rows,
                                  const void *indptr, const void *x,
                                  const void *cot, void *out,
                                  const msx_csr_plan *plan, void *stream);
+msx_status msx_csr_spmv_data_vjp_ws(msx_vtype vt, msx_itype it, int64_t n_rows,
+                                    int64_t n_cols, int64_t nnz,
+                                    const void *indices, const void *indptr,
+                                    const void *x, const void *cot, void *out,
+                                    const msx_csr_plan *plan, void *scratch,
+                                    size_t scratch_bytes, void *stream);
 msx_status msx_csr_spmm_data_vjp(msx_vtype vt, msx_itype it, int64_t n_rows,
                                  int64_t n_cols, int64_t nnz, const void *indices,
                                  const void *indptr, int64_t k, const void *X,

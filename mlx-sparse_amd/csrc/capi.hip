@@ -112,6 +112,15 @@ extern "C" msx_status msx_csr_spmv(msx_vtype vt, msx_itype it, int64_t n_rows, i
                                    int64_t nnz, const void *data, const void *indices,
                                    const void *indptr, const void *x, void *y,
                                    const msx_csr_plan *plan, void *stream) {
+  return msx_csr_spmv_ws(vt, it, n_rows, n_cols, nnz, data, indices, indptr, x, y, plan, nullptr, 0,
+                         stream);
+}
+
+extern "C" msx_status msx_csr_spmv_ws(msx_vtype vt, msx_itype it, int64_t n_rows, int64_t n_cols,
+                                      int64_t nnz, const void *data, const void *indices,
+                                      const void *indptr, const void *x, void *y,
+                                      const msx_csr_plan *plan, void *scratch,
+                                      size_t scratch_bytes, void *stream) {
   clear_error();
   msx_status st = check_common("csr_matvec", vt, it, n_rows, n_cols, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
@@ -120,7 +129,9 @@ extern "C" msx_status msx_csr_spmv(msx_vtype vt, msx_itype it, int64_t n_rows, i
   st = check_plan("csr_matvec", plan, vt, it, n_rows, n_cols, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
   if (n_rows == 0) return MSX_OK;
-  return launch_spmv(vt, it, n_rows, n_cols, nnz, data, indices, indptr, x, y, plan,
+  const PlanUse use(plan, scratch, scratch_bytes, static_cast<hipStream_t>(stream));
+  if (use.status() != MSX_OK) return use.status();
+  return launch_spmv(vt, it, n_rows, n_cols, nnz, data, indices, indptr, x, y, use.plan(),
                      static_cast<hipStream_t>(stream));
 }
 

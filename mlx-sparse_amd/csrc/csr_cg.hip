@@ -659,7 +659,9 @@ extern "C" msx_status msx_csr_cg(msx_itype it, int64_t n, int64_t nnz, const flo
   if (st != MSX_OK) return st;
   st = check_plan("csr_cg", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
-  const Solve s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
+  const PlanUse use(plan, nullptr, 0, static_cast<hipStream_t>(stream));
+  if (use.status() != MSX_OK) return use.status();
+  const Solve s{n, nnz, it, data, indices, indptr, use.plan(), static_cast<hipStream_t>(stream),
                 in_one_group(plan, n, nnz, kGroupMany) ? 1 : blocks_for(n),
                 in_one_group(plan, n, nnz, kGroupMany)};
   return solve(s, b, x0, nullptr, x, rtol, atol, maxiter, result);
@@ -678,7 +680,9 @@ extern "C" msx_status msx_csr_pcg_jacobi(msx_itype it, int64_t n, int64_t nnz, c
   if (inv_diag == nullptr) return fail(MSX_EINVAL, "csr_pcg_jacobi inverse diagonal is NULL.");
   st = check_plan("csr_pcg_jacobi", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
-  const Solve s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
+  const PlanUse use(plan, nullptr, 0, static_cast<hipStream_t>(stream));
+  if (use.status() != MSX_OK) return use.status();
+  const Solve s{n, nnz, it, data, indices, indptr, use.plan(), static_cast<hipStream_t>(stream),
                 in_one_group(plan, n, nnz, kGroupMany) ? 1 : blocks_for(n),
                 in_one_group(plan, n, nnz, kGroupMany)};
   return solve(s, b, x0, inv_diag, x, rtol, atol, maxiter, result);

@@ -554,7 +554,9 @@ extern "C" msx_status msx_csr_gmres(msx_itype it, int64_t n, int64_t nnz, const 
   const msx_status st = check_plan("csr_gmres", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
   const uint32_t blocks = blocks_for(n);
-  const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
+  const PlanUse use(plan, nullptr, 0, static_cast<hipStream_t>(stream));
+  if (use.status() != MSX_OK) return use.status();
+  const System s{n, nnz, it, data, indices, indptr, use.plan(), static_cast<hipStream_t>(stream),
                  dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks)};
   return gmres<false>(s, b, x0, nullptr, x, rtol, atol, restart, maxiter, result);
 }
@@ -582,7 +584,9 @@ extern "C" msx_status msx_csr_gmres_jacobi(msx_itype it, int64_t n, int64_t nnz,
       check_plan("csr_gmres_jacobi", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
   const uint32_t blocks = blocks_for(n);
-  const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
+  const PlanUse use(plan, nullptr, 0, static_cast<hipStream_t>(stream));
+  if (use.status() != MSX_OK) return use.status();
+  const System s{n, nnz, it, data, indices, indptr, use.plan(), static_cast<hipStream_t>(stream),
                  dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks)};
   return gmres<true>(s, b, x0, inv_diag, x, rtol, atol, restart, maxiter, result);
 }

@@ -1251,7 +1251,9 @@ extern "C" msx_status msx_csr_bicgstab(msx_itype it, int64_t n, int64_t nnz, con
   st = check_plan("csr_bicgstab", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
   const uint32_t blocks = blocks_for(n);
-  const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
+  const PlanUse use(plan, nullptr, 0, static_cast<hipStream_t>(stream));
+  if (use.status() != MSX_OK) return use.status();
+  const System s{n, nnz, it, data, indices, indptr, use.plan(), static_cast<hipStream_t>(stream),
                  dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks),
                  bi_in_one_group(plan, n, nnz)};
   return bicgstab<false>(s, b, x0, nullptr, x, rtol, atol, maxiter, result);
@@ -1273,7 +1275,9 @@ extern "C" msx_status msx_csr_bicgstab_jacobi(msx_itype it, int64_t n, int64_t n
   st = check_plan("csr_bicgstab_jacobi", plan, MSX_F32, it, n, n, nnz, data, indices, indptr);
   if (st != MSX_OK) return st;
   const uint32_t blocks = blocks_for(n);
-  const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
+  const PlanUse use(plan, nullptr, 0, static_cast<hipStream_t>(stream));
+  if (use.status() != MSX_OK) return use.status();
+  const System s{n, nnz, it, data, indices, indptr, use.plan(), static_cast<hipStream_t>(stream),
                  dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks),
                  bi_in_one_group(plan, n, nnz)};
   return bicgstab<true>(s, b, x0, inv_diag, x, rtol, atol, maxiter, result);
@@ -1291,7 +1295,9 @@ extern "C" msx_status msx_csr_minres(msx_itype it, int64_t n, int64_t nnz, const
   if (st != MSX_OK) return st;
   const bool group = in_one_group(plan, n, nnz, kGroupFew);
   const uint32_t blocks = group ? 1 : blocks_for(n);
-  const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
+  const PlanUse use(plan, nullptr, 0, static_cast<hipStream_t>(stream));
+  if (use.status() != MSX_OK) return use.status();
+  const System s{n, nnz, it, data, indices, indptr, use.plan(), static_cast<hipStream_t>(stream),
                  dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks),
                  group};
   return minres<false>(s, b, x0, nullptr, x, rtol, atol, maxiter, shift, result);
@@ -1313,7 +1319,9 @@ extern "C" msx_status msx_csr_minres_jacobi(msx_itype it, int64_t n, int64_t nnz
   if (st != MSX_OK) return st;
   const bool group = in_one_group(plan, n, nnz, kGroupFew);
   const uint32_t blocks = group ? 1 : blocks_for(n);
-  const System s{n, nnz, it, data, indices, indptr, plan, static_cast<hipStream_t>(stream),
+  const PlanUse use(plan, nullptr, 0, static_cast<hipStream_t>(stream));
+  if (use.status() != MSX_OK) return use.status();
+  const System s{n, nnz, it, data, indices, indptr, use.plan(), static_cast<hipStream_t>(stream),
                  dim3(blocks), dim3(kSolverThreads), static_cast<int>(blocks),
                  group};
   return minres<true>(s, b, x0, inv_diag, x, rtol, atol, maxiter, shift, result);

@@ -638,7 +638,7 @@ msx_status build_layout(msx_csr_plan *p, const typename V::Storage *data, const 
   // The copy and its product buffer.
   const size_t b_data = round256(sizeof(S) * std::max<int64_t>(n_values, 1));
   const size_t b_u16 = round256(sizeof(uint16_t) * std::max<int64_t>(n_values, 1));
-  const size_t b_prod = round256(sizeof(A) * std::max<int64_t>(n_values, 1));
+  const size_t b_prod = p->call_scratch ? 0 : round256(sizeof(A) * std::max<int64_t>(n_values, 1));
   char *base = nullptr;
   if (hipMalloc(&base, b_data + 2 * b_u16 + b_prod) != hipSuccess) {
     (void)hipGetLastError();
@@ -649,7 +649,7 @@ msx_status build_layout(msx_csr_plan *p, const typename V::Storage *data, const 
   p->pn_data = base;
   p->pn_col = reinterpret_cast<uint16_t *>(base + b_data);
   p->pn_dest = reinterpret_cast<uint16_t *>(base + b_data + b_u16);
-  p->pn_prod = base + b_data + 2 * b_u16;
+  p->pn_prod = p->call_scratch ? nullptr : base + b_data + 2 * b_u16;
   // Padding entries: value 0, column 0, word 0xFFFF.
   MSX_HIP_TRY(hipMemsetAsync(p->pn_data, 0, b_data, stream));
   MSX_HIP_TRY(hipMemsetAsync(p->pn_col, 0, b_u16, stream));

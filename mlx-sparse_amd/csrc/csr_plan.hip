@@ -267,7 +267,64 @@ msx_status build_plan(msx_csr_plan *p, const I *indptr, hipStream_t stream) {
   return MSX_OK;
 }
 
+// Device bytes of a plan's scratch arrays, each on a 256-byte boundary.
+struct ScratchSizes {
+  size_t prod, vpart, spart, chunk, ls;
+  size_t total() const { return prod + vpart + spart + chunk + ls; }
+};
+
+ScratchSizes scratch_sizes(const msx_csr_plan *p) {
+  const size_t a = p->vtype == MSX_C64 ? 8 : 4;
+  const auto bytes = [](int64_t n, size_t each) { return align_up(static_cast<size_t>(n) * each, 256); };
+  ScratchSizes z{};
+  if (p->n_panels > 0) z.prod = bytes(p->pn_values, a);
+  if (p->pn_vstart != nullptr) z.vpart = bytes(p->pn_vrows, a);
+  if (p->n_slices > 0) z.spart = bytes(int64_t{kSlices} * p->n_rows, a);
+  if (p->pn_vstart == nullptr) z.chunk = bytes(p->n_chunks > p->n_long ? p->n_chunks : 0, 8);
+  z.ls = bytes(p->ls_units, a);
+  return z;
+}
+
 }  // namespace
+
+PlanUse::PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStream_t stream)
+    : plan_(plan), stream_(stream) {
+  if (plan == nullptr || !plan->call_scratch) return;
+  const ScratchSizes z = scratch_sizes(plan);
+  if (z.total() == 0) return;
+  if (scratch == nullptr) {
+    const hipError_t e = hipMallocAsync(&owned_, z.total(), stream);
+    if (e != hipSuccess) {
+      owned_ = nullptr;
+      (void)hipGetLastError();
+      status_ = fail(MSX_ENOMEM, "device allocation of a plan's call scratch failed.");
+      return;
+    }
+    scratch = owned_;
+  } else if (bytes < z.total() || (reinterpret_cast<uintptr_t>(scratch) & 255u) != 0) {
+    status_ = fail(MSX_EINVAL, "plan scratch must be 256-byte aligned and hold "
+                               "msx_csr_plan_scratch bytes.");
+    return;
+  }
+  mine_ = *plan;
+  char *at = static_cast<char *>(scratch);
+  const auto take = [&](size_t b) {
+    void *here = at;
+    at += b;
+    return here;
+  };
+  mine_.pn_prod = take(z.prod);
+  mine_.pn_partial = take(z.vpart);
+  mine_.s_partial = take(z.spart);
+  mine_.partials = take(z.chunk);
+  mine_.ls_partial = take(z.ls);
+  plan_ = &mine_;
+}
+
+PlanUse::~PlanUse() {
+  if (owned_ != nullptr) (void)hipFreeAsync(owned_, stream_);
+}
+
 }  // namespace msx
 
 using namespace msx;
@@ -350,7 +407,8 @@ extern "C" msx_status msx_csr_plan_create_bound(msx_vtype vt, msx_itype it, int6
     return fail(MSX_EINVAL, "msx_csr_plan_create_bound: data and indices must be non-NULL.");
   const msx_plan_options defaults{0, MSX_SLICE_AUTO, 0};
   if (opts == nullptr) opts = &defaults;
-  if (opts->slice_mode < MSX_SLICE_AUTO || opts->slice_mode > MSX_SLICE_PANELS || opts->reserved != 0)
+  if (opts->slice_mode < MSX_SLICE_AUTO || opts->slice_mode > MSX_SLICE_PANELS ||
+      (opts->flags & ~MSX_PLAN_CALL_SCRATCH) != 0)
     return fail(MSX_EINVAL, "msx_csr_plan_create_bound: invalid options.");
   // complex64 keeps the narrow default: a 512-value block holds twice the
   // registers for its 8-byte values, which halves occupancy (banded matrix,
@@ -363,6 +421,7 @@ extern "C" msx_status msx_csr_plan_create_bound(msx_vtype vt, msx_itype it, int6
   p->n_cols = n_cols;
   p->slice_mode = opts->slice_mode;
   p->bound = true;
+  p->call_scratch = (opts->flags & MSX_PLAN_CALL_SCRATCH) != 0;
   p->bound_data = data;
   p->bound_indices = indices;
   auto s = static_cast<hipStream_t>(stream);
@@ -429,6 +488,10 @@ extern "C" msx_status msx_csr_plan_refresh(msx_csr_plan *plan, const void *data,
   if (st == MSX_OK && plan->n_panels > 0) st = refresh_panels(plan, data, s);
   if (st == MSX_OK) plan->bound_data = data;
   return st;
+}
+
+extern "C" size_t msx_csr_plan_scratch(const msx_csr_plan *plan) {
+  return plan != nullptr && plan->call_scratch ? scratch_sizes(plan).total() : 0;
 }
 
 extern "C" msx_status msx_csr_plan_destroy(msx_csr_plan *plan) {

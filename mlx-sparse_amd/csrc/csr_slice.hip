@@ -437,7 +437,7 @@ msx_status build_typed(msx_csr_plan *p, const void *data, const void *indices, c
   const size_t b_data = ((static_cast<size_t>(p->nnz) * sizeof(S) + 255) / 256) * 256;
   const size_t b_col = ((static_cast<size_t>(p->nnz) * 4 + 255) / 256) * 256;
   const size_t b_seg = ((static_cast<size_t>(n_super) * (kSlices + 1) * 4 + 255) / 256) * 256;
-  const size_t b_part = static_cast<size_t>(kSlices) * p->n_rows * sizeof(A);
+  const size_t b_part = p->call_scratch ? 0 : static_cast<size_t>(kSlices) * p->n_rows * sizeof(A);
   char *base = nullptr;
   if (hipMalloc(&base, b_data + b_col + b_seg + b_part) != hipSuccess) {
     (void)hipGetLastError();
@@ -447,7 +447,7 @@ msx_status build_typed(msx_csr_plan *p, const void *data, const void *indices, c
   p->s_data = base;
   p->s_col = reinterpret_cast<uint32_t *>(base + b_data);
   p->s_seg = reinterpret_cast<uint32_t *>(base + b_data + b_col);
-  p->s_partial = base + b_data + b_col + b_seg;
+  p->s_partial = p->call_scratch ? nullptr : base + b_data + b_col + b_seg;
   p->s_bytes = b_data + b_col + b_seg + b_part;
   p->slice_width = width;
   p->col_bits = col_bits;

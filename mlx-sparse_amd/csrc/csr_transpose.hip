@@ -1534,6 +1534,15 @@ extern "C" msx_status msx_csr_spmv_data_vjp(msx_vtype vt, msx_itype it, int64_t 
                                             int64_t n_cols, int64_t nnz, const void *indices,
                                             const void *indptr, const void *x, const void *cot,
                                             void *out, const msx_csr_plan *plan, void *stream) {
+  return msx_csr_spmv_data_vjp_ws(vt, it, n_rows, n_cols, nnz, indices, indptr, x, cot, out, plan,
+                                  nullptr, 0, stream);
+}
+
+extern "C" msx_status msx_csr_spmv_data_vjp_ws(msx_vtype vt, msx_itype it, int64_t n_rows,
+                                               int64_t n_cols, int64_t nnz, const void *indices,
+                                               const void *indptr, const void *x, const void *cot,
+                                               void *out, const msx_csr_plan *plan, void *scratch,
+                                               size_t scratch_bytes, void *stream) {
   clear_error();
   msx_status st = check_csr("csr_matvec_data_vjp", vt, it, n_rows, n_cols, nnz, indices, indptr);
   if (st != MSX_OK) return st;
@@ -1547,8 +1556,11 @@ extern "C" msx_status msx_csr_spmv_data_vjp(msx_vtype vt, msx_itype it, int64_t 
   if (nnz == 0 || n_rows == 0) return MSX_OK;
   // A panel plan turns the gather of x into LDS reads (two streaming passes)
   // when its copy holds every value (no invalid column was dropped).
-  if (plan != nullptr && plan->bound && plan->vtype == vt && panel_data_vjp_fits(plan))
-    return launch_panel_data_vjp(plan, indptr, x, cot, out, static_cast<hipStream_t>(stream));
+  if (plan != nullptr && plan->bound && plan->vtype == vt && panel_data_vjp_fits(plan)) {
+    const PlanUse use(plan, scratch, scratch_bytes, static_cast<hipStream_t>(stream));
+    if (use.status() != MSX_OK) return use.status();
+    return launch_panel_data_vjp(use.plan(), indptr, x, cot, out, static_cast<hipStream_t>(stream));
+  }
   return dispatch<SpmvDataVjpOp>(vt, it, n_rows, n_cols, nnz, indices, indptr, x, cot, out,
                                  plan != nullptr && plan->n_long > 0,
                                  static_cast<hipStream_t>(stream));

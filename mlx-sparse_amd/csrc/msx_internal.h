@@ -75,6 +75,7 @@ struct msx_csr_plan {
   int col_bits;
   const void *indptr;         // the row pointers the plan was built from
   bool bound;                 // built by msx_csr_plan_create_bound
+  bool call_scratch;          // MSX_PLAN_CALL_SCRATCH: pn_prod and s_partial are null
   const void *bound_data;     // the buffers a bound plan was built from (data: as last refreshed)
   const void *bound_indices;
   void *s_data;               // values reordered by slice inside each short block
@@ -157,6 +158,27 @@ namespace msx {
 msx_status check_plan(const char *op, const msx_csr_plan *plan, msx_vtype vt, msx_itype it,
                       int64_t n_rows, int64_t n_cols, int64_t nnz, const void *data,
                       const void *indices, const void *indptr);
+
+// A plan as one call's launches use it: with MSX_PLAN_CALL_SCRATCH a copy whose
+// products and partial sums lie in the call's own scratch - the caller's, else
+// memory of `stream`'s allocator, given back when the object ends - so that
+// calls on several streams share only what they read.
+class PlanUse {
+ public:
+  PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStream_t stream);
+  ~PlanUse();
+  PlanUse(const PlanUse &) = delete;
+  PlanUse &operator=(const PlanUse &) = delete;
+  msx_status status() const { return status_; }
+  const msx_csr_plan *plan() const { return plan_; }
+
+ private:
+  const msx_csr_plan *plan_;
+  msx_csr_plan mine_;
+  void *owned_ = nullptr;
+  hipStream_t stream_;
+  msx_status status_ = MSX_OK;
+};
 
 // Launchers (csr_spmv.hip / csr_spmm.hip).  Arguments are already checked.
 msx_status launch_spmv(msx_vtype vt, msx_itype it, int64_t n_rows, int64_t n_cols, int64_t nnz,

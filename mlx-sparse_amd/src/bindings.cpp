@@ -194,7 +194,8 @@ std::shared_ptr<Plan> make_plan(py::handle indptr_obj, int64_t n_rows, int64_t n
     msx::require_contiguous(vd, "csr_plan data");
     msx::require_contiguous(vi, "csr_plan indices");
     plan->bound = py::make_tuple(data_obj, indices_obj, indptr);
-    msx_plan_options opts{block_nnz, slice_mode, 0};
+    // A plan is cached with its matrix and used from every stream and thread.
+    msx_plan_options opts{block_nnz, slice_mode, MSX_PLAN_CALL_SCRATCH};
     py::gil_scoped_release nogil;
     st = msx_csr_plan_create_bound(msx::to_vtype(vd.dtype), msx::to_itype(v.dtype), n_rows, n_cols,
                                    nnz, vd.ptr, vi.ptr, v.ptr, &opts, stream, &plan->p);
@@ -289,6 +290,7 @@ py::object csr_matvec(py::handle data_o, py::handle indices_o, py::handle indptr
   ctx.stream = vd.device >= 0 ? stream_for(vd.device) : nullptr;
   const msx_csr_plan *p = plan_ptr(plan);
   if (vd.device >= 0) {
+    const at::Tensor scratch = scratch_for(ctx, data, msx_csr_plan_scratch(p));
     msx::csr_matvec(vd, vi, vp, vx, vo, n_rows, n_cols, p, ctx);
   } else {
     py::gil_scoped_release nogil;
@@ -560,9 +562,11 @@ py::object csr_matvec_data_vjp(py::handle indices_o, py::handle indptr_o, py::ha
   if (vi.ndim != 1) msx::require_rank(vi, 1, "csr_matvec_data_vjp indices");
   py::object out = empty_like_out(vx, x, py::make_tuple(vi.shape[0]));
   const ArrayView vo = view_of(out);
-  const msx::ExecContext ctx = context_for(vx, n_threads);
+  msx::ExecContext ctx = context_for(vx, n_threads);
   if (vx.device >= 0) {
-    msx::csr_matvec_data_vjp(vi, vp, vx, vc, vo, n_rows, n_cols, ctx, plan_ptr(plan));
+    const msx_csr_plan *p = plan_ptr(plan);
+    const at::Tensor scratch = scratch_for(ctx, x, msx_csr_plan_scratch(p));
+    msx::csr_matvec_data_vjp(vi, vp, vx, vc, vo, n_rows, n_cols, ctx, p);
   } else {
     py::gil_scoped_release nogil;
     msx::csr_matvec_data_vjp(vi, vp, vx, vc, vo, n_rows, n_cols, ctx);

@@ -152,9 +152,9 @@ void csr_matvec_data_vjp(const ArrayView &indices, const ArrayView &indptr, cons
   const msx_vtype vt = to_vtype(x.dtype);
   const msx_itype it = to_itype(indices.dtype);
   if (x.device >= 0)
-    check_status(msx_csr_spmv_data_vjp(vt, it, n_rows, n_cols, indices.size(), indices.ptr,
-                                       indptr.ptr, x.ptr, cotangent.ptr, out.ptr, plan,
-                                       ctx.stream),
+    check_status(msx_csr_spmv_data_vjp_ws(vt, it, n_rows, n_cols, indices.size(), indices.ptr,
+                                          indptr.ptr, x.ptr, cotangent.ptr, out.ptr, plan,
+                                          ctx.scratch, ctx.scratch_bytes, ctx.stream),
                  op);
   else
     check_status(msx_csr_spmv_data_vjp_cpu(vt, it, n_rows, n_cols, indices.size(), indices.ptr,

@@ -37,8 +37,8 @@ void csr_matvec(const ArrayView &data, const ArrayView &indices, const ArrayView
   const msx_itype it = to_itype(indices.dtype);
   const int64_t nnz = data.size();
   if (data.device >= 0) {
-    check_status(msx_csr_spmv(vt, it, n_rows, n_cols, nnz, data.ptr, indices.ptr, indptr.ptr,
-                              x.ptr, out.ptr, plan, ctx.stream),
+    check_status(msx_csr_spmv_ws(vt, it, n_rows, n_cols, nnz, data.ptr, indices.ptr, indptr.ptr,
+                                 x.ptr, out.ptr, plan, ctx.scratch, ctx.scratch_bytes, ctx.stream),
                  "csr_matvec");
   } else {
     check_status(msx_csr_spmv_cpu(vt, it, n_rows, n_cols, nnz, data.ptr, indices.ptr, indptr.ptr,
