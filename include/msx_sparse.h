@@ -205,8 +205,9 @@ msx_status msx_csr_plan_create_bound(msx_vtype vt, msx_itype it,
  * `stream`, asynchronously, and bind the plan to `data` from now on.  A
  * gather through the layout the plan already holds: O(nnz), no allocation
  * and no re-sort (the headline matrix: one pass over its values instead of
- * the 20 ms build).  Row-block plans hold no values: a no-op.  Calls that
- * share the plan must be ordered after this one (same stream).
+ * the 20 ms build).  Row-block plans hold no values: a no-op.  Products,
+ * gradients and solves that are called afterwards on another stream wait for
+ * it (not inside a capture: order those yourself).
  *
  * No reference counterpart: the reference's arrays are immutable
  * (reference: mlx_sparse/_csr.py:33), so its kernels always read the

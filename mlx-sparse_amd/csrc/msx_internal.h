@@ -78,6 +78,10 @@ struct msx_csr_plan {
   bool call_scratch;          // MSX_PLAN_CALL_SCRATCH: pn_prod and s_partial are null
   const void *bound_data;     // the buffers a bound plan was built from (data: as last refreshed)
   const void *bound_indices;
+  // The last refresh of the value copies outside a capture: calls on other
+  // streams than its own wait for it.
+  hipEvent_t refreshed;       // null before the first
+  hipStream_t refreshed_on;
   void *s_data;               // values reordered by slice inside each short block
   uint32_t *s_col;            // (row_in_block << col_bits) | column_in_slice
   uint32_t *s_seg;            // per 256-row super-block: kSlices + 1 offsets from its first value
@@ -159,7 +163,8 @@ msx_status check_plan(const char *op, const msx_csr_plan *plan, msx_vtype vt, ms
                       int64_t n_rows, int64_t n_cols, int64_t nnz, const void *data,
                       const void *indices, const void *indptr);
 
-// A plan as one call's launches use it: with MSX_PLAN_CALL_SCRATCH a copy whose
+// A plan as one call's launches on `stream` use it, ordered after the plan's
+// last refresh on another stream; with MSX_PLAN_CALL_SCRATCH a copy whose
 // products and partial sums lie in the call's own scratch - the caller's, else
 // memory of `stream`'s allocator, given back when the object ends - so that
 // calls on several streams share only what they read.

@@ -69,6 +69,35 @@ def test_products_and_value_gradients_on_two_streams(mode, long_rows):
         assert all(torch.equal(d, want_g[i]) for d in grads[i])
 
 
+@pytest.mark.parametrize("mode", ["panels", "on", "off"])
+def test_new_values_reach_a_product_on_another_stream(mode):
+    """The values change on one stream; a product on another that waits for
+    that change, and no more, uses them also where the copy that the plan
+    holds is rewritten later, in the first stream's own time."""
+    rng = np.random.default_rng(79)
+    a = _matrix(rng, rng.integers(2, 12, 40_000), 30_000)
+    with runtime.context("gpu_slice", mode):
+        a.plan()
+    x = torch.from_numpy(rng.integers(-2, 3, 30_000).astype(np.float32)).to(DEV)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    old = a @ x
+    torch.cuda.synchronize()
+    print(f"new values {mode}", flush=True)
+    for _ in range(3):
+        old = 2 * old
+        changed = torch.cuda.Event()
+        with torch.cuda.stream(first):
+            a.data.mul_(2)
+            changed.record()
+            torch.cuda._sleep(20_000_000)  # about 10 ms before the copy is rewritten
+            y1 = a @ x
+        with torch.cuda.stream(second):
+            second.wait_event(changed)
+            y2 = a @ x
+        torch.cuda.synchronize()
+        assert torch.equal(y1, old) and torch.equal(y2, old)
+
+
 def test_solves_in_two_threads():
     rng = np.random.default_rng(73)
     n, per = 60_000, 6
