@@ -88,13 +88,20 @@ typedef enum msx_slice_mode {
  * solvers), so calls that share the plan may run on several streams at once.
  */
 #define MSX_PLAN_CALL_SCRATCH 1
+/*
+ * With MSX_SLICE_AUTO: keep row blocks where panels are worth their build only
+ * over some tens of products (x below 8 MB or fewer than 16 Mi values).
+ * msx_csr_plan_deferred is then 1; a plan built again without the flag holds
+ * the panels.
+ */
+#define MSX_PLAN_DEFER 2
 
 typedef struct msx_plan_options {
   int64_t block_nnz;  /* W: 0 = default (512 when rows average 20 or more
                          values and the values are not complex64, else 256),
                          else a power of two in [64, 1024] */
   int32_t slice_mode; /* msx_slice_mode */
-  int32_t flags;      /* 0 or MSX_PLAN_CALL_SCRATCH */
+  int32_t flags;      /* MSX_PLAN_CALL_SCRATCH, MSX_PLAN_DEFER */
 } msx_plan_options;
 
 /* Summary of a plan, for callers that report or test it. */
@@ -219,6 +226,9 @@ msx_status msx_csr_plan_refresh(msx_csr_plan *plan, const void *data,
 
 /* Release a plan (NULL is accepted).  Synchronises the plan's device. */
 msx_status msx_csr_plan_destroy(msx_csr_plan *plan);
+
+/* 1 when MSX_PLAN_DEFER kept panels from a plan, else 0. */
+int msx_csr_plan_deferred(const msx_csr_plan *plan);
 
 /* Fill `info` from a plan. */
 msx_status msx_csr_plan_info(const msx_csr_plan *plan, msx_plan_info *info);

@@ -296,7 +296,18 @@ bool capturing(hipStream_t stream) {
   return true;
 }
 
+// The capture that `stream` takes part in, 0: none.
+unsigned long long capture_of(hipStream_t stream) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(stream, &s, &id) == hipSuccess && s == hipStreamCaptureStatusActive)
+    return id;
+  (void)hipGetLastError();
+  return 0;
+}
+
 msx_status mark_refreshed(msx_csr_plan *p, hipStream_t stream) {
+  p->refreshed_in = capture_of(stream);
   if (capturing(stream)) return MSX_OK;
   if (p->refreshed == nullptr)
     MSX_HIP_TRY(hipEventCreateWithFlags(&p->refreshed, hipEventDisableTiming | hipEventDisableSystemFence));
@@ -307,18 +318,26 @@ msx_status mark_refreshed(msx_csr_plan *p, hipStream_t stream) {
 
 }  // namespace
 
-PlanUse::PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStream_t stream)
+PlanUse::PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStream_t stream,
+                 bool values)
     : plan_(plan), stream_(stream) {
   if (plan == nullptr) return;
-  if (plan->refreshed != nullptr && plan->refreshed_on != stream && !capturing(stream)) {
+  if (values && plan->refreshed != nullptr && plan->refreshed_on != stream && !capturing(stream)) {
     const hipError_t e = hipStreamWaitEvent(stream, plan->refreshed, 0);
     if (e != hipSuccess) {
       status_ = hip_fail(e, "waiting for a plan's refresh");
       return;
     }
   }
+  if (values && plan->late && capturing(stream) &&
+      (plan->refreshed_in == 0 || plan->refreshed_in != capture_of(stream))) {
+    mine_ = *plan;
+    mine_.n_panels = 0;
+    mine_.pn_vstart = nullptr;
+    plan_ = &mine_;
+  }
   if (!plan->call_scratch) return;
-  const ScratchSizes z = scratch_sizes(plan);
+  const ScratchSizes z = scratch_sizes(plan_);
   if (z.total() == 0) return;
   if (scratch == nullptr) {
     const hipError_t e = hipMallocAsync(&owned_, z.total(), stream);
@@ -334,7 +353,7 @@ PlanUse::PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStrea
                                "msx_csr_plan_scratch bytes.");
     return;
   }
-  mine_ = *plan;
+  if (plan_ != &mine_) mine_ = *plan;
   char *at = static_cast<char *>(scratch);
   const auto take = [&](size_t b) {
     void *here = at;
@@ -437,7 +456,7 @@ extern "C" msx_status msx_csr_plan_create_bound(msx_vtype vt, msx_itype it, int6
   const msx_plan_options defaults{0, MSX_SLICE_AUTO, 0};
   if (opts == nullptr) opts = &defaults;
   if (opts->slice_mode < MSX_SLICE_AUTO || opts->slice_mode > MSX_SLICE_PANELS ||
-      (opts->flags & ~MSX_PLAN_CALL_SCRATCH) != 0)
+      (opts->flags & ~(MSX_PLAN_CALL_SCRATCH | MSX_PLAN_DEFER)) != 0)
     return fail(MSX_EINVAL, "msx_csr_plan_create_bound: invalid options.");
   // complex64 keeps the narrow default: a 512-value block holds twice the
   // registers for its 8-byte values, which halves occupancy (banded matrix,
@@ -470,6 +489,11 @@ extern "C" msx_status msx_csr_plan_create_bound(msx_vtype vt, msx_itype it, int6
     const bool slices = x_bytes >= kSliceMinX;
     if (panels || slices) st = probe_scattered(p, indices, s, &scattered, &short_values);
     if (scattered) mode = panels ? MSX_SLICE_PANELS : MSX_SLICE_ON;
+    if (mode == MSX_SLICE_PANELS && !panels_at_once(p)) {
+      p->deferred = (opts->flags & MSX_PLAN_DEFER) != 0;
+      p->late = !p->deferred;
+      if (p->deferred) mode = MSX_SLICE_OFF;
+    }
   }
   if (st == MSX_OK && mode == MSX_SLICE_PANELS && p->n_blocks > 0) {
     if (!panels_eligible(p))
@@ -518,6 +542,10 @@ extern "C" msx_status msx_csr_plan_refresh(msx_csr_plan *plan, const void *data,
   if (st == MSX_OK && (plan->n_slices > 0 || plan->n_panels > 0)) st = mark_refreshed(plan, s);
   if (st == MSX_OK) plan->bound_data = data;
   return st;
+}
+
+extern "C" int msx_csr_plan_deferred(const msx_csr_plan *plan) {
+  return plan != nullptr && plan->deferred ? 1 : 0;
 }
 
 extern "C" size_t msx_csr_plan_scratch(const msx_csr_plan *plan) {

@@ -1557,7 +1557,7 @@ extern "C" msx_status msx_csr_spmv_data_vjp_ws(msx_vtype vt, msx_itype it, int64
   // A panel plan turns the gather of x into LDS reads (two streaming passes)
   // when its copy holds every value (no invalid column was dropped).
   if (plan != nullptr && plan->bound && plan->vtype == vt && panel_data_vjp_fits(plan)) {
-    const PlanUse use(plan, scratch, scratch_bytes, static_cast<hipStream_t>(stream));
+    const PlanUse use(plan, scratch, scratch_bytes, static_cast<hipStream_t>(stream), false);
     if (use.status() != MSX_OK) return use.status();
     return launch_panel_data_vjp(use.plan(), indptr, x, cot, out, static_cast<hipStream_t>(stream));
   }

@@ -82,6 +82,14 @@ struct msx_csr_plan {
   // streams than its own wait for it.
   hipEvent_t refreshed;       // null before the first
   hipStream_t refreshed_on;
+  unsigned long long refreshed_in;  // the capture that holds a refresh, 0: none
+  // Panels that AUTO takes below the sizes where it always does
+  // (panels_at_once): `deferred`, row blocks until the caller asks again
+  // without MSX_PLAN_DEFER; `late`, they are there.  A captured product leaves
+  // late panels alone unless their refresh is captured with it: its replays
+  // read the values as they are then, as row blocks do.
+  bool deferred;
+  bool late;
   void *s_data;               // values reordered by slice inside each short block
   uint32_t *s_col;            // (row_in_block << col_bits) | column_in_slice
   uint32_t *s_seg;            // per 256-row super-block: kSlices + 1 offsets from its first value
@@ -170,7 +178,9 @@ msx_status check_plan(const char *op, const msx_csr_plan *plan, msx_vtype vt, ms
 // calls on several streams share only what they read.
 class PlanUse {
  public:
-  PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStream_t stream);
+  // values: the call reads the matrix's values.
+  PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStream_t stream,
+          bool values = true);
   ~PlanUse();
   PlanUse(const PlanUse &) = delete;
   PlanUse &operator=(const PlanUse &) = delete;
@@ -224,6 +234,15 @@ constexpr int64_t kSliceMinX = int64_t{16} << 20;
 constexpr int64_t kPanelAnyValues = int64_t{16} << 20;
 // True when those sizes favour panels (csr_panel_build.hip).
 bool panels_pay(const msx_csr_plan *p);
+// From these sizes on the first product is worth the copy to every caller; below, it is
+// repaid after many (build beyond the row blocks' 0.2 ms, gain a product, us:
+// 1.3 M rows of 16 1,900 and 60, 1.5 M power-law rows 1,500 and 28, 350,000
+// rows of 16 over 4.4 MB of x 1,050 and 8), so a plan can be asked to wait.
+constexpr int64_t kAtOnceMinX = int64_t{8} << 20;
+constexpr int64_t kAtOnceValues = int64_t{16} << 20;
+inline bool panels_at_once(const msx_csr_plan *p) {
+  return p->nnz >= kAtOnceValues && p->n_cols * static_cast<int64_t>(value_bytes(p->vtype)) >= kAtOnceMinX;
+}
 
 // Panel plans (csr_panel_build.hip / csr_panel.hip).
 bool panels_eligible(const msx_csr_plan *p);

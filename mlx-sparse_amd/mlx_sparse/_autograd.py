@@ -58,14 +58,14 @@ def _adjoint_csr(a, data: torch.Tensor):
     return a._transpose_on(device, conjugate=a.data.is_complex())
 
 
-def _own_plan(a, data: torch.Tensor):
+def _own_plan(a, data: torch.Tensor, products: int):
     """``a``'s plan when ``data`` is the very buffer the plan is bound to
     (``a``'s values, contiguous on their device), else None: values
     elsewhere run plan-free."""
     bufs = a.buffers(data.device)
     if data.data_ptr() != bufs[0].data_ptr() or not data.is_contiguous():
         return None
-    return a.plan(data.device)
+    return a.prepared(data.device, products)[1]
 
 
 def rmatvec(a, data: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
@@ -73,7 +73,7 @@ def rmatvec(a, data: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     _, indices, indptr = a.buffers(data.device)
     ah = _adjoint_csr(a, data)
     if ah is not None:
-        (d, i, p), plan = ah.prepared(data.device)
+        (d, i, p), plan = ah.prepared(data.device, 1)
         return _native.csr_matvec(d, i, p, g, ah.shape, plan=plan)
     return _native.csr_matvec_transpose(_conj(data), indices, indptr, g, a.shape)
 
@@ -115,7 +115,7 @@ class CSRMatVec(torch.autograd.Function):
 
     @staticmethod
     def forward(data, x, a, planned=True):
-        plan = _own_plan(a, data) if planned else None
+        plan = _own_plan(a, data, 1) if planned else None
         _, indices, indptr = a.buffers(data.device)
         return _native.csr_matvec(data, indices, indptr, x, a.shape, plan=plan)
 
@@ -166,7 +166,7 @@ class CSRMatMul(torch.autograd.Function):
     @staticmethod
     def forward(data, X, a, planned=True):
         _, indices, indptr = a.buffers(data.device)
-        plan = _own_plan(a, data) if planned else None
+        plan = _own_plan(a, data, 0) if planned else None
         return _native.csr_matmul(data, indices, indptr, X, a.shape, plan=plan)
 
     @staticmethod
@@ -267,7 +267,7 @@ class MatVecDataVjp(torch.autograd.Function):
     def forward(x, g, a):
         # the gradient does not read the values: the plan serves whatever
         # values it is bound to
-        (_, indices, indptr), plan = a.prepared(x.device)
+        (_, indices, indptr), plan = a.prepared(x.device, 1)
         return _native.csr_matvec_data_vjp(indices, indptr, _conj(x), g.contiguous(), a.shape,
                                            plan=plan)
 

@@ -38,6 +38,10 @@ from mlx_sparse._validation import (
 )
 
 
+# Products after which a plan's deferred panels are built: they are repaid
+# after 32 (1.3 M rows of 16) to 130 (350,000 over 1.1 M columns).
+_REPAID = 64
+
 # Cache keys of a device: building its name anew cost 1 us a call.
 _DEVICE_NAMES: dict[torch.device, str] = {}
 
@@ -140,13 +144,19 @@ class CSRArray:
     def plan(self, device=None):
         """The GPU plan for ``device``, bound to :meth:`buffers` (None on the
         CPU, or when the ``gpu_plan`` runtime option is off).  Built once;
-        refreshed when the values changed, rebuilt when the structure did."""
+        refreshed when the values changed, rebuilt when the structure did.
+        Asked for here, it holds all it will hold; a product that finds none
+        builds one whose panels, where only many products repay them, wait for
+        that many."""
         device = _indexed(device if device is not None else self.device)
-        return self.prepared(device)[1] if device.type == "cuda" and runtime.gpu_plan() else None
+        if device.type != "cuda" or not runtime.gpu_plan():
+            return None
+        self._cache["kept"] = True
+        return self.prepared(device)[1]
 
-    def prepared(self, device) -> tuple:
-        """``(buffers(device), plan(device))``, the cached state looked up
-        and checked once for both."""
+    def prepared(self, device, products: int = 0) -> tuple:
+        """``(buffers(device), plan)``, the cached state looked up and checked
+        once for both, ahead of ``products`` products with a vector."""
         device = _indexed(device)
         now = self._stamps()
         bufs = self._buffers(device, now)
@@ -160,16 +170,29 @@ class CSRArray:
                 if built[0] != now[0]:
                     plan.refresh(bufs[0])
                     self._cache[key] = (now, plan)
-                return bufs, plan
+                if not plan.deferred or not self._repaid(plan, products):
+                    return bufs, plan
         from mlx_sparse import _native
 
-        # bound to these buffers: may hold a reordered copy of the values
+        # bound to these buffers: may hold a reordered copy of the values (a
+        # late one only where torch counts what is written to them)
         data, indices, indptr = bufs
         plan = _native.csr_plan(indptr, self.shape[0], self.nnz, data=data, indices=indices,
                                 n_cols=self.shape[1],
-                                slice_mode=int(runtime.get(runtime.RuntimeOption.GPU_SLICE)))
+                                slice_mode=int(runtime.get(runtime.RuntimeOption.GPU_SLICE)),
+                                defer="kept" not in self._cache or now[0][1] < 0)
+        if plan.deferred:
+            plan.served = products
         self._cache[key] = (now, plan)
         return bufs, plan
+
+    def _repaid(self, plan, products: int) -> bool:
+        """Whether a deferred plan is to be built again with its panels."""
+        plan.served += products
+        if plan.served > _REPAID:
+            self._cache["kept"] = True
+        return ("kept" in self._cache and not self.data.is_inference()
+                and not torch.cuda.is_current_stream_capturing())
 
     def _with_values(self, data: torch.Tensor) -> "CSRArray":
         """The same structure with other values, taking over this array's
@@ -181,7 +204,15 @@ class CSRArray:
         for key in [k for k in self._cache if k[0] == "plan"]:
             built, plan = self._cache.pop(key)
             out._cache[key] = (((None, None),) + tuple(built[1:]), plan)
+        self._share_use(out)
         return out
+
+    def _share_use(self, other: "CSRArray") -> "CSRArray":
+        """``other`` is used as often as this array: its panels do not wait
+        where this one's no longer do."""
+        if "kept" in self._cache:
+            other._cache["kept"] = True
+        return other
 
     # -- operators ---------------------------------------------------------
     def __matmul__(self, rhs):
@@ -219,7 +250,7 @@ class CSRArray:
         if hit is not None:
             built, T, layout = hit
             if built == now:
-                return T
+                return self._share_use(T)
             if built[1:] == now[1:] and data.device.type == "cuda":
                 if layout is None:
                     pos = _native.csr_transpose_positions(indices, indptr, self.shape)[0]
@@ -230,7 +261,7 @@ class CSRArray:
                 _native.csr_transpose_values_layout(data.detach(), layout, conjugate, scratch, t_data)
                 T = T._with_values(t_data)
                 self._cache[key] = (now, T, layout)
-                return T
+                return self._share_use(T)
         src = data.detach()
         if conjugate:
             src = src.conj().resolve_conj()
@@ -244,7 +275,7 @@ class CSRArray:
             has_canonical_format=self.has_canonical_format,
         )
         self._cache[key] = (now, T, None)
-        return T
+        return self._share_use(T)
 
     def transpose(self) -> "CSRArray":
         """Transpose, returning a ``CSRArray`` of shape ``(n_cols, n_rows)``

@@ -149,9 +149,10 @@ def csr_gmres_jacobi(data, indices, indptr, b, x0, inv_diag, shape: Shape2D, *, 
 
 
 def csr_plan(indptr, n_rows: int, nnz: int, block_nnz: int = 0, *, data=None, indices=None,
-             n_cols: int = -1, slice_mode: int = 0):
+             n_cols: int = -1, slice_mode: int = 0, defer: bool = False):
     """Row-block plan; with ``data``/``indices`` a plan bound to the matrix,
     which may hold a reordered copy for scattered gathers (slice_mode 0 auto,
-    1 off, 2 XCD column slices, 3 LDS column panels)."""
+    1 off, 2 XCD column slices, 3 LDS column panels; ``defer``: auto's panels
+    wait where only many products repay their build)."""
     return extension().csr_plan(indptr, n_rows, nnz, block_nnz, data=data, indices=indices,
-                                n_cols=n_cols, slice_mode=slice_mode)
+                                n_cols=n_cols, slice_mode=slice_mode, defer=defer)

@@ -67,7 +67,7 @@ def csr_matvec(a: CSRArray, x) -> torch.Tensor:
         from mlx_sparse._autograd import CSRMatVec
 
         return CSRMatVec.apply(a.data.to(x.device), x, a, True)
-    (data, indices, indptr), plan = a.prepared(device)
+    (data, indices, indptr), plan = a.prepared(device, 1)
     return _native.csr_matvec(data, indices, indptr, x, a.shape, plan=plan)
 
 

@@ -40,6 +40,11 @@ def _float32_csr(A, solver: str = "cg") -> CSRArray:
     return A
 
 
+def _solve_plan(csr: CSRArray, device):
+    # a solve multiplies some tens of times
+    return csr.prepared(device, 24)[1]
+
+
 def _float32_vector(x, device) -> torch.Tensor:
     t = ensure_array(x, device=device)
     if t.is_complex():
@@ -78,7 +83,7 @@ def cg(A, b, *, x0=None, rtol: float = 1e-5, atol: float = 0.0, maxiter: int | N
     if maxiter_value < 0:
         raise ValueError("maxiter must be non-negative.")
     data, indices, indptr = csr.buffers(device)
-    plan = csr.plan(device)
+    plan = _solve_plan(csr, device)
     kind = None
     inv_diag = None
     if M is not None:
@@ -209,11 +214,11 @@ def bicgstab(A, b, x0=None, *, rtol: float | None = None, atol: float = 0.0,
     if inv_diag is None:
         x, info, residual, iterations = _native.csr_bicgstab(
             data, indices, indptr, rhs, guess, csr.shape, rtol=rtol_value, atol=atol_value,
-            maxiter=maxiter_value, plan=csr.plan(device))
+            maxiter=maxiter_value, plan=_solve_plan(csr, device))
     else:
         x, info, residual, iterations = _native.csr_bicgstab_jacobi(
             data, indices, indptr, rhs, guess, inv_diag, csr.shape, rtol=rtol_value,
-            atol=atol_value, maxiter=maxiter_value, plan=csr.plan(device))
+            atol=atol_value, maxiter=maxiter_value, plan=_solve_plan(csr, device))
     return finish(x, info, residual, iterations, solver="bicgstab", return_info=bool(return_info),
                   callback=callback, rtol=rtol_value, atol=atol_value, maxiter=maxiter_value,
                   preconditioner=kind)
@@ -242,7 +247,7 @@ def minres(A, b, *, x0=None, rtol: float = 1e-5, atol: float = 0.0, shift: float
     if inv_diag is None:
         x, info, residual, iterations = _native.csr_minres(
             data, indices, indptr, rhs, guess, csr.shape, rtol=float(rtol), atol=float(atol),
-            maxiter=maxiter_value, shift=shift_value, plan=csr.plan(device))
+            maxiter=maxiter_value, shift=shift_value, plan=_solve_plan(csr, device))
     else:
         # reference: mlx_sparse/linalg/_iterative.py:1087-1096
         if check_preconditioner and (not pc.is_symmetric
@@ -252,7 +257,7 @@ def minres(A, b, *, x0=None, rtol: float = 1e-5, atol: float = 0.0, shift: float
                              "diagonal inverse entries must be finite and strictly positive.")
         x, info, residual, iterations = _native.csr_minres_jacobi(
             data, indices, indptr, rhs, guess, inv_diag, csr.shape, rtol=float(rtol),
-            atol=float(atol), maxiter=maxiter_value, shift=shift_value, plan=csr.plan(device))
+            atol=float(atol), maxiter=maxiter_value, shift=shift_value, plan=_solve_plan(csr, device))
     return finish(x, info, residual, iterations, solver="minres", return_info=bool(return_info),
                   callback=callback, rtol=float(rtol), atol=float(atol), maxiter=maxiter_value,
                   preconditioner=kind)
@@ -290,12 +295,12 @@ def gmres(A, b, *, x0=None, rtol: float = 1e-5, atol: float = 0.0, restart: int 
     if inv_diag is None:
         x, info, residual, iterations = _native.csr_gmres(
             data, indices, indptr, rhs, guess, csr.shape, rtol=float(rtol), atol=float(atol),
-            restart=restart_value, maxiter=maxiter_value, plan=csr.plan(device))
+            restart=restart_value, maxiter=maxiter_value, plan=_solve_plan(csr, device))
     else:
         x, info, residual, iterations = _native.csr_gmres_jacobi(
             data, indices, indptr, rhs, guess, inv_diag, csr.shape, rtol=float(rtol),
             atol=float(atol), restart=restart_value, maxiter=maxiter_value,
-            plan=csr.plan(device))
+            plan=_solve_plan(csr, device))
     return finish(x, info, residual, iterations, solver="gmres", return_info=bool(return_info),
                   callback=callback, callback_type=callback_type, rtol=float(rtol),
                   atol=float(atol), maxiter=maxiter_value, restart=restart_value,

@@ -154,6 +154,7 @@ struct Plan {
   int64_t nnz = 0;
   std::string index_dtype;
   int device = -1;
+  int64_t served = 0;  // products since the panels were deferred
   py::object bound;  // tensors a bound plan was built from (kept alive)
   ~Plan() {
     if (p) msx_csr_plan_destroy(p);
@@ -162,7 +163,7 @@ struct Plan {
 
 std::shared_ptr<Plan> make_plan(py::handle indptr_obj, int64_t n_rows, int64_t nnz,
                                 int64_t block_nnz, py::object data_obj, py::object indices_obj,
-                                int64_t n_cols, int slice_mode) {
+                                int64_t n_cols, int slice_mode, bool defer) {
   py::object indptr = contiguous(indptr_obj);
   ArrayView v = view_of(indptr);
   msx::require_rank(v, 1, "csr_plan indptr");
@@ -195,7 +196,8 @@ std::shared_ptr<Plan> make_plan(py::handle indptr_obj, int64_t n_rows, int64_t n
     msx::require_contiguous(vi, "csr_plan indices");
     plan->bound = py::make_tuple(data_obj, indices_obj, indptr);
     // A plan is cached with its matrix and used from every stream and thread.
-    msx_plan_options opts{block_nnz, slice_mode, MSX_PLAN_CALL_SCRATCH};
+    msx_plan_options opts{block_nnz, slice_mode,
+                          MSX_PLAN_CALL_SCRATCH | (defer ? MSX_PLAN_DEFER : 0)};
     py::gil_scoped_release nogil;
     st = msx_csr_plan_create_bound(msx::to_vtype(vd.dtype), msx::to_itype(v.dtype), n_rows, n_cols,
                                    nnz, vd.ptr, vi.ptr, v.ptr, &opts, stream, &plan->p);
@@ -795,6 +797,8 @@ PYBIND11_MODULE(_ext, m) {
       .def_readonly("nnz", &Plan::nnz)
       .def_readonly("index_dtype", &Plan::index_dtype)
       .def_readonly("device", &Plan::device)
+      .def_property_readonly("deferred", [](const Plan &p) { return msx_csr_plan_deferred(p.p) != 0; })
+      .def_readwrite("served", &Plan::served)
       .def("info", &plan_info, "Plan summary (block and long-row counts, sizes).")
       .def("refresh", &plan_refresh, py::arg("data"),
            "The values changed (indices and indptr did not): rewrite the plan's copies "
@@ -811,9 +815,10 @@ PYBIND11_MODULE(_ext, m) {
         py::arg("n_cols"), "True when a product's operands pass every metadata check.");
   m.def("csr_plan", &make_plan, py::arg("indptr"), py::arg("n_rows"), py::arg("nnz"),
         py::arg("block_nnz") = 0, py::arg("data") = py::none(), py::arg("indices") = py::none(),
-        py::arg("n_cols") = -1, py::arg("slice_mode") = 0,
+        py::arg("n_cols") = -1, py::arg("slice_mode") = 0, py::arg("defer") = false,
         "Build a row-block plan from a GPU indptr; with data/indices, a plan bound to the "
-        "matrix (slice_mode 0 auto, 1 off, 2 column slices per XCD, 3 LDS column panels).");
+        "matrix (slice_mode 0 auto, 1 off, 2 column slices per XCD, 3 LDS column panels; "
+        "defer: auto's panels wait where only many products repay them).");
   m.def("csr_matvec", &csr_matvec, py::arg("data"), py::arg("indices"), py::arg("indptr"),
         py::arg("x"), py::arg("n_rows"), py::arg("n_cols"), py::arg("plan") = py::none(),
         py::arg("n_threads") = 0, "Multiply CSR buffers by a dense vector.");

@@ -1,0 +1,119 @@
+"""Panels that only many products repay: they wait for those, and until then -
+and where torch does not count what is written to the values, or a graph
+replays a product - the values are read as they are."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import mlx_sparse as ms
+from mlx_sparse import _csr
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+N_ROWS, N_COLS, VALUES = 400_000, (4 << 20) // 4, 5 << 20  # the smallest that take panels
+
+
+@pytest.fixture(autouse=True)
+def on_the_gpu():
+    ms.use_gpu()
+
+
+@pytest.fixture(scope="module")
+def buffers():
+    rng = np.random.default_rng(83)
+    indptr = np.zeros(N_ROWS + 1, np.int32)
+    np.cumsum(rng.multinomial(VALUES, np.ones(N_ROWS) / N_ROWS), out=indptr[1:])
+    # small integers: every order of additions is exact
+    data = rng.integers(-2, 3, VALUES).astype(np.float32)
+    indices = rng.integers(0, N_COLS, VALUES).astype(np.int32)
+    return tuple(torch.from_numpy(t).to(DEV) for t in (data, indices, indptr))
+
+
+def _array(buffers):
+    data, indices, indptr = buffers
+    return ms.csr_array((data.clone(), indices, indptr), shape=(N_ROWS, N_COLS))
+
+
+def _want(a, x):
+    rows = torch.repeat_interleave(torch.arange(N_ROWS, device=DEV), a.indptr.diff())
+    out = torch.zeros(N_ROWS, dtype=torch.float64, device=DEV)
+    return out.index_add_(0, rows, (a.data.detach() * x[a.indices]).double()).float()
+
+
+def _panels(a):
+    return a._cache[("plan", "cuda:0")][1].info()["n_panels"]
+
+
+def _x(seed=1):
+    rng = np.random.default_rng(seed)
+    return torch.from_numpy(rng.integers(-2, 3, N_COLS).astype(np.float32)).to(DEV)
+
+
+def test_panels_wait_for_the_products_that_repay_them(buffers):
+    a, x = _array(buffers), _x()
+    want = _want(a, x)
+    print("late panels", flush=True)
+    for _ in range(3):  # products with a matrix do not use them
+        a @ x[:, None]
+    for i in range(_csr._REPAID):
+        assert torch.equal(a @ x, want)
+        assert _panels(a) == 0, i
+    assert torch.equal(a @ x, want) and _panels(a) > 0
+    assert a.T._cache["kept"]  # used as often
+    b = _array(buffers)
+    b.plan()
+    assert _panels(b) > 0 and torch.equal(b @ x, want)
+    b.data.mul_(2)
+    assert torch.equal(b @ x, 2 * want)
+
+
+@pytest.mark.parametrize("planned", [False, True])
+def test_uncounted_values_are_read_as_they_are(buffers, planned):
+    x = _x()
+    print(f"inference values planned={planned}", flush=True)
+    with torch.inference_mode():
+        a = _array(buffers)
+        want = _want(a, x)
+        if planned:
+            a.plan()
+        for _ in range(_csr._REPAID + 2):
+            y = a @ x
+        assert torch.equal(y, want)
+        a.data.mul_(2)
+        assert torch.equal(a @ x, 2 * want)
+
+
+def test_replayed_products_read_the_values_as_they_are(buffers):
+    a, x = _array(buffers), _x()
+    a.plan()
+    assert _panels(a) > 0
+    want = _want(a, x)
+    a @ x
+    torch.cuda.synchronize()
+    alone = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(alone):
+        y = a @ x
+    new = a.data.clone()
+    step = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(step):
+        a.data.copy_(new)
+        z = a @ x
+    print("replays", flush=True)
+    for i in range(1, 4):
+        new.mul_(2)
+        want = 2 * want
+        step.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z, want), i
+        alone.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), i
+        assert torch.equal(a @ x, want), i
+        a.data.mul_(-1)
+        alone.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, -want) and torch.equal(a @ x, -want), i
