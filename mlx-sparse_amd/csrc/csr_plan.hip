@@ -483,11 +483,10 @@ extern "C" msx_status msx_csr_plan_create_bound(msx_vtype vt, msx_itype it, int6
     // or more and panels are not taken.
     mode = MSX_SLICE_OFF;
     bool scattered = false;
-    int64_t short_values = 0;
     const int64_t x_bytes = n_cols * static_cast<int64_t>(value_bytes(vt));
     const bool panels = panels_pay(p) && panels_eligible(p);
     const bool slices = x_bytes >= kSliceMinX;
-    if (panels || slices) st = probe_scattered(p, indices, s, &scattered, &short_values);
+    if (panels || slices) st = probe_scattered(p, indices, s, &scattered);
     if (scattered) mode = panels ? MSX_SLICE_PANELS : MSX_SLICE_ON;
     if (mode == MSX_SLICE_PANELS && !panels_at_once(p)) {
       p->deferred = (opts->flags & MSX_PLAN_DEFER) != 0;

@@ -74,24 +74,23 @@ __device__ inline BlockRange block_range(const int32_t *bounds, const int64_t *b
 
 // ---------------------------------------------------------------------------
 // Probe: count short blocks whose valid columns span more than n_cols / 4
-// (counter[0]) and the values of all short blocks (counter[1]).
+// (*counter).
 template <class I, int W>
 __global__ void __launch_bounds__(kThreads)
     slice_probe(const I *__restrict__ indices, const int32_t *__restrict__ bounds,
                 const int64_t *__restrict__ bounds_nnz, int64_t n_bounds, int64_t nnz,
                 int64_t n_cols, unsigned long long *__restrict__ counter) {
   // Each wave walks blocks with a stride of the grid and keeps its counts in
-  // registers; one atomic per counter and workgroup (an atomic per block
-  // serialises hundreds of thousands of them on two addresses).
-  __shared__ unsigned long long wg_count[2][kWavesPerGroup];
+  // registers; one atomic per workgroup (an atomic per block serialises
+  // hundreds of thousands of them on one address).
+  __shared__ unsigned long long wg_count[kWavesPerGroup];
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
-  unsigned long long scattered = 0, values = 0;
+  unsigned long long scattered = 0;
   for (int64_t b = static_cast<int64_t>(blockIdx.x) * kWavesPerGroup + wave; b < n_bounds;
        b += static_cast<int64_t>(gridDim.x) * kWavesPerGroup) {
     const BlockRange br = block_range<W>(bounds, bounds_nnz, b, nnz);
     if (!br.valid || br.p1 <= br.p0) continue;
-    values += static_cast<unsigned long long>(br.p1 - br.p0);
     int64_t lo = INT64_MAX, hi = -1;
     // a block holds < 2W values: four unconditional loads per lane and step
     const auto rr = make_rsrc(indices + br.p0, static_cast<uint64_t>(br.p1 - br.p0) * sizeof(I));
@@ -118,19 +117,12 @@ __global__ void __launch_bounds__(kThreads)
     }
     if (hi >= lo && hi - lo > n_cols / 4) ++scattered;
   }
-  if (lane == 0) {
-    wg_count[0][wave] = scattered;
-    wg_count[1][wave] = values;
-  }
+  if (lane == 0) wg_count[wave] = scattered;
   __syncthreads();
   if (threadIdx.x == 0) {
-    unsigned long long a = 0, v = 0;
-    for (int w = 0; w < kWavesPerGroup; ++w) {
-      a += wg_count[0][w];
-      v += wg_count[1][w];
-    }
+    unsigned long long a = 0;
+    for (int w = 0; w < kWavesPerGroup; ++w) a += wg_count[w];
     if (a > 0) atomicAdd(counter, a);
-    if (v > 0) atomicAdd(counter + 1, v);
   }
 }
 
@@ -393,35 +385,34 @@ int bits_for(int64_t v) {  // smallest b with v <= 2^b
 
 template <class I, int W>
 msx_status probe_typed(const msx_csr_plan *p, const void *indices, hipStream_t stream,
-                       bool *scattered, int64_t *short_values) {
+                       bool *scattered) {
   const int64_t groups = std::min<int64_t>((p->n_bounds + kWavesPerGroup - 1) / kWavesPerGroup, 2048);
-  unsigned long long *counter = nullptr;
-  MSX_HIP_TRY(hipMallocAsync(reinterpret_cast<void **>(&counter), 2 * sizeof(*counter), stream));
-  MSX_HIP_TRY(hipMemsetAsync(counter, 0, 2 * sizeof(*counter), stream));
+  // in the plan's own scratch, which no call uses yet (an allocation for it
+  // took 40 us)
+  auto *counter = static_cast<unsigned long long *>(p->partials);
+  MSX_HIP_TRY(hipMemsetAsync(counter, 0, sizeof(*counter), stream));
   hipLaunchKernelGGL((slice_probe<I, W>), dim3(static_cast<uint32_t>(groups)), dim3(kThreads), 0,
                      stream, static_cast<const I *>(indices), p->bounds, p->bounds_nnz,
                      p->n_bounds, p->nnz, p->n_cols, counter);
-  unsigned long long count[2] = {0, 0};
+  unsigned long long count = 0;
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
-    e = hipMemcpyAsync(count, counter, sizeof(count), hipMemcpyDeviceToHost, stream);
+    e = hipMemcpyAsync(&count, counter, sizeof(count), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  (void)hipFreeAsync(counter, stream);
   if (e != hipSuccess) return hip_fail(e, "slice probe");
-  *scattered = 2 * static_cast<int64_t>(count[0]) > p->n_blocks;  // else mostly local
-  *short_values = static_cast<int64_t>(count[1]);
+  *scattered = 2 * static_cast<int64_t>(count) > p->n_blocks;  // else mostly local
   return MSX_OK;
 }
 
 template <class I>
 msx_status probe_w(const msx_csr_plan *p, const void *indices, hipStream_t stream,
-                   bool *scattered, int64_t *short_values) {
+                   bool *scattered) {
   switch (p->block_nnz) {
-  case 64: return probe_typed<I, 64>(p, indices, stream, scattered, short_values);
-  case 128: return probe_typed<I, 128>(p, indices, stream, scattered, short_values);
-  case 256: return probe_typed<I, 256>(p, indices, stream, scattered, short_values);
-  case 512: return probe_typed<I, 512>(p, indices, stream, scattered, short_values);
-  default: return probe_typed<I, 1024>(p, indices, stream, scattered, short_values);
+  case 64: return probe_typed<I, 64>(p, indices, stream, scattered);
+  case 128: return probe_typed<I, 128>(p, indices, stream, scattered);
+  case 256: return probe_typed<I, 256>(p, indices, stream, scattered);
+  case 512: return probe_typed<I, 512>(p, indices, stream, scattered);
+  default: return probe_typed<I, 1024>(p, indices, stream, scattered);
   }
 }
 
@@ -540,13 +531,12 @@ msx_status refresh_slices(msx_csr_plan *p, const void *data, hipStream_t stream)
 }
 
 msx_status probe_scattered(const msx_csr_plan *p, const void *indices, hipStream_t stream,
-                           bool *scattered, int64_t *short_values) {
+                           bool *scattered) {
   *scattered = false;
-  *short_values = 0;
   const int64_t x_bytes = p->n_cols * static_cast<int64_t>(value_bytes(p->vtype));
   if (x_bytes < kPanelMinX || p->n_bounds == 0 || p->n_blocks == 0) return MSX_OK;
-  return p->itype == MSX_I32 ? probe_w<int32_t>(p, indices, stream, scattered, short_values)
-                             : probe_w<int64_t>(p, indices, stream, scattered, short_values);
+  return p->itype == MSX_I32 ? probe_w<int32_t>(p, indices, stream, scattered)
+                             : probe_w<int64_t>(p, indices, stream, scattered);
 }
 
 msx_status launch_spmv_sliced(const msx_csr_plan *p, const void *x, void *y, hipStream_t stream) {

@@ -209,10 +209,10 @@ msx_status launch_spmv_sliced(const msx_csr_plan *p, const void *x, void *y, hip
 msx_status refresh_slices(msx_csr_plan *p, const void *data, hipStream_t stream);
 msx_status refresh_panels(msx_csr_plan *p, const void *data, hipStream_t stream);
 // True when most short blocks have valid columns spread over more than a
-// quarter of x (the AUTO rule's test for a reordered copy); also the number
-// of values in short blocks.  Synchronises `stream`.
+// quarter of x (the AUTO rule's test for a reordered copy).  Synchronises
+// `stream`.
 msx_status probe_scattered(const msx_csr_plan *p, const void *indices, hipStream_t stream,
-                           bool *scattered, int64_t *short_values);
+                           bool *scattered);
 // The AUTO rule's sizes for a panel copy of a scattered matrix.  In row
 // blocks each value costs a gather that misses more often the further x
 // outgrows an XCD's 4 MB L2 (per million values: 4.7 us at 1 MB of x, 6.9 at
