@@ -136,7 +136,7 @@ class CSRArray:
             return hit[1]
         old_stamps, old = hit if hit is not None else ((None,) * 3, (None,) * 3)
         bufs = tuple(
-            o if o is not None and was == cur else t.to(device).contiguous()
+            o if o is not None and was == cur else t.to(device).resolve_conj().resolve_neg().contiguous()
             for t, o, was, cur in zip((self.data, self.indices, self.indptr), old, old_stamps, now))
         self._cache[key] = (now, bufs)
         return bufs

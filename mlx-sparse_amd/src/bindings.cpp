@@ -130,8 +130,12 @@ py::object as_tensor(py::handle obj) {
   return torch().attr("as_tensor")(obj);
 }
 
+// Contiguous memory that holds the operand's own values: torch keeps
+// conjugates and some negations as a flag on the memory of another tensor.
 py::object contiguous(py::handle obj) {
   py::object t = as_tensor(obj);
+  if (tensor_of(t).is_conj()) t = t.attr("resolve_conj")();
+  if (tensor_of(t).is_neg()) t = t.attr("resolve_neg")();
   if (tensor_of(t).is_contiguous()) return t;
   return t.attr("contiguous")();
 }
