@@ -285,8 +285,6 @@ ScratchSizes scratch_sizes(const msx_csr_plan *p) {
   return z;
 }
 
-// No system fence: the event orders work of this device alone (2.5 us of a
-// training step of 454 instead of 5).
 // Events inside and outside a capture cannot order each other; a stream whose
 // state cannot be asked for (another one captures) counts as capturing.
 bool capturing(hipStream_t stream) {
@@ -309,10 +307,15 @@ unsigned long long capture_of(hipStream_t stream) {
 msx_status mark_refreshed(msx_csr_plan *p, hipStream_t stream) {
   p->refreshed_in = capture_of(stream);
   if (capturing(stream)) return MSX_OK;
-  if (p->refreshed == nullptr)
-    MSX_HIP_TRY(hipEventCreateWithFlags(&p->refreshed, hipEventDisableTiming | hipEventDisableSystemFence));
-  MSX_HIP_TRY(hipEventRecord(p->refreshed, stream));
   p->refreshed_on = stream;
+  const bool event = __atomic_load_n(&p->shared, __ATOMIC_ACQUIRE);
+  if (event) {
+    // no system fence: it orders work of this device alone
+    if (p->refreshed == nullptr)
+      MSX_HIP_TRY(hipEventCreateWithFlags(&p->refreshed, hipEventDisableTiming | hipEventDisableSystemFence));
+    MSX_HIP_TRY(hipEventRecord(p->refreshed, stream));
+  }
+  __atomic_store_n(&p->unmarked, !event, __ATOMIC_RELEASE);
   return MSX_OK;
 }
 
@@ -322,8 +325,17 @@ PlanUse::PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStrea
                  bool values)
     : plan_(plan), stream_(stream) {
   if (plan == nullptr) return;
-  if (values && plan->refreshed != nullptr && plan->refreshed_on != stream && !capturing(stream)) {
-    const hipError_t e = hipStreamWaitEvent(stream, plan->refreshed, 0);
+  const bool unmarked = __atomic_load_n(&plan->unmarked, __ATOMIC_ACQUIRE);
+  if (values && (unmarked || plan->refreshed != nullptr) && plan->refreshed_on != stream &&
+      !capturing(stream)) {
+    hipError_t e;
+    if (unmarked) {
+      __atomic_store_n(&plan->shared, true, __ATOMIC_RELEASE);
+      e = hipDeviceSynchronize();
+      if (e == hipSuccess) __atomic_store_n(&plan->unmarked, false, __ATOMIC_RELEASE);
+    } else {
+      e = hipStreamWaitEvent(stream, plan->refreshed, 0);
+    }
     if (e != hipSuccess) {
       status_ = hip_fail(e, "waiting for a plan's refresh");
       return;

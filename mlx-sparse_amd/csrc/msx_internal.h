@@ -78,10 +78,14 @@ struct msx_csr_plan {
   bool call_scratch;          // MSX_PLAN_CALL_SCRATCH: pn_prod and s_partial are null
   const void *bound_data;     // the buffers a bound plan was built from (data: as last refreshed)
   const void *bound_indices;
-  // The last refresh of the value copies outside a capture: calls on other
-  // streams than its own wait for it.
-  hipEvent_t refreshed;       // null before the first
+  // The last refresh of the value copies outside a capture, which calls on
+  // other streams wait for.  The first that comes waits on the host; from then
+  // on each refresh leaves an event (a plan of one stream goes without: 4 us
+  // of a training step of 453).
   hipStream_t refreshed_on;
+  hipEvent_t refreshed;       // null before the first event
+  mutable bool unmarked;      // no event since the refresh (accessed atomically)
+  mutable bool shared;        // used from several streams (accessed atomically)
   unsigned long long refreshed_in;  // the capture that holds a refresh, 0: none
   // Panels that AUTO takes below the sizes where it always does
   // (panels_at_once): `deferred`, row blocks until the caller asks again
