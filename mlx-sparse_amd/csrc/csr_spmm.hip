@@ -224,7 +224,7 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
 // SKIP: rows of more than max_len values that the plan lists are left to
 // spmm_long.  Its own instance: the test's registers cost the LR = 8 one two
 // spills (k = 32 on the 3D Poisson matrix: 176 -> 214 us).
-// ANY: rows of any length k >= CW at any element alignment: the lane whose
+// ANY (ragged_sixteen): rows of any length k >= CW at any element alignment: the lane whose
 // columns would pass k takes the row's last CW instead (its neighbour's in
 // part, the same sums), so every load and store is whole.  16-bit, k = 100,
 // 300,007 rows of 20: one 2-byte column per lane 683 us, this 266.
@@ -1132,6 +1132,37 @@ __attribute__((amdgpu_waves_per_eu(LG <= 3 ? 7 : 1, 8)))
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Whether rows of X that are no whole aligned sixteen-byte vectors are read
+// sixteen bytes a lane (spmm_rows' ANY) or one column a lane.  16-bit values
+// always (1.03 to 7 times faster).  Others, measured one column a lane ->
+// sixteen bytes, us:
+// - windows of a plan that reach over at most a quarter of the columns (X rows
+//   come from the caches): sixteen bytes (3D Poisson 100^3 float32 k = 9 81 ->
+//   35, banded 21 a row k = 9 38 -> 18), but not two lanes a row on longer
+//   rows, whose values then pass one by one (banded complex64, 21 a row, k = 3
+//   21.7 -> 33.5, six a row 26.9 -> 20.1; float32 52 a row k = 5 8.7 -> 9.3, 21
+//   a row 22.8 -> 18.3);
+// - elsewhere, or not known: k > 32 (float32, 1 M rows of 16, k = 33 645 ->
+//   580); from eight lanes a row on where X is at most 16 MB or rows are short
+//   (30,000 rows of 16, k = 25 10.1 -> 8.6, 200,000 of 8 51 -> 45, 1 M of 16 484
+//   -> 514); fewer lanes load a row's indices and values in pieces (200,000
+//   rows of 16, k = 6 27.6 -> 34.7), worth it for rows of fewer than eight
+//   values (200,000 rows of 5, k = 9 19.7 -> 16.2; not complex64 where the
+//   plan knows that columns are scattered: 300,000 rows of 7, k = 5 38 -> 44).
+bool ragged_sixteen(size_t sv, int64_t n_rows, int64_t n_cols, int64_t nnz, int64_t k,
+                    const msx_csr_plan *plan) {
+  const int64_t per16 = 16 / static_cast<int64_t>(sv);
+  if (k < per16) return false;
+  if (sv == 2) return true;
+  const int64_t mean = nnz / n_rows;
+  const int64_t lanes = (k + per16 - 1) / per16;
+  const bool known = plan != nullptr && plan->win_rows_max > 0;
+  if (known && 4 * plan->win_rows_max <= n_cols) return lanes > 2 || mean < (sv == 4 ? 32 : 10);
+  if (k > 32) return true;
+  if (lanes > 4) return mean < 14 || n_cols * k * static_cast<int64_t>(sv) <= (int64_t{16} << 20);
+  return mean < 8 && !(known && sv == 8);
+}
+
 
 
 template <class V, class I>
@@ -1242,7 +1273,7 @@ msx_status spmm_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *d
   }
   // Sixteen bytes a lane; shorter rows (k < CWV, at most eight lanes) one
   // column a lane (float32, k = 3, 1 M rows of 16: 268 us, two columns 285).
-  const int CW = k >= CWV ? CWV : 1;
+  const int CW = vec || ragged_sixteen(sizeof(S), n_rows, n_cols, nnz, k, plan) ? CWV : 1;
   const int64_t lanes = (k + CW - 1) / CW;
   int LR = 1;
   while (LR < lanes && LR < 64) LR <<= 1;

@@ -187,6 +187,45 @@ def test_spmm_rows_of_any_length_and_alignment(vtype):
             assert bool((out[:, :skip] == 7).all()) and bool((out[:, skip + k:] == 7).all())
 
 
+@pytest.mark.parametrize("kind", ["short_rows", "banded_plan", "scattered"])
+@pytest.mark.parametrize("vtype", VTYPES)
+def test_spmm_ragged_rows_on_either_side_of_the_rule(kind, vtype):
+    """Ragged and misaligned X rows where they are read sixteen bytes a lane
+    (short rows; a plan with narrow column windows; 16-bit values) and where
+    one column a lane: the oracle's bits, nothing written past a row's end."""
+    rng = np.random.default_rng(71)
+    n_rows, n_cols = 700, 40_000
+    if kind == "short_rows":
+        lengths = rng.integers(0, 13, n_rows)
+    else:
+        lengths = rng.integers(8, 21, n_rows)
+    assert (lengths.sum() // n_rows < 8) == (kind == "short_rows")
+    indices, indptr = _csr(rng, lengths, n_cols)
+    if kind == "banded_plan":
+        indices = (indices % 40 + np.repeat(np.arange(n_rows) * 50, lengths)).astype(np.int32)
+    data = _values(rng, indices.size, vtype)
+    d, i, p = to_torch(data, vtype, DEV), to_torch(indices, None, DEV), to_torch(indptr, None, DEV)
+    plan = None
+    if kind == "banded_plan":
+        plan = _capi.Plan(p, n_rows, indices.size, data=d, indices=i, n_cols=n_cols)
+        assert 0 < 4 * plan.info().window_rows <= n_cols
+    for k in (2, 3, 4, 5, 7, 9, 13, 15, 17, 31, 33):
+        X = _values(rng, (n_cols, k), vtype)
+        want = orc.csr_matmul(data, indices, indptr, X, n_rows, vtype=vtype)
+        print(f"spmm ragged {kind} {vtype} k={k}", flush=True)
+        for pad, skip in ((0, 0), (2, 1)):
+            wide = torch.zeros(n_cols, k + pad + skip, dtype=d.dtype, device=DEV)
+            wide[:, skip:skip + k] = to_torch(X, vtype, DEV)
+            out = torch.full((n_rows, k + pad + skip), 7, dtype=d.dtype, device=DEV)
+            _capi.spmm(d, i, p, wide[:, skip:skip + k], n_rows, n_cols, plan=plan,
+                       Y=out[:, skip:skip + k])
+            got = out[:, skip:skip + k].contiguous()
+            assert to_numpy(got).tobytes() == want.tobytes(), (k, pad)
+            assert bool((out[:, :skip] == 7).all()) and bool((out[:, skip + k:] == 7).all())
+    if plan is not None:
+        plan.close()
+
+
 @pytest.mark.parametrize("kind", ["one_row", "edges", "empty_runs", "skewed"])
 @pytest.mark.parametrize("vtype", ["float32", "bfloat16", "complex64"])
 def test_transposed_products_by_positions(kind, vtype):
