@@ -47,12 +47,14 @@ struct Counts {
   int64_t bounds;  // rows that start a short block or are long
   int64_t longs;
   int64_t chunks;
+  int64_t longest;  // values of the longest row; read from the totals only
 };
 
 struct RowClass {
   bool start;
   bool is_long;
   int64_t chunks;
+  int64_t len;
 };
 
 template <class I>
@@ -62,6 +64,7 @@ __device__ inline RowClass classify(const I *__restrict__ indptr, int64_t r, int
   const int64_t e = static_cast<int64_t>(indptr[r + 1]);
   const int64_t len = e - b;
   RowClass c;
+  c.len = len;
   c.is_long = len > W;
   c.chunks = c.is_long ? (len + C - 1) / C : 0;
   if (c.is_long) {
@@ -77,6 +80,20 @@ __device__ inline RowClass classify(const I *__restrict__ indptr, int64_t r, int
     c.start = prev_long || wb != wp;
   }
   return c;
+}
+
+// Largest of one int64 per thread across a 256-thread workgroup.
+__device__ inline int64_t block_max(int64_t v, int64_t *lds_waves) {
+#pragma unroll
+  for (int d = kWave / 2; d >= 1; d >>= 1) {
+    const int64_t u = __shfl_xor(v, d, kWave);
+    v = u > v ? u : v;
+  }
+  if (threadIdx.x % kWave == 0) lds_waves[threadIdx.x / kWave] = v;
+  __syncthreads();
+  for (int w = 0; w < kPlanThreads / kWave; ++w) v = lds_waves[w] > v ? lds_waves[w] : v;
+  __syncthreads();
+  return v;
 }
 
 // Inclusive scan of one int64 per thread across a 256-thread workgroup.
@@ -103,7 +120,7 @@ __global__ void __launch_bounds__(kPlanThreads)
   __shared__ int64_t lds[3][kPlanThreads / kWave];
   const int64_t tile = blockIdx.x;
   const int64_t r0 = tile * kTileRows + static_cast<int64_t>(threadIdx.x) * kRowsPerThread;
-  Counts c{0, 0, 0};
+  Counts c{0, 0, 0, 0};
   for (int i = 0; i < kRowsPerThread; ++i) {
     const int64_t r = r0 + i;
     if (r >= n) break;
@@ -111,34 +128,38 @@ __global__ void __launch_bounds__(kPlanThreads)
     c.bounds += rc.start || rc.is_long;
     c.longs += rc.is_long;
     c.chunks += rc.chunks;
+    c.longest = rc.len > c.longest ? rc.len : c.longest;
   }
   const int64_t s = block_inclusive_scan(c.bounds, lds[0]);
   const int64_t l = block_inclusive_scan(c.longs, lds[1]);
   const int64_t k = block_inclusive_scan(c.chunks, lds[2]);
-  if (threadIdx.x == kPlanThreads - 1) tile_counts[tile] = Counts{s, l, k};
+  const int64_t m = block_max(c.longest, lds[0]);
+  if (threadIdx.x == kPlanThreads - 1) tile_counts[tile] = Counts{s, l, k, m};
 }
 
 // Exclusive scan of the tile counts in place; totals land in `totals`.
 __global__ void __launch_bounds__(kPlanThreads)
     plan_scan(Counts *__restrict__ tile_counts, int64_t n_tiles, Counts *__restrict__ totals) {
   __shared__ int64_t lds[3][kPlanThreads / kWave];
-  Counts carry{0, 0, 0};
+  Counts carry{0, 0, 0, 0};
   for (int64_t base = 0; base < n_tiles; base += kPlanThreads) {
     const int64_t t = base + threadIdx.x;
-    const Counts v = t < n_tiles ? tile_counts[t] : Counts{0, 0, 0};
+    const Counts v = t < n_tiles ? tile_counts[t] : Counts{0, 0, 0, 0};
     const int64_t s = block_inclusive_scan(v.bounds, lds[0]);
     const int64_t l = block_inclusive_scan(v.longs, lds[1]);
     const int64_t k = block_inclusive_scan(v.chunks, lds[2]);
+    const int64_t m = block_max(v.longest, lds[0]);
     if (t < n_tiles)
       tile_counts[t] = Counts{carry.bounds + s - v.bounds, carry.longs + l - v.longs,
-                              carry.chunks + k - v.chunks};
+                              carry.chunks + k - v.chunks, 0};
     // the last thread holds the batch total; broadcast through LDS
     __shared__ Counts batch_total;
-    if (threadIdx.x == kPlanThreads - 1) batch_total = Counts{s, l, k};
+    if (threadIdx.x == kPlanThreads - 1) batch_total = Counts{s, l, k, m};
     __syncthreads();
     carry.bounds += batch_total.bounds;
     carry.longs += batch_total.longs;
     carry.chunks += batch_total.chunks;
+    carry.longest = batch_total.longest > carry.longest ? batch_total.longest : carry.longest;
     __syncthreads();
   }
   if (threadIdx.x == 0) *totals = carry;
@@ -154,7 +175,7 @@ __global__ void __launch_bounds__(kPlanThreads)
   __shared__ int64_t lds[3][kPlanThreads / kWave];
   const int64_t tile = blockIdx.x;
   const int64_t r0 = tile * kTileRows + static_cast<int64_t>(threadIdx.x) * kRowsPerThread;
-  Counts c{0, 0, 0};
+  Counts c{0, 0, 0, 0};
   for (int i = 0; i < kRowsPerThread; ++i) {
     const int64_t r = r0 + i;
     if (r >= n) break;
@@ -204,7 +225,7 @@ msx_status build_plan(msx_csr_plan *p, const I *indptr, hipStream_t stream) {
                        stream, indptr, n, p->block_nnz, p->block_rows, p->chunk_nnz, tmp);
     hipLaunchKernelGGL(plan_scan, dim3(1), dim3(kPlanThreads), 0, stream, tmp, n_tiles,
                        tmp + n_tiles);
-    Counts totals{0, 0, 0};
+    Counts totals{0, 0, 0, 0};
     hipError_t e = hipMemcpyAsync(&totals, tmp + n_tiles, sizeof(Counts), hipMemcpyDeviceToHost,
                                   stream);
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
@@ -215,6 +236,7 @@ msx_status build_plan(msx_csr_plan *p, const I *indptr, hipStream_t stream) {
     p->n_bounds = totals.bounds;
     p->n_long = totals.longs;
     p->n_chunks = totals.chunks;
+    p->longest = totals.longest;
     p->n_blocks = p->n_bounds - p->n_long;
   } else {
     p->n_bounds = p->n_blocks = p->n_long = p->n_chunks = 0;

@@ -56,6 +56,7 @@ struct msx_csr_plan {
   int64_t n_bounds;    // short blocks + long rows
   int64_t n_long;
   int64_t n_chunks;
+  int64_t longest;     // values of the longest row when the plan was built
   int device;
   size_t bytes;
   // Device arrays (rows < 2^31; chunk ids < 2^31 checked at build).

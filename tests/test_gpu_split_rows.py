@@ -160,6 +160,30 @@ def test_spmm_long_rows_in_stored_order(vtype, index_dtype):
     plan.close()
 
 
+@pytest.mark.parametrize("longest", [600, 9600, 9601])
+def test_spmm_where_every_row_is_long(longest):
+    """Rows of 600 values throughout, the longest at sixteen times the mean
+    and one value above it (then a workgroup takes it): the oracle's bits."""
+    rng = np.random.default_rng(83)
+    lengths = np.full(3000, 600)
+    lengths[1500] = longest
+    lengths[:100] -= (longest - 600) // 100
+    n_rows, n_cols = len(lengths), 2001
+    assert lengths.sum() // n_rows == 600
+    indices, indptr = _csr(rng, lengths, n_cols)
+    data = _values(rng, indices.size, "float32")
+    d, i, p = (to_torch(t, None, DEV) for t in (data, indices, indptr))
+    plan = _capi.Plan(p, n_rows, indices.size, data=d, indices=i, n_cols=n_cols)
+    assert plan.info().n_long_rows >= 2900
+    for k in (1, 6, 32, 64):
+        X = _values(rng, (n_cols, k), "float32")
+        print(f"every row long {longest} k={k}", flush=True)
+        got = _capi.spmm(d, i, p, to_torch(X, None, DEV), n_rows, n_cols, plan=plan)
+        want = orc.csr_matmul(data, indices, indptr, X, n_rows, n_threads=8)
+        assert to_numpy(got).tobytes() == want.tobytes(), k
+    plan.close()
+
+
 @pytest.mark.parametrize("vtype", VTYPES)
 def test_spmm_rows_of_any_length_and_alignment(vtype):
     """Rows of X and Y that are no multiple of sixteen bytes, or start off
