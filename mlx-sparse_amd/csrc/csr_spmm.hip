@@ -34,6 +34,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr uint32_t kMaxGrid = 1u << 20;
 constexpr int64_t kMaxBatchGrid = 65535;  // batches per launch (grid y extent)
+constexpr int64_t kMaxLongGrid = int64_t{1} << 22;  // workgroups of 576 threads: below 2^32 threads
 // A row is spmm_long's when it is long for the plan and longer than this many
 // mean rows: where most rows are alike, lane groups keep more of them going.
 constexpr int64_t kLongMeans = 16;
@@ -1239,7 +1240,10 @@ msx_status spmm_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *d
   int64_t max_len = INT64_MAX, n_long = 0;
   const int32_t *long_rows = nullptr;
   const int64_t over = std::max<int64_t>(plan != nullptr ? plan->block_nnz : 0, kLongMeans * (nnz / n_rows));
-  if (batch == 1 && plan != nullptr && plan->longest > over && plan->n_rows == n_rows && n_cols > 0) {
+  // (as many rows and column tiles as a grid holds; beyond, the other kernels
+  // take every row)
+  if (batch == 1 && plan != nullptr && plan->longest > over && plan->n_rows == n_rows && n_cols > 0 &&
+      plan->n_long <= kMaxLongGrid && k <= kMaxBatchGrid * (k > 32 ? 64 : 16)) {
     max_len = over;
     long_rows = plan->long_rows;
     n_long = plan->n_long;

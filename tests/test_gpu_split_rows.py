@@ -184,6 +184,31 @@ def test_spmm_where_every_row_is_long(longest):
     plan.close()
 
 
+@pytest.mark.parametrize("k", [65535 * 64, 65535 * 64 + 1])
+def test_spmm_long_row_with_more_column_tiles_than_a_grid_holds(k):
+    """A long row at the last column count whose 64-column tiles fit a grid's
+    y extent, and at the first that does not (small integers: exact)."""
+    rng = np.random.default_rng(89)
+    n_rows, n_cols = 40, 3
+    lengths = np.zeros(n_rows, np.int64)
+    lengths[[3, 7, 39]] = [600, 5, 1]
+    indices, indptr = _csr(rng, lengths, n_cols)
+    data = storage(rng.integers(-1, 2, indices.size).astype(np.float64), "float16")
+    d, i, p = to_torch(data, "float16", DEV), to_torch(indices, None, DEV), to_torch(indptr, None, DEV)
+    plan = _capi.Plan(p, n_rows, indices.size, data=d, indices=i, n_cols=n_cols)
+    assert plan.info().n_long_rows == 1
+    X = (torch.arange(n_cols * k, device=DEV) % 3 - 1).to(torch.float16).view(n_cols, k)
+    dense = torch.zeros(n_rows, n_cols, device=DEV)
+    rows = torch.repeat_interleave(torch.arange(n_rows, device=DEV), torch.from_numpy(lengths).to(DEV))
+    dense.index_put_((rows, i.long()), d.float(), accumulate=True)
+    print(f"spmm long row k={k}", flush=True)
+    got = _capi.spmm(d, i, p, X, n_rows, n_cols, plan=plan)
+    for r in (0, 3, 7, 39):
+        want = (dense[r, :, None] * X.float()).sum(0)
+        assert torch.equal(got[r].float(), want), r
+    plan.close()
+
+
 @pytest.mark.parametrize("vtype", VTYPES)
 def test_spmm_rows_of_any_length_and_alignment(vtype):
     """Rows of X and Y that are no multiple of sixteen bytes, or start off
