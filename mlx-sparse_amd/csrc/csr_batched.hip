@@ -14,8 +14,8 @@
 // kernels.  Batched SpMV transposes the vectors into the columns of one
 // n_cols x B matrix (padded to a 16-byte row), runs one SpMM - the matrix is
 // read once and each gather fetches all B values of a column together - and
-// transposes the n_rows x B result back.  The two scratch matrices come from
-// the stream-ordered allocator of `stream`.
+// transposes the n_rows x B result back, or stores straight to Y.  The scratch
+// matrices are the caller's or come from the stream-ordered allocator.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -251,8 +251,8 @@ using namespace msx;
 
 namespace {
 
-// The transposed operand Xt (n_cols x kpad) and the result Yt of the widths
-// that do not store straight to Y.  Columns are padded so that a row is a
+// The transposed operand Xt (n_cols x kpad) and, for the widths that do not
+// store straight to Y, the result Yt (n_rows x kpad).  Columns are padded so that a row is a
 // whole number of 16-byte vectors (the SpMM's vector path); padding columns
 // read zero.
 struct BatchScratch {
@@ -278,7 +278,7 @@ BatchScratch batch_scratch(msx_vtype vt, int64_t n_rows, int64_t n_cols, int64_t
   else if (vectors >= 5 && vectors <= 7) vectors = 8;
   b.kpad = vectors * per16;
   b.bx = static_cast<size_t>(std::max<int64_t>(n_cols, 1) * b.kpad * sv);
-  b.by = static_cast<size_t>(n_rows * b.kpad * sv);
+  b.by = batch_rows_direct(vectors) ? 0 : static_cast<size_t>(n_rows * b.kpad * sv);
   return b;
 }
 
@@ -313,6 +313,7 @@ msx_status run_batched_spmv(msx_vtype vt, msx_itype it, int64_t n_rows, int64_t 
     st = launch_spmv_batch_rows(vt, it, n_rows, n_cols, nnz, data, indices, indptr, Xt, kpad, Y,
                                 ldy, batch, stream, &direct);
   if (st == MSX_OK && !direct) {
+    if (b.by == 0) return fail(MSX_EINVAL, "csr_batched_matvec scratch holds no result.");
     st = launch_spmm_batched(vt, it, n_rows, n_cols, nnz, data, indices, indptr, 1, kpad, Xt, 0,
                              kpad, Yt, 0, kpad, false, stream);  // Yt is read back next
     if (st == MSX_OK)

@@ -1429,7 +1429,7 @@ bool batch_rows_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *d
   constexpr int CW = static_cast<int>(16 / sizeof(S));
   if (kpad % CW != 0 || (reinterpret_cast<uintptr_t>(Xt) & 15u) != 0) return false;
   const int64_t LR = kpad / CW;
-  if (LR != 1 && LR != 2 && LR != 4 && LR != 8) return false;
+  if (!batch_rows_direct(LR)) return false;
   const int64_t rows_per_group = kThreads / LR;
   const int64_t tiles = (n_rows + rows_per_group - 1) / rows_per_group;
   const uint32_t grid = static_cast<uint32_t>(std::max<int64_t>(1, std::min<int64_t>(tiles, kMaxGrid)));

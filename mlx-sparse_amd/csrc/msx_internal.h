@@ -272,6 +272,11 @@ msx_status launch_spmm_batched(msx_vtype vt, msx_itype it, int64_t n_rows, int64
                                int64_t x_batch, int64_t ldx, void *Y, int64_t y_batch, int64_t ldy,
                                bool y_nt, hipStream_t stream);
 
+// Sixteen-byte vectors a row of Xt for which launch_spmv_batch_rows has a kernel.
+inline bool batch_rows_direct(int64_t vectors) {
+  return vectors == 1 || vectors == 2 || vectors == 4 || vectors == 8;
+}
+
 // Batched SpMV from transposed vectors (Xt: n_cols x kpad, 16-byte aligned
 // rows) into batch-major Y (Y[b * ldy + i], b < batch); *done is false when
 // kpad is not a width the kernel takes (nothing is launched then).

@@ -110,3 +110,19 @@ def test_transpose_layout_argument_errors():
     assert f(0, 10, d, d, d, d, 0, None, d, None) == _capi.EINVAL
     assert f(3, 10, d, d, d, d, 1, d, None, None) == _capi.EINVAL
     assert f(0, 0, None, None, None, None, 0, None, None, None) == _capi.OK
+
+
+@pytest.mark.parametrize("vtype,size", [(0, 4), (1, 2), (2, 2), (3, 8)])
+def test_batch_scratch_holds_a_result_only_where_one_is_stored(vtype, size):
+    """Widths of 1, 2, 4 or 8 sixteen-byte vectors a row store straight to Y:
+    the transposed operand is all their scratch."""
+    f = _capi.lib().msx_csr_batched_spmv_scratch
+    f.argtypes, f.restype = [ctypes.c_int] + [ctypes.c_int64] * 3, ctypes.c_size_t
+    n_cols, per16 = 977, 16 // size
+    for n_rows in (301, 1 << 18):
+        for batch in range(2, 12 * per16):
+            vectors = -(-batch // per16)
+            padded = 8 if 5 <= vectors <= 7 else 4 if vectors == 3 and n_rows >= 1 << 18 else vectors
+            rows = n_cols + (0 if padded in (1, 2, 4, 8) else n_rows)
+            assert f(vtype, n_rows, n_cols, batch) == rows * padded * 16, (n_rows, batch)
+    assert f(vtype, 301, n_cols, 1) == 0
