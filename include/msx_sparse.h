@@ -577,6 +577,17 @@ typedef struct msx_solver_result {
 } msx_solver_result;
 
 /*
+ * 1 when a solve of the plan's matrix with `solver` runs its iterations in one
+ * workgroup (small systems), 0 when in a kernel a pass.
+ */
+typedef enum msx_solver_kind {
+  MSX_SOLVER_CG = 0,      /* and its Jacobi variant */
+  MSX_SOLVER_MINRES = 1,
+  MSX_SOLVER_BICGSTAB = 2
+} msx_solver_kind;
+int msx_csr_one_workgroup(msx_solver_kind solver, const msx_csr_plan *plan);
+
+/*
  * Conjugate gradients for a square symmetric positive-definite float32 CSR
  * matrix (n x n): x from x0 (device pointers; x0 and x may not overlap).
  * Device-wide: the path's SpMV with `plan` (nullable; a plan from

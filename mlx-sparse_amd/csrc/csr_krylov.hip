@@ -1240,6 +1240,17 @@ msx_status check(const char *op, msx_itype it, int64_t n, int64_t nnz, const voi
 
 using namespace msx;
 
+extern "C" int msx_csr_one_workgroup(msx_solver_kind solver, const msx_csr_plan *plan) {
+  if (plan == nullptr) return 0;
+  const int64_t n = plan->n_rows, nnz = plan->nnz;
+  switch (solver) {
+  case MSX_SOLVER_CG: return in_one_group(plan, n, nnz, kGroupMany);
+  case MSX_SOLVER_MINRES: return in_one_group(plan, n, nnz, kGroupFew);
+  case MSX_SOLVER_BICGSTAB: return bi_in_one_group(plan, n, nnz);
+  }
+  return 0;
+}
+
 extern "C" msx_status msx_csr_bicgstab(msx_itype it, int64_t n, int64_t nnz, const float *data,
                                        const void *indices, const void *indptr, const float *b,
                                        const float *x0, float *x, float rtol, float atol,

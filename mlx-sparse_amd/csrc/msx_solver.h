@@ -208,13 +208,16 @@ class BatchSchedule {
 // compute unit's rate.  The passes are the kernels' own, over one block.  The
 // matrix stays in registers for the launch (kValues values a thread), its row
 // pointers in LDS, so a product is one round of gathers of x.
-// Only for row-block plans without long rows (a row is one thread's sum).
+// Only for row-block plans without rows of more than kGroupRowValues values: a
+// row is one thread's sum in stored order, as in the row blocks, which take
+// lanes and a tree of sums for blocks that average more than that.
 // Whole solves to 1e-5, kernels -> one workgroup, us: CG, Laplacian 30^2 673
 // -> 297, 63^2 726 -> 486; MINRES 35^2 975 -> 411, 63^2 981 -> 951 (there 48
 // values a thread do not fit the registers beside its passes, so MINRES and
 // BiCGSTAB stop at 16); BiCGSTAB 43^2 857 -> 592.  A pass takes about 2.5 us, the
 // latency of its two reductions.
 constexpr int64_t kGroupRows = 4608;
+constexpr int64_t kGroupRowValues = 32;
 constexpr int64_t kGroupBatch = 128;  // iterations a launch: it ends with the solve
 constexpr int kGroupFew = 16, kGroupMany = 48;  // values a thread
 
@@ -228,8 +231,8 @@ struct GroupMatrix {
 
 // `values`: the most values a thread that the solver's loop is built for.
 inline bool in_one_group(const msx_csr_plan *plan, int64_t n, int64_t nnz, int values) {
-  return plan != nullptr && plan->n_long == 0 && plan->n_panels == 0 && plan->n_slices == 0 &&
-         n <= kGroupRows && nnz <= int64_t{values} * kSolverThreads;
+  return plan != nullptr && plan->longest <= kGroupRowValues && plan->n_panels == 0 &&
+         plan->n_slices == 0 && n <= kGroupRows && nnz <= int64_t{values} * kSolverThreads;
 }
 
 // LDS of a launch: the products of all values, then n + 1 row pointers.

@@ -430,6 +430,14 @@ def cg(data, indices, indptr, b, x0=None, *, rtol=1e-5, atol=0.0, maxiter=None, 
     return x, res.info, res.residual, res.iterations
 
 
+def one_workgroup(kind, plan) -> bool:
+    """Whether a solve ("cg", "minres", "bicgstab") of the plan's matrix runs in
+    one workgroup."""
+    f = lib().msx_csr_one_workgroup
+    f.argtypes, f.restype = [ctypes.c_int, ctypes.c_void_p], ctypes.c_int
+    return f({"cg": 0, "minres": 1, "bicgstab": 2}[kind], plan.ptr) == 1
+
+
 def krylov(kind, data, indices, indptr, b, x0=None, *, rtol=1e-5, atol=0.0, maxiter=None,
            shift=0.0, plan=None, inv_diag=None):
     """(x, info, residual, iterations) through msx_csr_bicgstab[_cpu]

@@ -326,8 +326,8 @@ def test_transposed_products_drop_columns_beyond_32_bits(vtype):
 @pytest.mark.parametrize("solver", ["cg", "pcg", "minres", "bicgstab"])
 @pytest.mark.parametrize("rows", [1, 2, 513, 1500, 2048, 2049, 4608])
 def test_small_systems_in_one_workgroup(solver, rows):
-    """Solves of systems around the one-workgroup loop's sizes, rows of one to
-    nine values (more values a thread than 16 from 2,049 rows on), both index
+    """Solves of small systems of up to about nine values a row, in one
+    workgroup and in a kernel a pass (the limits: the next test), both index
     types and a budget that ends inside a launch: status and iterations as
     the oracle's, x within the tolerance's bound of the float64 solution
     (condition number at most 5)."""
@@ -375,5 +375,84 @@ def test_small_systems_in_one_workgroup(solver, rows):
         assert info == want[1] and abs(its - want[3]) <= 1, (info, its, want[1:])
         if info == 0:
             # |x - exact| <= cond * rtol * |x|, cond <= (2 + 1) / (2 - 1) of the row sums' bound
+            assert np.linalg.norm(to_numpy(x) - exact) <= 5e-5 * np.linalg.norm(exact)
+    plan.close()
+
+
+def _system(n, values, longest=None):
+    """A symmetric diagonally dominant n x n system of exactly `values` stored
+    values in rows of about the same length, as (data, indices, indptr, rows);
+    with `longest`, row 0 has that many (diagonal entries split)."""
+    rng = np.random.default_rng(n + values)
+    pairs = (values - n) // 2
+    i = np.arange(pairs) % n
+    j = (i + 1 + np.arange(pairs) // n) % n
+    v = rng.uniform(-0.2, 0.2, pairs)
+    near = np.zeros(n)
+    np.add.at(near, np.concatenate([i, j]), np.abs(np.concatenate([v, v])))
+    diagonal = np.full(n, 2.0 * max(near.max(), 0.5))
+    rows = np.concatenate([i, j, np.arange(n)])
+    cols = np.concatenate([j, i, np.arange(n)])
+    data = np.concatenate([v, v, diagonal])
+    extra = values - rows.size if longest is None else longest - int((rows == 0).sum())
+    assert extra >= 0
+    if extra:  # row 0's diagonal entry in 1 + extra parts
+        data[2 * pairs] /= 1 + extra
+        rows, cols = np.append(rows, np.zeros(extra, int)), np.append(cols, np.zeros(extra, int))
+        data = np.append(data, np.full(extra, data[2 * pairs]))
+    order = np.lexsort((cols, rows))
+    index_dtype = np.int64 if n % 2 else np.int32
+    rows = rows[order]
+    return (data[order].astype(np.float32), cols[order].astype(index_dtype),
+            np.searchsorted(rows, np.arange(n + 1)).astype(index_dtype), rows)
+
+
+@pytest.mark.parametrize("solver,rows,values,longest,inside", [
+    case for solvers, cases in (
+        (("cg", "pcg"), [(4608, 24576, None, True), (4608, 24577, None, False),
+                         (4609, 24000, None, False), (2000, 24576, None, True),
+                         (300, 8700, 32, True), (300, 8700, 33, False)]),
+        (("minres", "minres_jacobi"), [(4608, 8192, None, True), (4608, 8193, None, False),
+                                       (4609, 8000, None, False), (513, 8192, None, True),
+                                       (250, 7250, 32, True), (250, 7250, 33, False)]),
+        (("bicgstab", "bicgstab_jacobi"), [(2048, 8192, None, True), (2048, 8193, None, False),
+                                           (2049, 8000, None, False), (513, 8192, None, True),
+                                           (250, 7250, 32, True), (250, 7250, 33, False)]))
+    for s in solvers for case in [(s, *c) for c in cases]])
+def test_one_workgroup_solves_at_their_limits(solver, rows, values, longest, inside):
+    """Systems at the most rows, values and values a row that a solver's
+    one-workgroup loop takes, and one beyond each: the loop runs where it
+    should, the status and (to one) the iterations are the oracle's, x within
+    the tolerance's bound of the float64 solution (condition number at most
+    5), also on a budget that ends inside a launch."""
+    data, indices, indptr, row_of = _system(rows, values, longest)
+    assert longest is not None or data.size == values
+    assert longest is None or np.diff(indptr).max() == longest
+    b = np.random.default_rng(rows).standard_normal(rows).astype(np.float32)
+    from scipy import sparse
+    from scipy.sparse.linalg import spsolve
+
+    m = sparse.csc_matrix((data.astype(np.float64), (row_of, indices)), shape=(rows, rows))
+    exact = spsolve(m, b.astype(np.float64))
+    inv = (1.0 / m.diagonal()).astype(np.float32)
+    d, i, p = (to_torch(t, None, DEV) for t in (data, indices, indptr))
+    plan = _capi.Plan(p, rows, data.size, data=d, indices=i, n_cols=rows)
+    kind = solver.replace("_jacobi", "").replace("pcg", "cg")
+    assert _capi.one_workgroup(kind, plan) == inside
+    jacobi = solver != kind
+    bt, jac = to_torch(b, None, DEV), to_torch(inv, None, DEV) if jacobi else None
+    print(f"limits {solver} {rows} {values} {longest}", flush=True)
+    for budget in (200, 2):
+        f = getattr(orc, {"cg": "csr_cg", "pcg": "csr_pcg_jacobi"}.get(solver, f"csr_{solver}"))
+        pre = (inv,) if jacobi else ()
+        want = f(data, indices, indptr, b, *pre, rtol=1e-5, maxiter=budget)
+        if kind == "cg":
+            x, info, _, its = _capi.cg(d, i, p, bt, rtol=1e-5, maxiter=budget, plan=plan,
+                                       inv_diag=jac)
+        else:
+            x, info, _, its = _capi.krylov(kind, d, i, p, bt, rtol=1e-5, maxiter=budget, plan=plan,
+                                           inv_diag=jac)
+        assert info == want[1] and abs(its - want[3]) <= 1, (info, its, want[1:])
+        if info == 0:
             assert np.linalg.norm(to_numpy(x) - exact) <= 5e-5 * np.linalg.norm(exact)
     plan.close()
