@@ -948,6 +948,12 @@ int msx_cpu_worker_count(void);
 msx_status msx_cpu_ranges(const int64_t *work, int64_t n, int parts,
                           int64_t *ranges, int64_t *n_ranges);
 
+/*
+ * For tests: the device allocation after the next `after` ones of this
+ * thread's panel builds fails as out of memory (-1: none does).
+ */
+void msx_test_panel_alloc_failure(int after);
+
 #ifdef __cplusplus
 } /* extern "C" */
 #endif

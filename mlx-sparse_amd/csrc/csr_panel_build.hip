@@ -444,6 +444,15 @@ int bits_for(uint64_t v) {
 
 size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
+// hipMalloc, or the failure that msx_test_panel_alloc_failure asked of this
+// thread's next build.
+thread_local int g_allocations_left = -1;
+hipError_t device_alloc(void **p, size_t bytes) {
+  if (g_allocations_left >= 0 && g_allocations_left-- == 0) return hipErrorOutOfMemory;
+  return hipMalloc(p, bytes);
+}
+hipError_t device_alloc(char **p, size_t bytes) { return device_alloc(reinterpret_cast<void **>(p), bytes); }
+
 // Device scratch of the build, released on every exit path: one block, as
 // large as the parts are expected to need (a hipFree takes 140 us and waits
 // for the device: twelve of them were 1.6 of the 3.8 ms that the build took at
@@ -481,7 +490,7 @@ class Scratch {
   char *grab(size_t bytes) {
     void *p = nullptr;
     if (bytes == 0) return nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
+    if (device_alloc(&p, bytes) != hipSuccess) {
       (void)hipGetLastError();
       return nullptr;
     }
@@ -578,7 +587,7 @@ msx_status build_layout(msx_csr_plan *p, const typename V::Storage *data, const 
   const size_t b_cb = round256(sizeof(int64_t) * (max_chunks + 1));
   const size_t b_cp = round256(sizeof(int32_t) * max_chunks);
   char *meta = nullptr;
-  if (hipMalloc(&meta, 2 * b_tb + b_seg + b_cb + b_cp) != hipSuccess) {
+  if (device_alloc(&meta, 2 * b_tb + b_seg + b_cb + b_cp) != hipSuccess) {
     (void)hipGetLastError();
     return no_memory();
   }
@@ -692,7 +701,7 @@ msx_status build_layout(msx_csr_plan *p, const typename V::Storage *data, const 
   const size_t b_u16 = round256(sizeof(uint16_t) * std::max<int64_t>(n_values, 1));
   const size_t b_prod = p->call_scratch ? 0 : round256(sizeof(A) * std::max<int64_t>(n_values, 1));
   char *base = nullptr;
-  if (hipMalloc(&base, b_data + 2 * b_u16 + b_prod) != hipSuccess) {
+  if (device_alloc(&base, b_data + 2 * b_u16 + b_prod) != hipSuccess) {
     (void)hipGetLastError();
     return no_memory();
   }
@@ -765,7 +774,7 @@ msx_status build_typed(msx_csr_plan *p, const void *data_v, const void *indices_
     const size_t b_slot = round256(sizeof(int32_t) * std::max<int64_t>(nv, 1));
     const size_t b_part = round256(sizeof(A) * std::max<int64_t>(nv, 1));
     char *vm = nullptr;
-    if (hipMalloc(&vm, b_base + b_start + b_slot + b_part) != hipSuccess) {
+    if (device_alloc(&vm, b_base + b_start + b_slot + b_part) != hipSuccess) {
       (void)hipGetLastError();
       return no_memory();
     }
@@ -827,6 +836,12 @@ msx_status build_v(msx_csr_plan *p, const void *data, const void *indices, const
 }
 
 }  // namespace
+
+}  // namespace msx
+
+extern "C" void msx_test_panel_alloc_failure(int after) { msx::g_allocations_left = after; }
+
+namespace msx {
 
 bool panels_pay(const msx_csr_plan *p) {
   const int64_t x_bytes = p->n_cols * static_cast<int64_t>(value_bytes(p->vtype));

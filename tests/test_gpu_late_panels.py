@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+import _capi
 import mlx_sparse as ms
 from mlx_sparse import _csr
 
@@ -117,3 +118,34 @@ def test_replayed_products_read_the_values_as_they_are(buffers):
         alone.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, -want) and torch.equal(a @ x, -want), i
+
+
+@pytest.mark.parametrize("long_rows", [False, True])
+def test_a_copy_that_cannot_be_allocated_leaves_row_blocks(buffers, long_rows):
+    """Whichever allocation of a panel build fails (injected on the host), AUTO
+    ends with row blocks that multiply and forced panels with MemoryError; the
+    scratch block alone can be done without."""
+    data, indices, indptr = buffers
+    if long_rows:
+        indptr = indptr.clone()
+        indptr[1:1001] = indptr[1000].item()  # row 0 takes the values of the next 999
+    want = _want(ms.csr_array((data, indices, indptr), shape=(N_ROWS, N_COLS)), _x())
+    fail = _capi.lib().msx_test_panel_alloc_failure
+    fatal = {1, 3, 4} if long_rows else {1, 2}
+    try:
+        for after in range(6 if long_rows else 4):
+            print(f"allocation {after} fails long={long_rows}", flush=True)
+            fail(after)
+            plan = _capi.Plan(indptr, N_ROWS, VALUES, data=data, indices=indices, n_cols=N_COLS)
+            assert (plan.info().n_panels == 0) == (after in fatal), after
+            assert plan.info().n_panels or plan.info().panel_bytes == 0
+            y = _capi.spmv(data, indices, indptr, _x(), N_ROWS, N_COLS, plan)
+            assert torch.equal(y, want), after
+            plan.close()
+            if after in fatal:
+                fail(after)
+                with pytest.raises((MemoryError, RuntimeError), match="allocation"):
+                    _capi.Plan(indptr, N_ROWS, VALUES, data=data, indices=indices, n_cols=N_COLS,
+                               slice_mode=_capi.SLICE_PANELS)
+    finally:
+        fail(-1)
