@@ -42,6 +42,7 @@ constexpr int64_t kLongMeans = 16;
 template <class S, int CW>
 struct Vec {
   S v[CW];
+  __device__ inline S at(int c) const { return v[c]; }
 };
 
 template <class S, int CW>
@@ -60,7 +61,7 @@ __device__ inline Vec<S, CW> load_vec(const S *p) {
 // CW elements as the dwords they were loaded in, taken apart where they are
 // used: 16-bit elements taken apart at the load (a Vec filled under a branch)
 // had every load of a chunk waited for before the next (k = 64 on the 3D
-// Poisson matrix, bfloat16: 372 -> 204 us).
+// Poisson matrix, bfloat16: 372 -> 204 us; where that is the better, unpacked_pays).
 template <class S, int CW>
 struct Packed {
   static constexpr int kBytes = CW * static_cast<int>(sizeof(S));
@@ -144,8 +145,8 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
                                    const I *__restrict__ indices, Fetch fetch, int64_t n_cols,
                                    int64_t s, int64_t e, int l, int LR,
                                    typename V::Acc (&acc)[CW]) {
-  using S = typename V::Storage;
   using A = typename V::Acc;
+  using X = decltype(fetch(0));  // Packed or Vec
   // Positions stay 64-bit: 32-bit ones measured 15 % slower here (the
   // address arithmetic of the index and value loads).
 #pragma unroll
@@ -156,7 +157,7 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
     for (; p + kUnrollDirect <= e; p += kUnrollDirect) {
       int cu[kUnrollDirect];
       A au[kUnrollDirect];
-      Packed<S, CW> xv[kUnrollDirect];
+      X xv[kUnrollDirect];
 #pragma unroll
       for (int u = 0; u < kUnrollDirect; ++u) {
         const I c = indices[p + u];
@@ -177,7 +178,7 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
       const I c = indices[p];
       if (static_cast<uint64_t>(static_cast<int64_t>(c)) < static_cast<uint64_t>(n_cols)) {
         const A a = V::widen(data[p]);
-        const Packed<S, CW> xv = fetch(static_cast<int>(c));
+        const X xv = fetch(static_cast<int>(c));
 #pragma unroll
         for (int q = 0; q < CW; ++q) acc[q] = vmadd<V>(acc[q], a, xv.at(q));
       }
@@ -199,7 +200,7 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
       cu[u] = __shfl(ci, u, LR);
       au[u] = shfl_idx(av, u, LR);
     }
-    Packed<S, CW> xv[kChunk];
+    X xv[kChunk];
 #pragma unroll
     for (int u = 0; u < kChunk; ++u)
       if (cu[u] >= 0) xv[u] = fetch(cu[u]);
@@ -230,7 +231,7 @@ __device__ inline void row_segment(const typename V::Storage *__restrict__ data,
 // part, the same sums), so every load and store is whole.  16-bit, k = 100,
 // 300,007 rows of 20: one 2-byte column per lane 683 us, this 266.
 template <class V, class I, int CW, bool SHUF, int LRT, bool NTY = true, bool SKIP = false,
-          bool ANY = false>
+          bool ANY = false, bool PK = true>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(std::is_same_v<V, F32> && CW == 4 && !ANY ? 7 : 1, 8)))
     spmm_rows(const typename V::Storage *__restrict__ data, const I *__restrict__ indices,
@@ -269,7 +270,10 @@ __attribute__((amdgpu_waves_per_eu(std::is_same_v<V, F32> && CW == 4 && !ANY ? 7
     const S *Xc = X + (col < k ? col : 0);
     row_segment<V, I, CW, SHUF>(
         data, indices,
-        [&](int c) { return load_packed<S, CW, ANY>(Xc + static_cast<int64_t>(c) * ldx); },
+        [&](int c) {
+          if constexpr (PK) return load_packed<S, CW, ANY>(Xc + static_cast<int64_t>(c) * ldx);
+          else return load_vec<S, CW>(Xc + static_cast<int64_t>(c) * ldx);
+        },
         n_cols, s, e, l, LR, acc);
     if (want >= k) continue;
     Vec<S, CW> out;
@@ -1131,6 +1135,18 @@ __attribute__((amdgpu_waves_per_eu(LG <= 3 ? 7 : 1, 8)))
   }
 }
 
+// Whether 16-bit X rows are taken apart as they are loaded (PK false) in groups
+// of up to four lanes: where the plan's windows say that columns are scattered,
+// rows are short and X outgrows an L2, waves with one load each in flight, more
+// of them, are faster.  bfloat16, packed -> apart, us: 200,000 rows of 16, k = 8
+// / 16 / 24 / 32 25.5 / 35.2 / 52.4 / 50.5 -> 23.3 / 29.2 / 40.2 / 42.0, 1 M rows
+// 259 -> 249 at k = 8; the other way 30,000 rows of 16 9.0 both, 60,000 of 40 15.2
+// -> 16.3, 20,000 of 200 35 -> 48, 3D Poisson 80^3 24.0 -> 26.1.
+bool unpacked_pays(int64_t n_rows, int64_t n_cols, int64_t nnz, int64_t k, const msx_csr_plan *plan) {
+  return plan != nullptr && 4 * plan->win_rows_max > n_cols && nnz < 32 * n_rows &&
+         2 * n_cols * k >= (int64_t{2} << 20);
+}
+
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Whether rows of X that are no whole aligned sixteen-byte vectors are read
@@ -1301,6 +1317,14 @@ msx_status spmm_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const void *d
     if (vec) {
       auto go = [&](auto nt, auto skip) {
         constexpr bool NT = decltype(nt)::value, SK = decltype(skip)::value;
+        if constexpr (sizeof(S) == 2 && NT && !SK) {
+          if (LR < kChunk && unpacked_pays(n_rows, n_cols, nnz, k, plan)) {
+            if (LR == 1) launch(spmm_rows<V, I, CWV, false, 1, NT, SK, false, false>);
+            else if (LR == 2) launch(spmm_rows<V, I, CWV, false, 2, NT, SK, false, false>);
+            else launch(spmm_rows<V, I, CWV, false, 4, NT, SK, false, false>);
+            return;
+          }
+        }
         switch (LR) {
         case 1: launch(spmm_rows<V, I, CWV, false, 1, NT, SK>); break;
         case 2: launch(spmm_rows<V, I, CWV, false, 2, NT, SK>); break;

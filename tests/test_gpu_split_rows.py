@@ -160,6 +160,29 @@ def test_spmm_long_rows_in_stored_order(vtype, index_dtype):
     plan.close()
 
 
+@pytest.mark.parametrize("vtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("n_cols", [32_700, 66_000, 140_000])
+def test_spmm_narrow_16_bit_rows_of_scattered_matrices(vtype, n_cols):
+    """16-bit X rows of one to four sixteen-byte vectors, X below 2 MB, about
+    there and above (where the loads are taken apart at once): the oracle's
+    bits."""
+    rng = np.random.default_rng(97)
+    lengths = rng.integers(0, 31, 2000)
+    n_rows = len(lengths)
+    indices, indptr = _csr(rng, lengths, n_cols)
+    data = _values(rng, indices.size, vtype)
+    d, i, p = to_torch(data, vtype, DEV), to_torch(indices, None, DEV), to_torch(indptr, None, DEV)
+    plan = _capi.Plan(p, n_rows, indices.size, data=d, indices=i, n_cols=n_cols)
+    assert 4 * plan.info().window_rows > n_cols
+    for k in (8, 16, 24, 32):
+        X = _values(rng, (n_cols, k), vtype)
+        print(f"narrow 16-bit {vtype} {n_cols} k={k}", flush=True)
+        got = _capi.spmm(d, i, p, to_torch(X, vtype, DEV), n_rows, n_cols, plan=plan)
+        want = orc.csr_matmul(data, indices, indptr, X, n_rows, vtype=vtype)
+        assert to_numpy(got).tobytes() == want.tobytes(), k
+    plan.close()
+
+
 @pytest.mark.parametrize("longest", [600, 9600, 9601])
 def test_spmm_where_every_row_is_long(longest):
     """Rows of 600 values throughout, the longest at sixteen times the mean
