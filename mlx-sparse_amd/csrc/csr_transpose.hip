@@ -562,10 +562,12 @@ constexpr int kVjpUnroll = 4;  // 64-position steps whose loads a wave issues to
 // The same gradient, 256 positions per wave: four index loads, then four
 // gathers of x, in flight at once, the rows found meanwhile.  Positions no
 // row holds (before indptr[0], from indptr[n_rows] on) are left as they are.
-// For matrices whose plan lists long rows; on rows of 16 the row search is a
-// chain that G lanes per row do not have (1.3 M rows: 145 us there, 177 us
-// here), on rows of up to 37,500 the longest row is the other's chain
-// (300,007 power-law rows: 1,370 us there, 28 us here).
+// For matrices whose plan's longest row is an exception, over kSplitMeans mean
+// rows; on rows of 16 the row search is a chain that G lanes per row do not
+// have (1.3 M rows: 145 us there, 177 us here; 20,000 rows of 600: 94 and 125),
+// on rows of up to 37,500 the longest row is the other's chain (300,007
+// power-law rows: 1,370 us there, 28 us here).
+constexpr int64_t kSplitMeans = 16;
 template <class V, class I>
 __global__ void __launch_bounds__(kThreads)
     spmv_data_vjp_split(const I *__restrict__ indices, const I *__restrict__ indptr,
@@ -1562,7 +1564,7 @@ extern "C" msx_status msx_csr_spmv_data_vjp_ws(msx_vtype vt, msx_itype it, int64
     return launch_panel_data_vjp(use.plan(), indptr, x, cot, out, static_cast<hipStream_t>(stream));
   }
   return dispatch<SpmvDataVjpOp>(vt, it, n_rows, n_cols, nnz, indices, indptr, x, cot, out,
-                                 plan != nullptr && plan->n_long > 0,
+                                 plan != nullptr && plan->longest > std::max(plan->block_nnz, kSplitMeans * (nnz / n_rows)),
                                  static_cast<hipStream_t>(stream));
 }
 

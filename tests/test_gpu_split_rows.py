@@ -77,6 +77,32 @@ def test_value_gradients_by_positions(kind, vtype):
         assert to_numpy(got).tobytes() == want.tobytes(), k
 
 
+@pytest.mark.parametrize("longest", [96, 97, 513])
+@pytest.mark.parametrize("vtype", VTYPES)
+def test_value_gradients_around_the_split_rule(longest, vtype):
+    """The vector's value gradient with the longest row at sixteen mean rows
+    (lanes a row), one value above and far above (by positions), rows ending
+    at the edges of a wave's 64 and 256 positions: the oracle's bits."""
+    rng = np.random.default_rng(101)
+    lengths = np.full(600, 6)
+    lengths[:10] = [64, 64, 90, 1, 63, 0, 0, 33, 31, 90]
+    lengths[300] = longest
+    lengths[10:200] -= np.minimum(6, np.diff(np.linspace(0, lengths.sum() - 3650, 191).astype(int)))
+    n_rows, n_cols = len(lengths), 777
+    assert lengths.min() >= 0 and lengths.sum() // n_rows == 6 and lengths.max() == longest
+    indices, indptr = _csr(rng, lengths, n_cols, np.int64, bad=0.02)
+    nnz = indices.size
+    x, cot = _values(rng, n_cols, vtype), _values(rng, n_rows, vtype)
+    i, p = to_torch(indices, None, DEV), to_torch(indptr, None, DEV)
+    plan = _capi.Plan(p, n_rows, nnz, 64)
+    print(f"split rule {longest} {vtype}", flush=True)
+    got = _capi.spmv_data_vjp(i, p, to_torch(x, vtype, DEV), to_torch(cot, vtype, DEV), n_rows,
+                              n_cols, plan=plan)
+    want = orc.csr_data_vjp(indices, indptr, x, cot, n_rows, n_cols, nnz, vtype=vtype)
+    assert to_numpy(got).tobytes() == want.tobytes()
+    plan.close()
+
+
 @pytest.mark.parametrize("vtype,index_dtype,n_rows,n_cols,values", [
     ("float32", np.int32, 700_001, (4 << 20) // 4, 5 << 20),
     ("float32", np.int64, 900_003, (5 << 19) // 4, 12 << 20),
