@@ -96,6 +96,30 @@ def test_batches_of_padded_widths(vtype, n_rows):
                                       err_msg=f"{vtype} batch={batch}")
 
 
+@pytest.mark.parametrize("vtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("longest_row", [8, 24])  # mean rows of four and of twelve
+def test_batches_of_16_bit_vectors_over_a_wide_matrix(vtype, longest_row):
+    """Vectors of 2 MB and more as one operand, one to four sixteen-byte
+    vectors a row: the oracle's bits with the loads packed and taken apart."""
+    rng = np.random.default_rng(longest_row)
+    n_rows, n_cols = 3000, 140_000
+    lengths = rng.integers(0, longest_row + 1, n_rows)
+    indptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(indptr[-1])
+    assert (nnz >= 8 * n_rows) == (longest_row == 24)
+    indices = rng.integers(0, n_cols, nnz).astype(np.int32)
+    data = _values(rng, nnz, vtype)
+    d, i, p = (to_torch(a, vtype if a is data else None, DEV) for a in (data, indices, indptr))
+    for batch in (8, 11, 16, 23, 29):
+        X = _values(rng, (batch, n_cols), vtype)
+        want = _want_vectors(data, indices, indptr, X, n_rows, vtype)
+        Y = torch.zeros((batch, n_rows), dtype=d.dtype, device=DEV)
+        _capi.batched_spmv(d, i, p, to_torch(X, vtype, DEV), n_rows, n_cols, Y=Y, ldx=n_cols,
+                           ldy=n_rows)
+        np.testing.assert_array_equal(_bytes(to_numpy(Y)), _bytes(want),
+                                      err_msg=f"{vtype} batch={batch}")
+
+
 @pytest.mark.parametrize("vtype", VTYPES)
 def test_batched_spmm_parity_and_batch_strides(vtype):
     rng = np.random.default_rng(6)
