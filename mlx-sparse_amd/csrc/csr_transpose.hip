@@ -398,7 +398,8 @@ msx_status transpose_typed(int64_t n_rows, int64_t n_cols, int64_t nnz, const vo
 // neighbouring columns on stencils and bands (64 consecutive positions a wave
 // instead: 3D Poisson 100^3 48 -> 82 us).  A row of more than kWholeRow values
 // is left to the whole workgroup after its other rows (300,007 power-law rows,
-// the longest 37,500: 2,165 -> 237 us at 1,024).
+// the longest 37,500: 2,039 -> 222 us; rows of 250, 300 and 600 values throughout
+// within 1 %).
 constexpr int64_t kWholeRow = 256;
 
 template <class V, class I>

@@ -233,8 +233,9 @@ constexpr int64_t kPanelMinXFew = int64_t{4} << 20;  // 4 MB of x
 constexpr int64_t kPanelValues = int64_t{12} << 20;
 constexpr int64_t kPanelFewValues = int64_t{5} << 20;
 // From 16 MB of x with at most two values per column on, panels only from 16
-// Mi values and XCD slices below, the choice that the selection tests pin (8
-// M values: panels 44 us, slices 186).
+// Mi values and XCD slices below: not the faster choice (8 M values: slices 186
+// us, panels 44) but the one AUTO has always made there, which callers and the
+// selection tests know.
 constexpr int64_t kSliceMinX = int64_t{16} << 20;
 constexpr int64_t kPanelAnyValues = int64_t{16} << 20;
 // True when those sizes favour panels (csr_panel_build.hip).

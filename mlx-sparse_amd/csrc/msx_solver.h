@@ -211,11 +211,11 @@ class BatchSchedule {
 // Only for row-block plans without rows of more than kGroupRowValues values: a
 // row is one thread's sum in stored order, as in the row blocks, which take
 // lanes and a tree of sums for blocks that average more than that.
-// Whole solves to 1e-5, kernels -> one workgroup, us: CG, Laplacian 30^2 673
-// -> 297, 63^2 726 -> 486; MINRES 35^2 975 -> 411, 63^2 981 -> 951 (there 48
-// values a thread do not fit the registers beside its passes, so MINRES and
-// BiCGSTAB stop at 16); BiCGSTAB 43^2 857 -> 592.  A pass takes about 2.5 us, the
-// latency of its two reductions.
+// Whole solves to 1e-5, kernels -> one workgroup, us: CG, Laplacian 30^2 712
+// -> 309, 63^2 707 -> 492; MINRES 35^2 955 -> 434, 40^2 982 -> 468 (48 values a
+// thread do not fit the registers beside its passes, 63^2 981 -> 951 with them,
+// so MINRES and BiCGSTAB stop at 16); BiCGSTAB 40^2 919 -> 456.  A pass takes
+// about 2.5 us, the latency of its two reductions.
 constexpr int64_t kGroupRows = 4608;
 constexpr int64_t kGroupRowValues = 32;
 constexpr int64_t kGroupBatch = 128;  // iterations a launch: it ends with the solve

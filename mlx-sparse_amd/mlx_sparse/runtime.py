@@ -7,7 +7,8 @@ the native CPU path reads on every call.  ``GPU_PLAN`` (new) toggles the
 cached row-block plan of the GPU SpMV; without it a plan-free kernel runs.
 ``GPU_SLICE`` (new) selects the reordered copy a plan may hold for scattered
 gathers: "auto" (default: panels when the columns are scattered over an x of
-at least 4 MB with 5 M values, or 2.5 MB with 12 M), "off", "on" (XCD
+at least 4 MB with 5 M values, or 2.5 MB with 12 M; below 8 MB or 16 M values
+only once ``plan()`` was asked for or 64 products with a vector were made), "off", "on" (XCD
 column slices) or "panels" (LDS column panels); it applies to plans built
 while it is set.  ``GPU_ADJOINT`` (new) routes the A^H products of the
 gradients on the GPU: "atomic" (scatter over A's rows), "transpose" (a

@@ -464,9 +464,8 @@ def test_auto_selection_and_binding():
     plan = _capi.Plan(p, g.shape[0], g.nnz, data=d, indices=i, n_cols=g.shape[1])
     assert plan.info().n_slices == 0 and plan.info().n_panels == 0
     plan.close()
-    # scattered, but too few short-row values to give each of the 256 compute
-    # units a 65536-value pass-1 chunk: row blocks at x = 8.4 MB, XCD slices
-    # from x = 16 MB on
+    # scattered, but no panels: fewer than 5 Mi values at x = 8.4 MB (row
+    # blocks), two values a column and fewer than 16 Mi at x = 16 MB (XCD slices)
     for n, kind in ((1 << 21, "blocks"), (1 << 22, "slices")):
         f = s.random_fixed_row(n, 2, seed=8)
         d, i, p = _upload(f.data, f.indices, f.indptr, "float32")
