@@ -92,7 +92,9 @@ typedef enum msx_slice_mode {
  * With MSX_SLICE_AUTO: keep row blocks where panels are worth their build only
  * over some tens of products (x below 8 MB or fewer than 16 Mi values).
  * msx_csr_plan_deferred is then 1; a plan built again without the flag holds
- * the panels.
+ * the panels.  Panels of those sizes are left alone by a product that is
+ * captured into a graph, unless a msx_csr_plan_refresh is captured before it:
+ * its replays read the caller's values, as row blocks do.
  */
 #define MSX_PLAN_DEFER 2
 

@@ -165,12 +165,12 @@ class CSRArray:
         key = ("plan", _device_name(device))
         hit = self._cache.get(key)
         if hit is not None:
-            built, plan = hit
+            built, plan, deferred = hit
             if built[1:] == now[1:]:
                 if built[0] != now[0]:
                     plan.refresh(bufs[0])
-                    self._cache[key] = (now, plan)
-                if not plan.deferred or not self._repaid(plan, products):
+                    self._cache[key] = (now, plan, deferred)
+                if not deferred or not self._repaid(plan, products):
                     return bufs, plan
         from mlx_sparse import _native
 
@@ -181,9 +181,8 @@ class CSRArray:
                                 n_cols=self.shape[1],
                                 slice_mode=int(runtime.get(runtime.RuntimeOption.GPU_SLICE)),
                                 defer="kept" not in self._cache or now[0][1] < 0)
-        if plan.deferred:
-            plan.served = products
-        self._cache[key] = (now, plan)
+        plan.served = products
+        self._cache[key] = (now, plan, plan.deferred)
         return bufs, plan
 
     def _repaid(self, plan, products: int) -> bool:
@@ -202,8 +201,8 @@ class CSRArray:
                        sorted_indices=self.sorted_indices,
                        has_canonical_format=self.has_canonical_format)
         for key in [k for k in self._cache if k[0] == "plan"]:
-            built, plan = self._cache.pop(key)
-            out._cache[key] = (((None, None),) + tuple(built[1:]), plan)
+            built, *rest = self._cache.pop(key)
+            out._cache[key] = (((None, None),) + tuple(built[1:]), *rest)
         self._share_use(out)
         return out
 
