@@ -88,8 +88,13 @@ def test_uncounted_values_are_read_as_they_are(buffers, planned):
         assert torch.equal(a @ x, 2 * want)
 
 
-def test_replayed_products_read_the_values_as_they_are(buffers):
-    a, x = _array(buffers), _x()
+@pytest.mark.parametrize("long_rows", [False, True])
+def test_replayed_products_read_the_values_as_they_are(buffers, long_rows):
+    data, indices, indptr = buffers
+    if long_rows:
+        indptr = indptr.clone()
+        indptr[1:1001] = indptr[1000].item()  # row 0 takes the values of the next 999
+    a, x = _array((data, indices, indptr)), _x()
     a.plan()
     assert _panels(a) > 0
     want = _want(a, x)
