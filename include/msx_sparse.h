@@ -293,7 +293,8 @@ msx_status msx_csr_spmv(msx_vtype vt, msx_itype it, int64_t n_rows,
  * The same with the call's device scratch: at least msx_csr_plan_scratch
  * bytes (0 for a plan that holds its own), 256-byte aligned, free for reuse
  * once the call's work on `stream` is done.  NULL: from the stream-ordered
- * allocator.
+ * allocator; where it has no room for a copy's products, the plan's row blocks
+ * serve.
  */
 size_t msx_csr_plan_scratch(const msx_csr_plan *plan);
 msx_status msx_csr_spmv_ws(msx_vtype vt, msx_itype it, int64_t n_rows,
@@ -952,7 +953,8 @@ msx_status msx_cpu_ranges(const int64_t *work, int64_t n, int parts,
 
 /*
  * For tests: the device allocation after the next `after` ones of this
- * thread's panel builds fails as out of memory (-1: none does).
+ * thread's panel builds and call scratch fails as out of memory (-1: none
+ * does).
  */
 void msx_test_panel_alloc_failure(int after);
 

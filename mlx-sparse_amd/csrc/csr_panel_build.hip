@@ -43,6 +43,10 @@
 
 namespace msx {
 namespace {
+thread_local int g_allocations_left = -1;
+}
+bool test_allocation_fails() { return g_allocations_left >= 0 && g_allocations_left-- == 0; }
+namespace {
 
 #define MSX_TRY_STATUS(expr)     \
   do {                           \
@@ -444,12 +448,9 @@ int bits_for(uint64_t v) {
 
 size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
-// hipMalloc, or the failure that msx_test_panel_alloc_failure asked of this
-// thread's next build.
-thread_local int g_allocations_left = -1;
+// hipMalloc, or the failure that a test asked for.
 hipError_t device_alloc(void **p, size_t bytes) {
-  if (g_allocations_left >= 0 && g_allocations_left-- == 0) return hipErrorOutOfMemory;
-  return hipMalloc(p, bytes);
+  return test_allocation_fails() ? hipErrorOutOfMemory : hipMalloc(p, bytes);
 }
 hipError_t device_alloc(char **p, size_t bytes) { return device_alloc(reinterpret_cast<void **>(p), bytes); }
 

@@ -371,15 +371,20 @@ PlanUse::PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStrea
     plan_ = &mine_;
   }
   if (!plan->call_scratch) return;
-  const ScratchSizes z = scratch_sizes(plan_);
+  ScratchSizes z = scratch_sizes(plan_);
   if (z.total() == 0) return;
   if (scratch == nullptr) {
-    const hipError_t e = hipMallocAsync(&owned_, z.total(), stream);
-    if (e != hipSuccess) {
-      owned_ = nullptr;
-      (void)hipGetLastError();
-      status_ = fail(MSX_ENOMEM, "device allocation of a plan's call scratch failed.");
-      return;
+    if (!take_scratch(z.total())) {
+      // the row blocks that every plan holds need room for long rows' sums only
+      mine_ = *plan;
+      mine_.n_panels = mine_.n_slices = 0;
+      mine_.pn_vstart = nullptr;
+      plan_ = &mine_;
+      z = scratch_sizes(plan_);
+      if (!values || (z.total() > 0 && !take_scratch(z.total()))) {
+        status_ = fail(MSX_ENOMEM, "device allocation of a plan's call scratch failed.");
+        return;
+      }
     }
     scratch = owned_;
   } else if (bytes < z.total() || (reinterpret_cast<uintptr_t>(scratch) & 255u) != 0) {
@@ -400,6 +405,13 @@ PlanUse::PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStrea
   mine_.partials = take(z.chunk);
   mine_.ls_partial = take(z.ls);
   plan_ = &mine_;
+}
+
+bool PlanUse::take_scratch(size_t bytes) {
+  if (!test_allocation_fails() && hipMallocAsync(&owned_, bytes, stream_) == hipSuccess) return true;
+  owned_ = nullptr;
+  (void)hipGetLastError();
+  return false;
 }
 
 PlanUse::~PlanUse() {

@@ -1561,8 +1561,10 @@ extern "C" msx_status msx_csr_spmv_data_vjp_ws(msx_vtype vt, msx_itype it, int64
   // when its copy holds every value (no invalid column was dropped).
   if (plan != nullptr && plan->bound && plan->vtype == vt && panel_data_vjp_fits(plan)) {
     const PlanUse use(plan, scratch, scratch_bytes, static_cast<hipStream_t>(stream), false);
-    if (use.status() != MSX_OK) return use.status();
-    return launch_panel_data_vjp(use.plan(), indptr, x, cot, out, static_cast<hipStream_t>(stream));
+    if (use.status() == MSX_OK)
+      return launch_panel_data_vjp(use.plan(), indptr, x, cot, out, static_cast<hipStream_t>(stream));
+    if (use.status() != MSX_ENOMEM) return use.status();
+    clear_error();  // no room for the gathered x: without the panels
   }
   return dispatch<SpmvDataVjpOp>(vt, it, n_rows, n_cols, nnz, indices, indptr, x, cot, out,
                                  plan != nullptr && plan->longest > std::max(plan->block_nnz, kSplitMeans * (nnz / n_rows)),

@@ -180,7 +180,9 @@ msx_status check_plan(const char *op, const msx_csr_plan *plan, msx_vtype vt, ms
 // last refresh on another stream; with MSX_PLAN_CALL_SCRATCH a copy whose
 // products and partial sums lie in the call's own scratch - the caller's, else
 // memory of `stream`'s allocator, given back when the object ends - so that
-// calls on several streams share only what they read.
+// calls on several streams share only what they read.  Where there is no room
+// for a copy's products the plan's row blocks serve.
+bool test_allocation_fails();  // msx_test_panel_alloc_failure (csr_panel_build.hip)
 class PlanUse {
  public:
   // values: the call reads the matrix's values.
@@ -193,6 +195,8 @@ class PlanUse {
   const msx_csr_plan *plan() const { return plan_; }
 
  private:
+  bool take_scratch(size_t bytes);
+
   const msx_csr_plan *plan_;
   msx_csr_plan mine_;
   void *owned_ = nullptr;

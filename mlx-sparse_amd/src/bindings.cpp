@@ -256,6 +256,16 @@ at::Tensor scratch_for(msx::ExecContext &ctx, py::handle like, size_t bytes) {
   return t;
 }
 
+// The same for a plan; none where torch has no room for it: the library then
+// asks the stream-ordered allocator or does without the plan's copy.
+at::Tensor plan_scratch_for(msx::ExecContext &ctx, py::handle like, const msx_csr_plan *plan) {
+  try {
+    return scratch_for(ctx, like, msx_csr_plan_scratch(plan));
+  } catch (const c10::OutOfMemoryError &) {
+    return {};
+  }
+}
+
 // What CSRArray's caches are checked against: storage address and version
 // counter of the three buffers (inference tensors keep no counter: -1).
 py::tuple stamps(py::handle data, py::handle indices, py::handle indptr) {
@@ -296,7 +306,7 @@ py::object csr_matvec(py::handle data_o, py::handle indices_o, py::handle indptr
   ctx.stream = vd.device >= 0 ? stream_for(vd.device) : nullptr;
   const msx_csr_plan *p = plan_ptr(plan);
   if (vd.device >= 0) {
-    const at::Tensor scratch = scratch_for(ctx, data, msx_csr_plan_scratch(p));
+    const at::Tensor scratch = plan_scratch_for(ctx, data, p);
     msx::csr_matvec(vd, vi, vp, vx, vo, n_rows, n_cols, p, ctx);
   } else {
     py::gil_scoped_release nogil;
@@ -571,7 +581,7 @@ py::object csr_matvec_data_vjp(py::handle indices_o, py::handle indptr_o, py::ha
   msx::ExecContext ctx = context_for(vx, n_threads);
   if (vx.device >= 0) {
     const msx_csr_plan *p = plan_ptr(plan);
-    const at::Tensor scratch = scratch_for(ctx, x, msx_csr_plan_scratch(p));
+    const at::Tensor scratch = plan_scratch_for(ctx, x, p);
     msx::csr_matvec_data_vjp(vi, vp, vx, vc, vo, n_rows, n_cols, ctx, p);
   } else {
     py::gil_scoped_release nogil;

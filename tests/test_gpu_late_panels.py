@@ -154,3 +154,44 @@ def test_a_copy_that_cannot_be_allocated_leaves_row_blocks(buffers, long_rows):
                                slice_mode=_capi.SLICE_PANELS)
     finally:
         fail(-1)
+
+
+@pytest.mark.parametrize("long_rows", [False, True])
+@pytest.mark.parametrize("stream_ordered", [True, False])
+def test_products_without_room_for_the_copys_scratch(buffers, long_rows, stream_ordered):
+    """torch may not allocate the scratch of a panel product or gradient: it
+    comes from the stream-ordered allocator, and where that fails too
+    (injected) the product runs over the plan's row blocks and the gradient
+    without the panels."""
+    data, indices, indptr = buffers
+    if long_rows:
+        indptr = indptr.clone()
+        indptr[1:1001] = indptr[1000].item()
+    a, x = _array((data, indices, indptr)), _x()
+    a.plan()
+    assert _panels(a) > 0
+    a.data.requires_grad_(True)
+    want, g = _want(a, x), torch.ones(N_ROWS, device=DEV)
+    y = a @ x
+    fail = _capi.lib().msx_test_panel_alloc_failure
+    total = torch.cuda.mem_get_info()[1]
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    held = torch.cuda.memory_reserved()
+    print(f"no room long={long_rows} stream ordered={stream_ordered}", flush=True)
+    try:
+        torch.cuda.set_per_process_memory_fraction((held + (4 << 20)) / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(VALUES, device=DEV)
+        fail(-1 if stream_ordered else 0)
+        with torch.no_grad():
+            assert torch.equal(a @ x, want)
+        torch.cuda.empty_cache()
+        held = torch.cuda.memory_reserved()
+        torch.cuda.set_per_process_memory_fraction((held + (30 << 20)) / total)  # the result, not both
+        fail(-1 if stream_ordered else 0)
+        d, = torch.autograd.grad(y, a.data, g)
+    finally:
+        fail(-1)
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(d, x[a.indices])
