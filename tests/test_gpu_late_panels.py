@@ -177,20 +177,31 @@ def test_products_without_room_for_the_copys_scratch(buffers, long_rows, stream_
     total = torch.cuda.mem_get_info()[1]
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
-    held = torch.cuda.memory_reserved()
     print(f"no room long={long_rows} stream ordered={stream_ordered}", flush=True)
-    try:
-        torch.cuda.set_per_process_memory_fraction((held + (4 << 20)) / total)
+
+    def leave(spare):
+        """torch may allocate `spare` bytes more in one piece, and no second scratch."""
+        room = torch.empty(spare, dtype=torch.uint8, device=DEV)
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        full = []
         with pytest.raises(torch.OutOfMemoryError):
-            torch.empty(VALUES, device=DEV)
+            while True:
+                full.append(torch.empty(VALUES, device=DEV))
+        del room
+        return full
+
+    try:
+        full = leave(8 << 20)  # the product's result
         fail(-1 if stream_ordered else 0)
         with torch.no_grad():
-            assert torch.equal(a @ x, want)
-        torch.cuda.empty_cache()
-        held = torch.cuda.memory_reserved()
-        torch.cuda.set_per_process_memory_fraction((held + (30 << 20)) / total)  # the result, not both
+            got = a @ x
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        del full
+        assert torch.equal(got, want)
+        full = leave(22 << 20)  # the gradient
         fail(-1 if stream_ordered else 0)
         d, = torch.autograd.grad(y, a.data, g)
+        del full
     finally:
         fail(-1)
         torch.cuda.set_per_process_memory_fraction(1.0)
