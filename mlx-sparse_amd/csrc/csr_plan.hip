@@ -346,7 +346,7 @@ msx_status mark_refreshed(msx_csr_plan *p, hipStream_t stream) {
 PlanUse::PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStream_t stream,
                  bool values)
     : plan_(plan), stream_(stream) {
-  if (plan == nullptr) return;
+  if (plan == nullptr || (plan->call_scratch && plan->call_bytes == 0)) return;  // no copy, no sums
   const bool unmarked = __atomic_load_n(&plan->unmarked, __ATOMIC_ACQUIRE);
   if (values && (unmarked || plan->refreshed != nullptr) && plan->refreshed_on != stream &&
       !capturing(stream)) {
@@ -567,6 +567,7 @@ extern "C" msx_status msx_csr_plan_create_bound(msx_vtype vt, msx_itype it, int6
     release(p);
     return st;
   }
+  if (p->call_scratch) p->call_bytes = scratch_sizes(p).total();
   *out = p;
   return MSX_OK;
 }
@@ -594,7 +595,7 @@ extern "C" int msx_csr_plan_deferred(const msx_csr_plan *plan) {
 }
 
 extern "C" size_t msx_csr_plan_scratch(const msx_csr_plan *plan) {
-  return plan != nullptr && plan->call_scratch ? scratch_sizes(plan).total() : 0;
+  return plan != nullptr ? plan->call_bytes : 0;
 }
 
 extern "C" msx_status msx_csr_plan_destroy(msx_csr_plan *plan) {

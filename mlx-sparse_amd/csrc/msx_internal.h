@@ -77,6 +77,7 @@ struct msx_csr_plan {
   const void *indptr;         // the row pointers the plan was built from
   bool bound;                 // built by msx_csr_plan_create_bound
   bool call_scratch;          // MSX_PLAN_CALL_SCRATCH: pn_prod and s_partial are null
+  size_t call_bytes;          // then the scratch of a call, else 0
   const void *bound_data;     // the buffers a bound plan was built from (data: as last refreshed)
   const void *bound_indices;
   // The last refresh of the value copies outside a capture, which calls on

@@ -134,10 +134,11 @@ py::object as_tensor(py::handle obj) {
 // conjugates and some negations as a flag on the memory of another tensor.
 py::object contiguous(py::handle obj) {
   py::object t = as_tensor(obj);
-  if (tensor_of(t).is_conj()) t = t.attr("resolve_conj")();
-  if (tensor_of(t).is_neg()) t = t.attr("resolve_neg")();
-  if (tensor_of(t).is_contiguous()) return t;
-  return t.attr("contiguous")();
+  {
+    const at::Tensor &a = tensor_of(t);
+    if (a.is_contiguous() && !a.is_conj() && !a.is_neg()) return t;
+  }
+  return t.attr("resolve_conj")().attr("resolve_neg")().attr("contiguous")();
 }
 
 // The stream torch's current stream of `device` wraps.
@@ -259,8 +260,10 @@ at::Tensor scratch_for(msx::ExecContext &ctx, py::handle like, size_t bytes) {
 // The same for a plan; none where torch has no room for it: the library then
 // asks the stream-ordered allocator or does without the plan's copy.
 at::Tensor plan_scratch_for(msx::ExecContext &ctx, py::handle like, const msx_csr_plan *plan) {
+  const size_t bytes = msx_csr_plan_scratch(plan);
+  if (bytes == 0) return {};
   try {
-    return scratch_for(ctx, like, msx_csr_plan_scratch(plan));
+    return scratch_for(ctx, like, bytes);
   } catch (const c10::OutOfMemoryError &) {
     return {};
   }
