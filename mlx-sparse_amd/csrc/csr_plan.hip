@@ -289,10 +289,13 @@ msx_status build_plan(msx_csr_plan *p, const I *indptr, hipStream_t stream) {
   return MSX_OK;
 }
 
-// Device bytes of a plan's scratch arrays, each on a 256-byte boundary.
+// Device bytes of a plan's scratch arrays, each on a 256-byte boundary.  The
+// panel products begin `lead` bytes in: on the boundary of a large block, which
+// the copy's values begin on too, 4.2 M rows of 16 took 212.8 us, 256 bytes past
+// it 210.7.
 struct ScratchSizes {
-  size_t prod, vpart, spart, chunk, ls;
-  size_t total() const { return prod + vpart + spart + chunk + ls; }
+  size_t lead, prod, vpart, spart, chunk, ls;
+  size_t total() const { return lead + prod + vpart + spart + chunk + ls; }
 };
 
 ScratchSizes scratch_sizes(const msx_csr_plan *p) {
@@ -300,6 +303,7 @@ ScratchSizes scratch_sizes(const msx_csr_plan *p) {
   const auto bytes = [](int64_t n, size_t each) { return align_up(static_cast<size_t>(n) * each, 256); };
   ScratchSizes z{};
   if (p->n_panels > 0) z.prod = bytes(p->pn_values, a);
+  if (z.prod > 0) z.lead = 256;
   if (p->pn_vstart != nullptr) z.vpart = bytes(p->pn_vrows, a);
   if (p->n_slices > 0) z.spart = bytes(int64_t{kSlices} * p->n_rows, a);
   if (p->pn_vstart == nullptr) z.chunk = bytes(p->n_chunks > p->n_long ? p->n_chunks : 0, 8);
@@ -399,6 +403,7 @@ PlanUse::PlanUse(const msx_csr_plan *plan, void *scratch, size_t bytes, hipStrea
     at += b;
     return here;
   };
+  take(z.lead);
   mine_.pn_prod = take(z.prod);
   mine_.pn_partial = take(z.vpart);
   mine_.s_partial = take(z.spart);
